@@ -146,9 +146,7 @@ __global__ __launch_bounds__(kThreads) void dbatch_integrate_kernel(
     for (unsigned i = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); i < n; i += waves) {
         const uint32_t tile = __builtin_amdgcn_readfirstlane(list[i].tile);
         const uint32_t v = __builtin_amdgcn_readfirstlane(list[i].volume);
-        const uint64_t mask =
-            ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(list[i].frames >> 32)) << 32) |
-            __builtin_amdgcn_readfirstlane((uint32_t)list[i].frames);
+        const uint64_t mask = uniform_mask(list[i].frames);
         const DVol& dv = vols[v];
         int x0, y0, z0;
         tile_origin<Shape>(dv.vp, tile, x0, y0, z0);

@@ -8,6 +8,8 @@
 
 #include "recon_common.hpp"
 
+#include <type_traits>
+
 namespace recon {
 
 constexpr int kThreads = 256;
@@ -44,6 +46,13 @@ struct ListEntry {
     uint32_t volume;   // volume index (batched path), 0 otherwise
     uint64_t frames;   // bit f: frame f of the volume may update the tile
 };
+
+// A list entry's frame mask as a wavefront-uniform value (readfirstlane gives
+// a signed 32-bit half, which must not be widened with its sign).
+__device__ __forceinline__ uint64_t uniform_mask(uint64_t m) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m);
+}
 
 // Max over a voxel-centre box of n.c + k.
 __device__ __forceinline__ float plane_max(const float* p, const float lo[3], const float hi[3]) {
@@ -361,10 +370,20 @@ __device__ __forceinline__ unsigned segment_slot(const unsigned* s_pre, int nseg
 }
 
 // ---- the per-voxel update -------------------------------------------------------
-// Projection is branch-free so the 4*NR depth gathers of a frame issue back
-// to back; D and W of a row are read only if one of its voxels passes, and
-// written once after all frames (frames are applied in order, so the result
-// equals one sweep per frame).
+// A wavefront takes a wave-tile; at step j its 64 lanes hold a patch of
+// LW x (64/LW) adjacent voxels of one z layer, so that a depth gather's lanes
+// land on neighbouring pixels, and its D and W accesses are runs of LW voxels
+// of a row (any gx: no vector alignment).  One frame per call is bound by
+// HBM (a 512^3 volume and a VGA frame move 377 MB at 4.5 TB/s, a large copy
+// 5.1): LW = 32, whole 128-byte rows (16 and 8 took 6 and 19 % longer).
+// Several frames are bound by the gathers (16 volumes of up to 40 frames of
+// 1280x720: address units 82 % busy, L2 misses at 6.2 TB/s, since a voxel
+// there spans about 6 pixels): the squarest patch.  Lanes of four voxels of a
+// row each, with its branches per voxel and IEEE divisions, took 818 M
+// instructions and 2.21 ms on that batch; this form takes 542 M and 1.95 ms,
+// and 40 HD frames into 301 x 237 x 174 with variance weights fell from 1127
+// to 999 us.  One test per frame and wavefront sends what the short
+// arithmetic does not cover to the divisions.
 //
 // COLOR (single-frame calls with a colour image): a voxel updated inside the
 // truncation band (-trunc <= sdf <= trunc) also averages the rgb pixel of its
@@ -376,157 +395,214 @@ __device__ __forceinline__ unsigned segment_slot(const unsigned* s_pre, int nseg
 // VARW (WEIGHT_BY_VARIANCE): an observation weighs
 // variance_weight(d) = sigma(1 m)^2 / sigma(d)^2 instead of 1, so
 // d' = ((d * w) + (wo * tsdf)) / (w + wo), w' = min(w + wo, max_weight).
-template <class S, class Frames, bool VEC, bool COUNT, bool COLOR = false, bool VARW = false>
-__device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const int nframes,
-                                               const Frames& frames, const uint64_t live,
-                                               const int x0, const int y0, const int z0,
-                                               unsigned& cnt, unsigned& touched,
-                                               const float* __restrict__ rtab = nullptr) {
-    constexpr int NR = S::kRows, NV = 4 * S::kRows;
-    float* __restrict__ D = vp.D;
-    float* __restrict__ W = vp.W;
+template <class S, int LW, class Frames, bool COUNT, bool COLOR = false, bool VARW = false>
+__device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Frames& frames,
+                                               const uint64_t live, const int x0, const int y0,
+                                               const int z0, unsigned& cnt, unsigned& touched) {
+    constexpr int LH = 64 / LW;                                // lanes in y
+    constexpr int NX = S::X / LW, NY = S::Y / LH, NR = S::Z;  // steps in x, y, z
+    constexpr int NV = NX * NY * NR;                          // voxels per lane
+    static_assert(NX * LW == S::X && NY * LH == S::Y, "lanes must tile the wave-tile");
+    constexpr bool kOne = Frames::kMax == 1;
     const int lane = threadIdx.x & 63;
-    const int x = x0 + 4 * (lane % S::kLanesX);
-    const int y = y0 + lane / S::kLanesX;
+    const int x = x0 + lane % LW, y = y0 + lane / LW;
     if (x >= vp.gx || y >= vp.gy) return;
-    const int nvox = VEC ? 4 : min(4, vp.gx - x);
-    int base[NR];
-    bool row_ok[NR];
-    float czw[NR];
+    // step j's voxel: (x + LW * jx, y + LH * jy, z0 + jz)
+    const auto jx = [](int j) { return j % NX; };
+    const auto jy = [](int j) { return (j / NX) % NY; };
+    const auto jz = [](int j) { return j / (NX * NY); };
+    bool in_grid[NV];
+    float cxw[NX], cyw[NY], czw[NR];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        const int z = z0 + r;
-        row_ok[r] = z < vp.gz;
-        base[r] = x + vp.gx * (y + vp.gy * min(z, vp.gz - 1));
-        czw[r] = voxel_centre(z, vp.vs[2], vp.off[2]);
-    }
-    const float cyw = voxel_centre(y, vp.vs[1], vp.off[1]);
-    float cxw[4];
+    for (int k = 0; k < NX; ++k) cxw[k] = voxel_centre(x + LW * k, vp.vs[0], vp.off[0]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) cxw[j] = voxel_centre(x + j, vp.vs[0], vp.off[0]);
+    for (int k = 0; k < NY; ++k) cyw[k] = voxel_centre(y + LH * k, vp.vs[1], vp.off[1]);
+#pragma unroll
+    for (int k = 0; k < NR; ++k) czw[k] = voxel_centre(z0 + k, vp.vs[2], vp.off[2]);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        in_grid[j] = (x + LW * jx(j) < vp.gx) & (y + LH * jy(j) < vp.gy) & (z0 + jz(j) < vp.gz);
+    // offset of step j's voxel from the lane's first, the same for all lanes
+    const auto step = [&](int j) {
+        return (int64_t)LW * jx(j) + (int64_t)vp.gx * (LH * jy(j) + (int64_t)vp.gy * jz(j));
+    };
+    // the tile's first voxel (uniform) and the lane's place from it
+    const int64_t first = x0 + (int64_t)vp.gx * (y0 + (int64_t)vp.gy * z0);
+    const int64_t place = lane % LW + (int64_t)vp.gx * (lane / LW);
+    GlobalFloat D = (GlobalFloat)vp.D + first, W = (GlobalFloat)vp.W + first;
+    // VARW: sigma within [1e-8, 1e8] keeps the weight's quotient normal
+    const float reach = vp.maxd + fabsf(vp.noise[2]);
+    const float guard_w =
+        VARW && !(vp.noise[0] >= 1e-8f && vp.noise[0] + vp.noise[1] * (reach * reach) <= 1e8f) ? INFINITY
+                                                                                             : 0.0f;
 
+    // several frames: D and W of the tile's voxels stay in registers, read
+    // before the first frame and written once after the last
     float d[NV], w[NV];
+    bool dirty[NV];
 #pragma unroll
-    for (int j = 0; j < NV; ++j) d[j] = w[j] = 0.0f;
-    bool loaded[NR], dirty[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) loaded[r] = dirty[r] = false;
+    for (int j = 0; j < NV; ++j) {
+        dirty[j] = false;
+        d[j] = w[j] = 0.0f;
+        if (!kOne && in_grid[j]) {
+            d[j] = D[place + step(j)];
+            w[j] = W[place + step(j)];
+        }
+    }
     unsigned upd = 0;  // COUNT: bit j set once voxel j is updated
 
-    // single-frame blocks: a compile-time trip count lets the frame loop
-    // unroll (91 -> 59 VGPRs for the plain kernel)
-    const int nf = Frames::kMax == 1 ? 1 : nframes;
-    for (int f = 0; f < nf; ++f) {
-        if (!((live >> f) & 1ull)) continue;
-        const FrameParams& F = frames.f[f];
-        const float rxy = F.R[1] * cyw, ryy = F.R[4] * cyw, rzy = F.R[7] * cyw;
+    // One frame, given the camera z and its reciprocals rz (exact: by the
+    // divisions instead): depth taps, pass test and update.
+    auto observe = [&](auto exact, const FrameParams& F, const float* pz, const float* rz) {
+        constexpr bool kExact = decltype(exact)::value;
         bool ok[NV];
-        float pz[NV], dep[NV];
-        int addr[NV];
-        int uu[COLOR ? NV : 1], vv[COLOR ? NV : 1];
+        float dep[NV];
+        int u[NV], v[NV];
+        uint32_t at[NV];
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const int r = j >> 2, i = j & 3;
-            const float px = ((F.R[0] * cxw[i] + rxy) + F.R[2] * czw[r]) + F.t[0];
-            const float py = ((F.R[3] * cxw[i] + ryy) + F.R[5] * czw[r]) + F.t[1];
-            pz[j] = ((F.R[6] * cxw[i] + rzy) + F.R[8] * czw[r]) + F.t[2];
-            int u, v;
-            const bool in_z = pz[j] > 0.0f;
-            const float rz = 1.0f / pz[j];  // one correctly rounded division for both axes
-            const bool in_u = pixel_index_rcp(px, vp.fx, pz[j], rz, vp.cx, vp.fcols, u);
-            const bool in_v = pixel_index_rcp(py, vp.fy, pz[j], rz, vp.cy, vp.frows, v);
-            ok[j] = in_z && in_u && in_v && row_ok[r] && (VEC || i < nvox);
-            addr[j] = ok[j] ? v * F.pitch + u : 0;
-            if (COLOR) {
-                uu[j] = u;
-                vv[j] = v;
+            const float cx = cxw[jx(j)], cy = cyw[jy(j)], cz = czw[jz(j)];
+            const float px = ((F.R[0] * cx + F.R[1] * cy) + F.R[2] * cz) + F.t[0];
+            const float py = ((F.R[3] * cx + F.R[4] * cy) + F.R[5] * cz) + F.t[1];
+            if (kExact) {
+                u[j] = v[j] = 0;
+                const bool in_u = pixel_index(px, vp.fx, pz[j], vp.cx, vp.fcols, u[j]);
+                const bool in_v = pixel_index(py, vp.fy, pz[j], vp.cy, vp.frows, v[j]);
+                ok[j] = (pz[j] > 0.0f) & in_u & in_v & in_grid[j];
+            } else {
+                // -1 < s < size is 0 <= (int)s < size
+                u[j] = to_int_sat(div_by_rcp(px * vp.fx, pz[j], rz[j]) + vp.cx);
+                v[j] = to_int_sat(div_by_rcp(py * vp.fy, pz[j], rz[j]) + vp.cy);
+                ok[j] = (pz[j] > 0.0f) & ((uint32_t)u[j] < (uint32_t)vp.cols) &
+                        ((uint32_t)v[j] < (uint32_t)vp.rows) & in_grid[j];
+                const uint32_t off = mul24((uint32_t)v[j], 4u * (uint32_t)F.pitch) + 4u * (uint32_t)u[j];
+                at[j] = ok[j] ? off : 0u;
             }
         }
 #pragma unroll
-        for (int j = 0; j < NV; ++j) dep[j] = F.depth[addr[j]];
-        bool pass[NV], any[NR], band[COLOR ? NV : 1];
+        for (int j = 0; j < NV; ++j)
+            dep[j] = kExact ? F.depth[ok[j] ? (int64_t)v[j] * F.pitch + u[j] : 0]
+                            : load_float((GlobalBytes)F.depth, at[j]);
+        bool pass[NV], band[COLOR ? NV : 1];
         float tsdf[NV];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) any[r] = false;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const float sdf = dep[j] - pz[j];
-            pass[j] = ok[j] && !(dep[j] <= 0.0f || dep[j] > vp.maxd) && (sdf >= -vp.trunc);
-            tsdf[j] = sdf > 0.0f ? fminf(sdf, vp.trunc) : sdf;
-            any[j >> 2] = any[j >> 2] || pass[j];
+            pass[j] = ok[j] & (dep[j] > 0.0f) & (dep[j] <= vp.maxd) & (sdf >= -vp.trunc);
+            tsdf[j] = min_bound(vp.trunc, sdf);
             if (COLOR) band[j] = sdf <= vp.trunc;
         }
+        const uint32_t place4 = 4u * (uint32_t)place;  // below 2^32 unless exact
+        if (kOne) {
+            // read back to back what the frame updates
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (pass[j]) {
+                    d[j] = kExact ? D[place + step(j)] : load_float((GlobalBytes)(D + step(j)), place4);
+                    w[j] = kExact ? W[place + step(j)] : load_float((GlobalBytes)(W + step(j)), place4);
+                }
+        }
+        constexpr int G = NX * NY;  // voxels of a layer share the test for the short forms
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
-            if (any[r] && !loaded[r]) {
-                if (VEC) {
-                    const float4 d4 = *reinterpret_cast<const float4*>(D + base[r]);
-                    const float4 w4 = *reinterpret_cast<const float4*>(W + base[r]);
-                    d[4 * r + 0] = d4.x; d[4 * r + 1] = d4.y; d[4 * r + 2] = d4.z; d[4 * r + 3] = d4.w;
-                    w[4 * r + 0] = w4.x; w[4 * r + 1] = w4.y; w[4 * r + 2] = w4.z; w[4 * r + 3] = w4.w;
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < G; ++i) any |= pass[G * r + i];
+            if (!any) continue;
+            // tsdf_volume.cu:178-186 with the weight cap
+            float num[G], nw[G], nd[G], bad = guard_w;
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int j = G * r + i;
+                if (VARW) {
+                    const float e = dep[j] - vp.noise[2];
+                    const float sig = vp.noise[0] + (vp.noise[1] * (e * e));
+                    const float s2 = sig * sig;
+                    const float wo = div_by_rcp(vp.wref, s2, recip_sum(s2, bad));
+                    nw[i] = w[j] + wo;
+                    num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
+                    // a quotient near the denormals is left to the division
+                    bad = pass[j] & !(fabsf(num[i]) >= 1e-30f) ? INFINITY : bad;
                 } else {
-                    for (int i = 0; i < nvox; ++i) {
-                        d[4 * r + i] = D[base[r] + i];
-                        w[4 * r + i] = W[base[r] + i];
-                    }
+                    nw[i] = w[j] + 1.0f;
+                    num[i] = (d[j] * w[j]) + tsdf[j];
                 }
-                loaded[r] = true;
+                nd[i] = div_by_rcp(num[i], nw[i], recip_sum(nw[i], bad));
+            }
+            if (__builtin_expect(__ballot(!(bad < kRecipBad)) != 0, 0)) {
+#pragma unroll
+                for (int i = 0; i < G; ++i) {
+                    const int j = G * r + i;
+                    if (VARW) {
+                        const float wo = variance_weight(vp.noise, vp.wref, dep[j]);
+                        nw[i] = w[j] + wo;
+                        num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
+                    }
+                    nd[i] = num[i] / nw[i];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int j = G * r + i;
+                const float w2 = min_bound(vp.maxw, nw[i]);
+                if (kOne) {
+                    if (pass[j]) {
+                        if (kExact) {
+                            D[place + step(j)] = nd[i];
+                            W[place + step(j)] = w2;
+                        } else {
+                            store_float((GlobalBytes)(D + step(j)), place4, nd[i]);
+                            store_float((GlobalBytes)(W + step(j)), place4, w2);
+                        }
+                    }
+                } else {
+                    d[j] = pass[j] ? nd[i] : d[j];
+                    w[j] = pass[j] ? w2 : w[j];
+                    dirty[j] |= pass[j];
+                }
+                if (COUNT && pass[j]) {
+                    ++cnt;
+                    upd |= 1u << j;
+                }
+                if (COLOR && pass[j] && band[j]) {
+                    float4* cp = reinterpret_cast<float4*>(vp.C) + first + place + step(j);
+                    float4 c = *cp;
+                    const uint8_t* q = F.rgb + (int64_t)v[j] * F.rgb_pitch + 3 * u[j];
+                    const float nwc = c.w + 1.0f;
+                    c.x = ((c.x * c.w) + (float)q[0]) / nwc;
+                    c.y = ((c.y * c.w) + (float)q[1]) / nwc;
+                    c.z = ((c.z * c.w) + (float)q[2]) / nwc;
+                    c.w = nwc < vp.maxw ? nwc : vp.maxw;
+                    *cp = c;
+                }
             }
         }
+    };
+    uint64_t rest = live;
+    do {
+        const int f = kOne ? 0 : (int)__builtin_ctzll(rest);
+        rest &= rest - 1;
+        const FrameParams& F = frames.f[f];
+        float pz[NV], rz[NV];
+        float bad = F.guard;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            if (!pass[j]) continue;
-            // tsdf_volume.cu:178-186 with the weight cap
-            if (VARW) {
-                const float wo = variance_weight(vp.noise, vp.wref, dep[j]);
-                const float nw = w[j] + wo;
-                d[j] = ((d[j] * w[j]) + (wo * tsdf[j])) / nw;
-                w[j] = nw < vp.maxw ? nw : vp.maxw;
-            } else {
-                const float nw = w[j] + 1.0f;
-                const float num = (d[j] * w[j]) + tsdf[j];
-                // weights are whole counts below the cap: RN(1/nw) from rtab
-                // (rtab[i] = 1.0f / (i + 1)) and div_by_rcp, else the division
-                const int wi = (int)w[j];
-                if (rtab && (float)wi == w[j] && wi < kRcpTable)
-                    d[j] = div_by_rcp(num, nw, rtab[wi]);
-                else
-                    d[j] = num / nw;
-                w[j] = nw < vp.maxw ? nw : vp.maxw;
-            }
-            dirty[j >> 2] = true;
-            if (COUNT) {
-                ++cnt;
-                upd |= 1u << j;
-            }
-            if (COLOR && band[j]) {
-                float4* cp = reinterpret_cast<float4*>(vp.C) + base[j >> 2] + (j & 3);
-                float4 c = *cp;
-                const uint8_t* px = F.rgb + (int64_t)vv[j] * F.rgb_pitch + 3 * uu[j];
-                const float nwc = c.w + 1.0f;
-                c.x = ((c.x * c.w) + (float)px[0]) / nwc;
-                c.y = ((c.y * c.w) + (float)px[1]) / nwc;
-                c.z = ((c.z * c.w) + (float)px[2]) / nwc;
-                c.w = nwc < vp.maxw ? nwc : vp.maxw;
-                *cp = c;
-            }
+            pz[j] = ((F.R[6] * cxw[jx(j)] + F.R[7] * cyw[jy(j)]) + F.R[8] * czw[jz(j)]) + F.t[2];
+            rz[j] = recip(pz[j], bad);  // serves both axes
         }
-    }
+        if (__builtin_expect(__ballot(bad > kRecipBad) == 0, 1))
+            observe(std::false_type{}, F, pz, rz);
+        else
+            observe(std::true_type{}, F, pz, rz);
+    } while (!kOne && rest);
     if (COUNT) touched += (unsigned)__builtin_popcount(upd);
+    if (!kOne) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        if (!dirty[r]) continue;
-        if (VEC) {
-            *reinterpret_cast<float4*>(D + base[r]) =
-                make_float4(d[4 * r + 0], d[4 * r + 1], d[4 * r + 2], d[4 * r + 3]);
-            *reinterpret_cast<float4*>(W + base[r]) =
-                make_float4(w[4 * r + 0], w[4 * r + 1], w[4 * r + 2], w[4 * r + 3]);
-        } else {
-            for (int i = 0; i < nvox; ++i) {
-                D[base[r] + i] = d[4 * r + i];
-                W[base[r] + i] = w[4 * r + i];
+        for (int j = 0; j < NV; ++j)
+            if (dirty[j]) {
+                D[place + step(j)] = d[j];
+                W[place + step(j)] = w[j];
             }
-        }
     }
 }
 

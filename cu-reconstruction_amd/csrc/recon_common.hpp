@@ -69,6 +69,7 @@ struct FrameParams {
     float zmargin;   // bound on float32 error of a camera z: 1e-6 * (|t| + max|c|)
     const uint8_t* rgb = nullptr;  // colour image (rgb triples) of the colour integrate
     int32_t rgb_pitch = 0;         // bytes per colour row
+    float guard;     // 0, or infinity when the kernels' short forms do not cover the frame
 };
 
 constexpr int kBound0 = 8, kBound1 = 32;  // pixel block edges of the two bound levels
@@ -128,6 +129,17 @@ __host__ __device__ inline void frame_planes(const VolumeParams& vp, FrameParams
     }
     const double tabs = ::fabs((double)fp->t[0]) + ::fabs((double)fp->t[1]) + ::fabs((double)fp->t[2]);
     fp->zmargin = (float)(1e-6 * (tabs + cmax[0] + cmax[1] + cmax[2]) + 1e-6);
+    // The short forms need camera coordinates and pixel products far from
+    // overflow, row bytes and row numbers below 2^24 (24-bit products), and
+    // 32-bit byte offsets within an image and within a wave-tile; anything
+    // else takes the divisions and 64-bit addresses.
+    double rabs = 0.0;
+    for (int i = 0; i < 9; ++i) rabs += ::fabs((double)fp->R[i]);
+    const double reach = rabs * (cmax[0] + cmax[1] + cmax[2]) + tabs;
+    const bool easy = reach * (::fabs(fx) + ::fabs(fy) + 1.0) < 1e30 && ::fabs(cx) + ::fabs(cy) < 1e30 &&
+                      fp->pitch < (1 << 22) && vp.rows < (1 << 24) && vp.gx < (1 << 26) &&
+                      4.0 * (double)fp->pitch * vp.rows < 4294967296.0;
+    fp->guard = easy ? 0.0f : __builtin_inff();
     for (int k = 0; k < 6; ++k) {
         double n[3];
         for (int i = 0; i < 3; ++i)  // n = R^T a
@@ -223,17 +235,66 @@ __device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
     return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
 }
 
-// pixel_index with rz = RN(1/pz) (1.0f / pz) shared by both axes: the same
-// index and validity.  Outside the normal range (pz near 0, or an overflow)
-// both quotients are infinite, NaN or below ulp(c) / 2, and both indices
-// invalid or equal after + c and the truncation.
-__device__ __forceinline__ bool pixel_index_rcp(float pa, float f, float pz, float rz, float c,
-                                                float size, int& out) {
-    const float s = div_by_rcp(pa * f, pz, rz) + c;
-    if (!(s > -1.0f && s < size)) return false;
-    out = (int)s;
-    return true;
+// RN(1/x): v_rcp_f32 and one Newton step, 3 instructions where the division
+// takes 11.  On gfx950 the step lands on the correctly rounded reciprocal for
+// every significand (tests/test_gpu_recip.py compares all of them with the
+// division); the residual e = 1 - x*y is then below 2^-22.  Where x or 1/x
+// is not a normal number, e is large (the estimate is 0 or infinite) and the
+// caller, having taken the largest |e| of its lanes, divides instead when it
+// exceeds kRecipBad.  A NaN residual (x zero, infinite or NaN) is not seen by
+// recip's maximum, which is for callers whose result is discarded for such x;
+// recip_sum carries it.
+constexpr float kRecipBad = 1e-3f;
+
+__device__ __forceinline__ float recip(float x, float& bad) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    const float e = __builtin_fmaf(-x, y, 1.0f);
+    bad = fmaxf(bad, fabsf(e));
+    return __builtin_fmaf(e, y, y);
 }
 
+__device__ __forceinline__ float recip_sum(float x, float& bad) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    const float e = __builtin_fmaf(-x, y, 1.0f);
+    bad = bad + fabsf(e);
+    return __builtin_fmaf(e, y, y);
+}
+
+// (int)s for any s: v_cvt_i32_f32 truncates, saturates and takes NaN to 0
+// (the language leaves out-of-range conversions undefined).
+__device__ __forceinline__ int to_int_sat(float s) {
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(s));
+    return i;
+}
+
+// The smaller of a wavefront-uniform bound and a value, without the
+// canonicalisation that fminf adds to operands of unknown origin.
+__device__ __forceinline__ float min_bound(float bound, float v) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "s"(bound), "v"(v));
+    return r;
+}
+
+// Low 32 bits of the product of two numbers below 2^24 (v_mul_u32_u24).
+__device__ __forceinline__ uint32_t mul24(uint32_t a, uint32_t b) {
+    return (a & 0xFFFFFFu) * (b & 0xFFFFFFu);
+}
+
+// Device memory as such: pointers read from a table would give flat
+// accesses.  load_float and store_float take a wavefront-uniform base and a
+// 32-bit byte offset per lane (the scalar-base form of the instructions).
+using GlobalFloat = __attribute__((address_space(1))) float*;
+using GlobalBytes = __attribute__((address_space(1))) char*;
+
+__device__ __forceinline__ float load_float(GlobalBytes base, uint32_t off) {
+    asm("" : "+v"(off));  // keeps the offset 32 bits wide up to the access
+    return *(GlobalFloat)(base + off);
+}
+
+__device__ __forceinline__ void store_float(GlobalBytes base, uint32_t off, float v) {
+    asm("" : "+v"(off));
+    *(GlobalFloat)(base + off) = v;
+}
 
 }  // namespace recon

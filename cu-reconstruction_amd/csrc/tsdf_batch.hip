@@ -119,19 +119,12 @@ __global__ __launch_bounds__(kThreads) void batch_integrate_kernel(
     for (unsigned i = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); i < n; i += waves) {
         const uint32_t tile = __builtin_amdgcn_readfirstlane(list[i].tile);
         const uint32_t v = __builtin_amdgcn_readfirstlane(list[i].volume);
-        const uint64_t mask =
-            ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(list[i].frames >> 32)) << 32) |
-            __builtin_amdgcn_readfirstlane((uint32_t)list[i].frames);
+        const uint64_t mask = uniform_mask(list[i].frames);
         const BatchVolParams& bv = vols[v];
         int x0, y0, z0;
         tile_origin<S>(bv.vp, tile, x0, y0, z0);
         const FrameTable ft{frames + bv.first_frame};
-        if (bv.vp.gx % 4 == 0)
-            integrate_tile<S, FrameTable, true, false>(bv.vp, bv.nframes, ft, mask, x0, y0, z0, cnt,
-                                                       cnt);
-        else
-            integrate_tile<S, FrameTable, false, false>(bv.vp, bv.nframes, ft, mask, x0, y0, z0, cnt,
-                                                        cnt);
+        integrate_tile<S, S::X / 4, FrameTable, false>(bv.vp, ft, mask, x0, y0, z0, cnt, cnt);
     }
 }
 

@@ -105,9 +105,7 @@ __global__ __launch_bounds__(kThreads) void diff_integrate_kernel(
     const unsigned waves = gridDim.x * (kThreads / 64);
     for (unsigned i = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); i < n; i += waves) {
         const uint32_t tile = __builtin_amdgcn_readfirstlane(list[i].tile);
-        const uint64_t frames =
-            ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(list[i].frames >> 32)) << 32) |
-            __builtin_amdgcn_readfirstlane((uint32_t)list[i].frames);
+        const uint64_t frames = uniform_mask(list[i].frames);
         int x0, y0, z0;
         tile_origin<Shape>(vp, tile, x0, y0, z0);
         diff_integrate_tile<Shape, FrameTable, VEC>(vp, nframes, ft, frames, x0, y0, z0, rtab);

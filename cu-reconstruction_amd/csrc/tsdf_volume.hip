@@ -76,20 +76,23 @@ __global__ __launch_bounds__(256) void cull_kernel(const VolumeParams vp, const 
     if (threadIdx.x == 0) counts[blockIdx.x] = n;
 }
 
+// Voxels of a row that a wavefront's lanes hold side by side
+// (integrate_tile's LW).
+template <int MAXF>
+constexpr int kLaneRow = MAXF == 1 ? 32 : 8;
+
 // The list's entries in dense order i = 0 .. total-1 (segment by segment):
 // each wavefront takes i = wave, wave + waves, ... (the grid is sized to the
 // resident wave slots, so every wave-tile costs about the same and the device
 // stays full until the list is done); lane j of a wave locates the list slot
 // of the wave's j-th next entry, so one search serves 64 entries.
-template <int MAXF, bool VEC, bool COUNT, bool COLOR = false, bool VARW = false>
+template <int MAXF, bool COUNT, bool COLOR = false, bool VARW = false>
 __global__ __launch_bounds__(kThreads) void integrate_list_kernel(
     const VolumeParams vp, const int nframes, const FrameBlock<MAXF> fb,
     const ListEntry* __restrict__ list, const unsigned* __restrict__ counts, const int nseg,
     const unsigned seg_len, unsigned long long* counter, unsigned long long* touch_counter) {
     __shared__ unsigned s_pre[kMaxSegments + 1];
     __shared__ unsigned s_wave[kThreads / 64];
-    __shared__ float rtab[kRcpTable];
-    rtab[threadIdx.x] = 1.0f / (float)(threadIdx.x + 1);  // ordered by segment_offsets' barrier
     const unsigned n = __builtin_amdgcn_readfirstlane(segment_offsets(counts, nseg, s_pre, s_wave));
     const unsigned waves = gridDim.x * (kThreads / 64);
     const unsigned lane = threadIdx.x & 63;
@@ -101,14 +104,11 @@ __global__ __launch_bounds__(kThreads) void integrate_list_kernel(
         for (unsigned j = 0; j < m; ++j) {
             const unsigned e = __builtin_amdgcn_readfirstlane(__shfl(slot, (int)j, 64));
             const uint32_t tile = __builtin_amdgcn_readfirstlane(list[e].tile);
-            const uint64_t frames =
-                ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(list[e].frames >> 32)) << 32) |
-                __builtin_amdgcn_readfirstlane((uint32_t)list[e].frames);
+            const uint64_t frames = uniform_mask(list[e].frames);
             int x0, y0, z0;
             tile_origin<Shape>(vp, tile, x0, y0, z0);
-            integrate_tile<Shape, FrameBlock<MAXF>, VEC, COUNT, COLOR, VARW>(vp, nframes, fb, frames,
-                                                                             x0, y0, z0, cnt,
-                                                                             touched, rtab);
+            integrate_tile<Shape, kLaneRow<MAXF>, FrameBlock<MAXF>, COUNT, COLOR, VARW>(
+                vp, fb, frames, x0, y0, z0, cnt, touched);
         }
     }
     if (COUNT && counter && cnt) atomicAdd(counter, (unsigned long long)cnt);
@@ -214,12 +214,12 @@ constexpr int kListMaxBlocksPerCU = 5;
 // slots (capped).  The grid never exceeds the resident slots, because every
 // wave takes the same share of the list and a workgroup beyond them would
 // start only when another has finished its share.
-template <int MAXF, bool VEC, bool COUNT, bool COLOR, bool VARW>
+template <int MAXF, bool COUNT, bool COLOR, bool VARW>
 static int list_occupancy() {
     static const int blocks = [] {
         int b = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &b, integrate_list_kernel<MAXF, VEC, COUNT, COLOR, VARW>, kThreads, 0) != hipSuccess ||
+                &b, integrate_list_kernel<MAXF, COUNT, COLOR, VARW>, kThreads, 0) != hipSuccess ||
             b < 1)
             b = 1;
         return std::min(b, kListMaxBlocksPerCU);
@@ -227,18 +227,18 @@ static int list_occupancy() {
     return blocks;
 }
 
-template <int MAXF, bool VEC, bool COUNT, bool COLOR>
+template <int MAXF, bool COUNT, bool COLOR>
 static void launch_list(bool varw, int num_cus, hipStream_t s, const VolumeParams& vp, int nframes,
                         const FrameBlock<MAXF>& fb, const ListArgs& la, unsigned long long* ctr,
                         unsigned long long* tctr) {
     if (varw)
-        hipLaunchKernelGGL((integrate_list_kernel<MAXF, VEC, COUNT, COLOR, true>),
-                           dim3(num_cus * list_occupancy<MAXF, VEC, COUNT, COLOR, true>()),
+        hipLaunchKernelGGL((integrate_list_kernel<MAXF, COUNT, COLOR, true>),
+                           dim3(num_cus * list_occupancy<MAXF, COUNT, COLOR, true>()),
                            dim3(kThreads), 0, s, vp, nframes, fb, la.list, la.counts, la.nseg,
                            la.seg_len, ctr, tctr);
     else
-        hipLaunchKernelGGL((integrate_list_kernel<MAXF, VEC, COUNT, COLOR, false>),
-                           dim3(num_cus * list_occupancy<MAXF, VEC, COUNT, COLOR, false>()),
+        hipLaunchKernelGGL((integrate_list_kernel<MAXF, COUNT, COLOR, false>),
+                           dim3(num_cus * list_occupancy<MAXF, COUNT, COLOR, false>()),
                            dim3(kThreads), 0, s, vp, nframes, fb, la.list, la.counts, la.nseg,
                            la.seg_len, ctr, tctr);
 }
@@ -286,29 +286,18 @@ static int launch_prestage(const VolumeParams& vp, const float* depth0, size_t s
 template <int MAXF>
 static int launch_liststage(recon_tsdf* h, const VolumeParams& vp, int nframes,
                             const FrameBlock<MAXF>& fb, const ListArgs& la, hipStream_t s) {
-    const bool vec = (vp.gx % 4) == 0;
     const bool varw = h->info.weight_type == RECON_WEIGHT_BY_VARIANCE;
     unsigned long long* ctr = h->update_counter;
     unsigned long long* tctr = h->touch_counter;
     bool color = false;
     if constexpr (MAXF == 1) color = fb.f[0].rgb && vp.C;  // colour integrate (no counting)
     if (color) {
-        if constexpr (MAXF == 1) {
-            if (vec)
-                launch_list<1, true, false, true>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
-            else
-                launch_list<1, false, false, true>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
-        }
+        if constexpr (MAXF == 1)
+            launch_list<1, false, true>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
     } else if (ctr || tctr) {
-        if (vec)
-            launch_list<MAXF, true, true, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
-        else
-            launch_list<MAXF, false, true, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
+        launch_list<MAXF, true, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
     } else {
-        if (vec)
-            launch_list<MAXF, true, false, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
-        else
-            launch_list<MAXF, false, false, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
+        launch_list<MAXF, false, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
     }
     RECON_HIP_TRY(hipGetLastError(), "integrate_list_kernel launch");
     return RECON_OK;

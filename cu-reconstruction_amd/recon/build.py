@@ -5,6 +5,7 @@ Outputs (all under cu-reconstruction_amd/lib/):
   librecon_host.so   C++ drop-in mirror of the reference's TSDF API over the C-ABI
   librecon_scene.so  synthetic depth renderer (host C++)
   tsdf_wrapper_test  C++ program exercising librecon_host.so (run by a GPU test)
+  recip_test         the kernels' reciprocal against the division (run by a GPU test)
 and oracle/lib/liboracle.so through oracle/Makefile (the CPU checker).
 
 Every call compiles from scratch.  Device code is built with IEEE float32
@@ -106,6 +107,11 @@ def build(verbose: bool = False, jobs: int = 8) -> dict[str, Path]:
                   f"-L{LIB}", f"-L{oracle_lib}", "-lrecon_host", "-lrecon", "-lrecon_scene",
                   "-loracle", "-Wl,-rpath,$ORIGIN:$ORIGIN/../../oracle/lib", "-o", exe], verbose)
             out["wrapper_test"] = exe
+    recip_src = ROOT / "tests" / "cpp" / "recip_test.hip"
+    if recip_src.exists():
+        exe = LIB / "recip_test"
+        _run([HIPCC, *HIP_FLAGS, recip_src, "-o", exe], verbose)
+        out["recip_test"] = exe
     return out
 
 
