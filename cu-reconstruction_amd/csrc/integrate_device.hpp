@@ -73,6 +73,18 @@ __device__ __forceinline__ void tile_origin(const VolumeParams& vp, uint32_t id,
     z0 = (int)(tyz / (uint32_t)vp.tiles_y) * S::Z;
 }
 
+// The box of a wave-tile's voxel centres.
+template <class S>
+__device__ __forceinline__ void tile_box(const VolumeParams& vp, int x0, int y0, int z0, float lo[3],
+                                         float hi[3]) {
+    lo[0] = voxel_centre(x0, vp.vs[0], vp.off[0]);
+    lo[1] = voxel_centre(y0, vp.vs[1], vp.off[1]);
+    lo[2] = voxel_centre(z0, vp.vs[2], vp.off[2]);
+    hi[0] = voxel_centre(min(x0 + S::X - 1, vp.gx - 1), vp.vs[0], vp.off[0]);
+    hi[1] = voxel_centre(min(y0 + S::Y - 1, vp.gy - 1), vp.vs[1], vp.off[1]);
+    hi[2] = voxel_centre(min(z0 + S::Z - 1, vp.gz - 1), vp.vs[2], vp.off[2]);
+}
+
 // ---- depth bounds -------------------------------------------------------------
 // One 32x32 pixel block (workgroup of 256 threads): the largest valid depth
 // (0 < d <= maxd) of each 8x8 sub-block into bound0 and of the block into
@@ -216,12 +228,7 @@ __device__ __forceinline__ uint64_t tile_frames(const VolumeParams& vp, const in
     int x0, y0, z0;
     tile_origin<S>(vp, id, x0, y0, z0);
     float lo[3], hi[3];
-    lo[0] = voxel_centre(x0, vp.vs[0], vp.off[0]);
-    lo[1] = voxel_centre(y0, vp.vs[1], vp.off[1]);
-    lo[2] = voxel_centre(z0, vp.vs[2], vp.off[2]);
-    hi[0] = voxel_centre(min(x0 + S::X - 1, vp.gx - 1), vp.vs[0], vp.off[0]);
-    hi[1] = voxel_centre(min(y0 + S::Y - 1, vp.gy - 1), vp.vs[1], vp.off[1]);
-    hi[2] = voxel_centre(min(z0 + S::Z - 1, vp.gz - 1), vp.vs[2], vp.off[2]);
+    tile_box<S>(vp, x0, y0, z0, lo, hi);
     uint64_t live = 0;
     for (int f = first; f < nframes; f += step)
         if (box_reaches<kMaxFine>(vp, frames.f[f], lo, hi)) live |= 1ull << f;

@@ -9,6 +9,7 @@ import pytest
 
 from helpers import assert_bitexact, gpu_run, oracle_run
 
+import recon
 from recon import scenes
 
 pytestmark = pytest.mark.gpu
@@ -207,3 +208,28 @@ def test_touch_counter_is_union_per_sweep(cuda):
     assert_bitexact(Wg, W, "fused W")
     assert_bitexact(Dg, D, "fused D")
     vol.close()
+
+
+@pytest.mark.parametrize("weight_type", [0, 1])
+@pytest.mark.parametrize("grid", [(1, 1, 1), (31, 7, 1), (33, 9, 3), (65, 17, 9), (37, 64, 50),
+                                  (256, 256, 256), (256, 256, 257)])
+def test_direct_and_list_kernels_agree(cuda, grid, weight_type):
+    """Small volumes take one launch without cull or list; a counted call
+    takes the list kernel at any size: equal bits, on both sides of the size
+    rule (32768 wave-tiles of 32 x 8 x 2) and at ragged edges."""
+    w = scenes.tiny(grid=grid, voxel_size=0.8 / max(grid), image=(96, 72), num_frames=3)
+    depth = cuda.from_numpy(w.render()).cuda()
+    cfg = w.config()
+    cfg.weight_type = weight_type
+    counter = cuda.zeros(1, dtype=cuda.int64, device="cuda")
+    got = []
+    for counted in (False, True):
+        v = recon.TSDFVolume(cfg)
+        v.set_update_counter(counter if counted else None)
+        for f in range(w.num_frames):
+            v.integrate(depth[f], w.poses[f])
+        cuda.cuda.synchronize()
+        got.append(v.download())
+        v.close()
+    assert_bitexact(got[0][0], got[1][0], "D")
+    assert_bitexact(got[0][1], got[1][1], "W")
