@@ -41,7 +41,12 @@
 namespace recon {
 
 using Shape = DefaultShape;
-constexpr int kUnit = 1024;          // merged pairs per adjoint work unit
+// Merged pairs per adjoint work unit (one wavefront, 64 / frames pairs a
+// pass): a pass is a chain of dependent loads, so a unit is short enough for
+// a few fragments to fill the device (8 fragments of 128^3, 10 frames: 322 us
+// with 1024 pairs a unit, 59 with 128).
+constexpr int kUnit = 128;
+constexpr int kFrameChunks = 8;      // workgroups per frame of the model-to-frame term
 constexpr int kMaxWaves = 8192;      // bound on the adjoint grid
 constexpr int kFill = 1024;          // voxels per fill workgroup
 
@@ -199,13 +204,34 @@ __global__ __launch_bounds__(256) void dbatch_loss_kernel(const DVol* __restrict
 }
 
 // Each volume's loss: its blocks' partials summed in the order of the
-// single-volume path's fixed_sum_kernel, times 1/K.
+// single-volume path's fixed_sum_kernel, times 1/K.  With the model-to-frame
+// term (ncomp of its sums per frame and chunk in fpart, else 0): the sums of
+// the volume's frames, chunks in order, into floss, fgrad and fhess, and
+// their losses added in frame order.
 __global__ __launch_bounds__(256) void dbatch_loss_sum_kernel(const DVol* __restrict__ vols,
                                                               const double* __restrict__ partials,
-                                                              const double* __restrict__ floss,
+                                                              const double* __restrict__ fpart,
+                                                              int ncomp, double* __restrict__ floss,
+                                                              double* __restrict__ fgrad,
+                                                              double* __restrict__ fhess,
                                                               double* __restrict__ loss) {
     __shared__ double s[256];
+    __shared__ double s_frame[64];
     const DVol& dv = vols[blockIdx.x];
+    const double fscale = dv.nfpairs > 0 ? dv.fweight / (double)dv.nfpairs : 0.0;
+    for (int i = threadIdx.x; i < dv.nframes * ncomp; i += 256) {
+        const int f = i / ncomp, c = i - f * ncomp, g = dv.first_frame + f;
+        const double* q = fpart + (size_t)g * kFrameChunks * ncomp + c;
+        double v[kFrameChunks];
+#pragma unroll
+        for (int k = 0; k < kFrameChunks; ++k) v[k] = q[(size_t)k * ncomp];
+        double sum = v[0];
+#pragma unroll
+        for (int k = 1; k < kFrameChunks; ++k) sum += v[k];
+        if (c == 0) floss[g] = s_frame[f] = sum * fscale;
+        else if (c < 7) fgrad[6 * g + c - 1] = sum;
+        else fhess[21 * g + c - 7] = 2.0 * fscale * sum;
+    }
     const double* src = partials + dv.first_loss_block;
     double acc = 0.0;
     for (int i = threadIdx.x; i < dv.nloss_blocks; i += 256) acc += src[i];
@@ -217,22 +243,25 @@ __global__ __launch_bounds__(256) void dbatch_loss_sum_kernel(const DVol* __rest
     }
     if (threadIdx.x == 0) {
         double l = dv.npoints > 0 ? s[0] * (1.0 / (double)dv.npoints) : 0.0;
-        if (floss && dv.nfpairs > 0)
-            for (int f = 0; f < dv.nframes; ++f) l += floss[dv.first_frame + f];
+        if (ncomp && dv.nfpairs > 0)
+            for (int f = 0; f < dv.nframes; ++f) l += s_frame[f];
         loss[blockIdx.x] = l;
     }
 }
 
-// Model-to-frame term: one workgroup per frame g over its pairs
-// [fr_range[2g], fr_range[2g+1]) of its volume, in float64 (the frame table's
-// float32 R, t widened): the weighted sum of min(r^2, tau^2) / K into
-// floss[g] (a truncated residual has no gradient) and its
-// gradient w.r.t. the frame's left perturbation into fgrad[6g..6g+5] (the
-// adjoint's formula at the point), each summed in a fixed order.  tau is the
+// Model-to-frame term: workgroup (g, k) takes the k-th of kFrameChunks equal
+// parts of frame g's pairs [fr_range[2g], fr_range[2g+1]) of its volume (one
+// workgroup per frame left most of the device idle: 117 us for 80 frames of
+// 4000 pairs, 33 now), in float64 (the frame table's
+// float32 R, t widened): the sum of min(r^2, tau^2) (a truncated residual has
+// no gradient) and the loss's gradient w.r.t. the frame's left perturbation
+// (the adjoint's formula at the point) into the part's slots of fpart, each
+// summed in a fixed order; dbatch_loss_sum_kernel adds the parts and scales
+// them to floss[g], fgrad[6g..6g+5] and fhess[21g..21g+20].  tau is the
 // volume's truncation, times ratio^min(1, step / ka) when `anneal` is given
 // (Gauss-Newton refinement).  With kHess, the frame's Gauss-Newton system
 // instead: fgrad = fweight * 2 sum r J / K and the upper triangle of
-// fweight * 2 sum J J^T / K into fhess[21g..21g+20] (row-major), over the
+// fweight * 2 sum J J^T / K (fhess, row-major), over the
 // pairs with |r| < tau, J = (j, p x j): j = -(z / (n . p)) n with n the
 // point's normal in the camera frame (point-to-plane; |n . p| < 0.1 |n| |p|
 // adds nothing) when the volume has normals, else the bilinear slopes'
@@ -246,15 +275,16 @@ template <bool kHess>
 __global__ __launch_bounds__(256) void dbatch_frame_loss_kernel(
     const DVol* __restrict__ vols, const DFrame* __restrict__ fr,
     const FrameParams* __restrict__ table, const int64_t* __restrict__ fr_range,
-    const FrameAnneal anneal, double* __restrict__ floss, double* __restrict__ fgrad,
-    double* __restrict__ fhess) {
+    const FrameAnneal anneal, double* __restrict__ fpart) {
     constexpr int kAcc = kHess ? 28 : 7;
     __shared__ double s_red[kAcc][4];
     const int g = blockIdx.x;
     const DVol& dv = vols[fr[g].volume];
     const VolumeParams& vp = dv.vp;
     const FrameParams& L = table[g];
-    const int64_t k0 = fr_range[2 * g], k1 = fr_range[2 * g + 1];
+    const int64_t all0 = fr_range[2 * g], all1 = fr_range[2 * g + 1];
+    const int64_t part = (all1 - all0 + kFrameChunks - 1) / kFrameChunks;
+    const int64_t k0 = min(all0 + part * (int64_t)blockIdx.y, all1), k1 = min(k0 + part, all1);
     const double scale = dv.nfpairs > 0 ? dv.fweight / (double)dv.nfpairs : 0.0;
     double tau = dv.ftrunc;
     if (anneal.step) tau *= pow(anneal.ratio, fmin(1.0, (double)*anneal.step / anneal.ka));
@@ -351,10 +381,8 @@ __global__ __launch_bounds__(256) void dbatch_frame_loss_kernel(
     __syncthreads();
     if (threadIdx.x < kAcc) {
         const int c = threadIdx.x;
-        const double sum = ((s_red[c][0] + s_red[c][1]) + s_red[c][2]) + s_red[c][3];
-        if (c == 0) floss[g] = sum * scale;
-        else if (c < 7) fgrad[6 * g + c - 1] = sum;
-        else fhess[21 * g + c - 7] = 2.0 * scale * sum;
+        fpart[((size_t)g * kFrameChunks + blockIdx.y) * kAcc + c] =
+            ((s_red[c][0] + s_red[c][1]) + s_red[c][2]) + s_red[c][3];
     }
 }
 
@@ -392,7 +420,7 @@ __global__ __launch_bounds__(256) void dbatch_units_kernel(const DVol* __restric
 __global__ __launch_bounds__(256) void dbatch_adjoint_kernel(
     const DVol* __restrict__ vols, int nvol, const FrameParams* __restrict__ table,
     const uint32_t* __restrict__ uid, const float* __restrict__ lam_u,
-    const long long* __restrict__ beg, const long long* __restrict__ unit_start,
+    const long long* __restrict__ beg, const long long* __restrict__ unit_start, const int max_frames,
     double* __restrict__ partial) {
     const unsigned waves = gridDim.x * 4u;
     const unsigned wave = blockIdx.x * 4u + (threadIdx.x >> 6);
@@ -423,30 +451,32 @@ __global__ __launch_bounds__(256) void dbatch_adjoint_kernel(
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
             const double sum = segment_sum(acc[c], ly);
-            if (ly.seg == 0 && ly.ok) partial[((size_t)u * 64 + ly.f) * 6 + c] = sum;
+            if (ly.seg == 0 && ly.ok) partial[((size_t)u * max_frames + ly.f) * 6 + c] = sum;
         }
     }
 }
 
-// grad[g*6 + c] = sum over the units of frame g's volume, in order.
+// grad[g*6 + c] = sum over the units of frame g's volume, one wavefront per
+// entry: lane l takes units l, l + 64, ... in order, then a fixed tree.
 __global__ __launch_bounds__(256) void dbatch_grad_kernel(const DVol* __restrict__ vols,
                                                           const DFrame* __restrict__ fr,
                                                           int total_frames,
                                                           const long long* __restrict__ unit_start,
                                                           const double* __restrict__ partial,
+                                                          const int max_frames,
                                                           const double* __restrict__ fgrad,
                                                           double* __restrict__ grad) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= total_frames * 6) return;
     const int g = i / 6, c = i - 6 * g;
     const int v = fr[g].volume;
     const int f = g - vols[v].first_frame;
     double s = 0.0;
     if (unit_start)
-        for (long long u = unit_start[v]; u < unit_start[v + 1]; ++u)
-            s += partial[((size_t)u * 64 + f) * 6 + c];
-    if (fgrad) s += fgrad[i];
-    grad[i] = s;
+        for (long long u = unit_start[v] + lane; u < unit_start[v + 1]; u += 64)
+            s += partial[((size_t)u * max_frames + f) * 6 + c];
+    s = wave_sum_f64(s);
+    if (lane == 0) grad[i] = fgrad ? s + fgrad[i] : s;
 }
 
 // ---- the update ----------------------------------------------------------------------
@@ -682,6 +712,7 @@ struct recon_diff_batch {
     double* floss = nullptr;      // per-frame model-to-frame loss and gradient
     double* fgrad = nullptr;
     double* fhess = nullptr;      // per-frame normal matrices (Gauss-Newton refinement)
+    double* fpart = nullptr;      // their sums by frame and chunk
     bool frame_term = false;
     bool all_frame_terms = false; // every volume has pairs
     // set while a Gauss-Newton step is captured: the annealed truncation and
@@ -694,6 +725,7 @@ struct recon_diff_batch {
     long long* beg = nullptr;
     long long* unit_start = nullptr;
     int64_t units_bound = 0;
+    int max_frames = 1;           // of any volume
     int adjoint_grid = 0;
     double* partial = nullptr;
     double* grad = nullptr;
@@ -732,21 +764,21 @@ int recon_diff_batch::forward(const float* poses, double* loss_out, hipStream_t 
         hipLaunchKernelGGL(dbatch_loss_kernel, dim3(loss_blocks), dim3(256), 0, s, d_vols,
                            d_loss_wg, loss_partials, lam_ids, lam);
     if (frame_term && want_hess)
-        hipLaunchKernelGGL(dbatch_frame_loss_kernel<true>, dim3(total_frames), dim3(256), 0, s,
-                           d_vols, d_frames, table, fr_range, anneal, floss, fgrad, fhess);
+        hipLaunchKernelGGL(dbatch_frame_loss_kernel<true>, dim3(total_frames, kFrameChunks), dim3(256), 0,
+                           s, d_vols, d_frames, table, fr_range, anneal, fpart);
     else if (frame_term)
-        hipLaunchKernelGGL(dbatch_frame_loss_kernel<false>, dim3(total_frames), dim3(256), 0, s,
-                           d_vols, d_frames, table, fr_range, anneal, floss, fgrad, nullptr);
-    hipLaunchKernelGGL(dbatch_loss_sum_kernel, dim3(n), dim3(256), 0, s, d_vols, loss_partials,
-                       frame_term ? floss : nullptr, loss_out);
+        hipLaunchKernelGGL(dbatch_frame_loss_kernel<false>, dim3(total_frames, kFrameChunks), dim3(256), 0,
+                           s, d_vols, d_frames, table, fr_range, anneal, fpart);
+    hipLaunchKernelGGL(dbatch_loss_sum_kernel, dim3(n), dim3(256), 0, s, d_vols, loss_partials, fpart,
+                       frame_term ? (want_hess ? 28 : 7) : 0, floss, fgrad, fhess, loss_out);
     RECON_HIP_TRY(hipGetLastError(), "diff batch loss launch");
     return RECON_OK;
 }
 
 int recon_diff_batch::backward(double* grad_out, hipStream_t s) {
     if (npairs == 0) {
-        hipLaunchKernelGGL(dbatch_grad_kernel, dim3((total_frames * 6 + 255) / 256), dim3(256), 0,
-                           s, d_vols, d_frames, total_frames, nullptr, nullptr,
+        hipLaunchKernelGGL(dbatch_grad_kernel, dim3((total_frames * 6 + 3) / 4), dim3(256), 0, s, d_vols,
+                           d_frames, total_frames, nullptr, nullptr, max_frames,
                            frame_term ? fgrad : nullptr, grad_out);
         RECON_HIP_TRY(hipGetLastError(), "diff batch gradient launch");
         return RECON_OK;
@@ -760,9 +792,9 @@ int recon_diff_batch::backward(double* grad_out, hipStream_t s) {
     hipLaunchKernelGGL(dbatch_units_kernel, dim3(1), dim3(256), 0, s, d_vols, n, uid, count, beg,
                        unit_start);
     hipLaunchKernelGGL(dbatch_adjoint_kernel, dim3(adjoint_grid), dim3(256), 0, s, d_vols, n, table,
-                       uid, lam_u, beg, unit_start, partial);
-    hipLaunchKernelGGL(dbatch_grad_kernel, dim3((total_frames * 6 + 255) / 256), dim3(256), 0, s,
-                       d_vols, d_frames, total_frames, unit_start, partial,
+                       uid, lam_u, beg, unit_start, max_frames, partial);
+    hipLaunchKernelGGL(dbatch_grad_kernel, dim3((total_frames * 6 + 3) / 4), dim3(256), 0, s, d_vols,
+                       d_frames, total_frames, unit_start, partial, max_frames,
                        frame_term ? fgrad : nullptr, grad_out);
     RECON_HIP_TRY(hipGetLastError(), "diff batch backward launch");
     return RECON_OK;
@@ -988,14 +1020,16 @@ static int plan(const recon_diff_volume* vols, int n, recon_diff_batch* b, hipSt
     if ((rc = b->alloc(&b->fgrad, (size_t)frames * 6, "diff batch frame gradients"))) return rc;
     if ((rc = b->alloc(&b->fhess, (size_t)frames * 21, "diff batch frame normal matrices")))
         return rc;
+    if ((rc = b->alloc(&b->fpart, (size_t)frames * kFrameChunks * 28, "diff batch frame sums"))) return rc;
     if ((rc = b->alloc(&b->owner, arena, "diff batch owner table"))) return rc;
     b->M = merge_layout(b->npairs);
     if ((rc = b->alloc(&b->merge_scratch, b->M.total, "diff batch merge scratch"))) return rc;
     if ((rc = b->alloc(&b->beg, n + 1, "diff batch ranges"))) return rc;
     if ((rc = b->alloc(&b->unit_start, n + 1, "diff batch units"))) return rc;
     b->units_bound = (b->npairs + kUnit - 1) / kUnit + n;
+    for (const DVol& dv : b->h_vols) b->max_frames = std::max(b->max_frames, dv.nframes);
     b->adjoint_grid = (int)((std::min<int64_t>(b->units_bound, kMaxWaves) + 3) / 4);
-    if ((rc = b->alloc(&b->partial, (size_t)b->units_bound * 64 * 6, "diff batch partials")))
+    if ((rc = b->alloc(&b->partial, (size_t)b->units_bound * b->max_frames * 6, "diff batch partials")))
         return rc;
     if ((rc = b->alloc(&b->grad, (size_t)frames * 6, "diff batch gradients"))) return rc;
     if ((rc = b->alloc(&b->adam_m, (size_t)frames * 6, "diff batch adam"))) return rc;

@@ -303,10 +303,11 @@ __device__ __forceinline__ void adjoint_lane_pass(const VolumeParams& vp, const 
     const bool act = ly.ok && v >= 0 && v < N && lam != 0.0f && isfinite(lam);
     float cx = 0.0f, cy = 0.0f, cz = 0.0f;
     if (act) {
-        const int64_t x = v % vp.gx, yz = v / vp.gx;
-        cx = voxel_centre((int)x, vp.vs[0], vp.off[0]);
-        cy = voxel_centre((int)(yz % vp.gy), vp.vs[1], vp.off[1]);
-        cz = voxel_centre((int)(yz / vp.gy), vp.vs[2], vp.off[2]);
+        // a volume holds less than 2^31 voxels
+        const uint32_t yz = (uint32_t)v / (uint32_t)vp.gx;
+        cx = voxel_centre((int)((uint32_t)v - yz * (uint32_t)vp.gx), vp.vs[0], vp.off[0]);
+        cz = voxel_centre((int)(yz / (uint32_t)vp.gy), vp.vs[2], vp.off[2]);
+        cy = voxel_centre((int)(yz % (uint32_t)vp.gy), vp.vs[1], vp.off[1]);
     }
     bool pass = false;
     BiProj s;
