@@ -13,7 +13,6 @@
 namespace recon {
 
 constexpr int kThreads = 256;
-constexpr int kRcpTable = 256;  // entries of an integrate workgroup's 1/(w+1) table
 
 // Wave-tile of 4*LX x (64/LX) x NR voxels.  Lane l owns voxels x..x+3
 // (x = x0 + 4*(l % LX)) of row y = y0 + l / LX for z = z0 .. z0+NR-1.  With

@@ -292,6 +292,14 @@ __device__ __forceinline__ float load_float(GlobalBytes base, uint32_t off) {
     return *(GlobalFloat)(base + off);
 }
 
+// Two neighbouring floats (4-byte aligned) in one load.
+__device__ __forceinline__ float2 load_float2(GlobalBytes base, uint32_t off) {
+    typedef float Pair __attribute__((ext_vector_type(2), aligned(4)));
+    asm("" : "+v"(off));
+    const Pair v = *(__attribute__((address_space(1))) Pair*)(base + off);
+    return make_float2(v.x, v.y);
+}
+
 __device__ __forceinline__ void store_float(GlobalBytes base, uint32_t off, float v) {
     asm("" : "+v"(off));
     *(GlobalFloat)(base + off) = v;

@@ -94,13 +94,9 @@ __global__ __launch_bounds__(64 * kCullWaves) void diff_cull_kernel(
     append_wave(live, id, 0u, list, list_count);
 }
 
-template <bool VEC>
 __global__ __launch_bounds__(kThreads) void diff_integrate_kernel(
-    const VolumeParams vp, const int nframes, const FrameTable ft,
-    const ListEntry* __restrict__ list, const unsigned* __restrict__ list_count) {
-    __shared__ float rtab[kRcpTable];
-    rtab[threadIdx.x] = 1.0f / (float)(threadIdx.x + 1);
-    __syncthreads();
+    const VolumeParams vp, const FrameTable ft, const ListEntry* __restrict__ list,
+    const unsigned* __restrict__ list_count) {
     const unsigned n = __builtin_amdgcn_readfirstlane(*list_count);
     const unsigned waves = gridDim.x * (kThreads / 64);
     for (unsigned i = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); i < n; i += waves) {
@@ -108,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void diff_integrate_kernel(
         const uint64_t frames = uniform_mask(list[i].frames);
         int x0, y0, z0;
         tile_origin<Shape>(vp, tile, x0, y0, z0);
-        diff_integrate_tile<Shape, FrameTable, VEC>(vp, nframes, ft, frames, x0, y0, z0, rtab);
+        diff_integrate_tile<Shape, 8, false>(vp, ft, frames, x0, y0, z0);
     }
 }
 
@@ -636,7 +632,7 @@ static void launch_setup(const VolumeParams& vp, const recon_depth_view* depth0,
 
 static int diff_occupancy() {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, diff_integrate_kernel<true>, kThreads,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, diff_integrate_kernel, kThreads,
                                                      0) != hipSuccess ||
         blocks < 1)
         blocks = 2;
@@ -707,12 +703,7 @@ extern "C" int recon_tsdf_diff_integrate(recon_tsdf* h, const recon_depth_view* 
                            dim3(64 * cull_waves(groups, n, h->num_cus)), 0, s, vp, n, ft, list,
                            h->list_count);
         RECON_HIP_TRY(hipGetLastError(), "diff_cull_kernel launch");
-        if (vp.gx % 4 == 0)
-            hipLaunchKernelGGL(diff_integrate_kernel<true>, grid, dim3(kThreads), 0, s, vp, n, ft,
-                               list, h->list_count);
-        else
-            hipLaunchKernelGGL(diff_integrate_kernel<false>, grid, dim3(kThreads), 0, s, vp, n, ft,
-                               list, h->list_count);
+        hipLaunchKernelGGL(diff_integrate_kernel, grid, dim3(kThreads), 0, s, vp, ft, list, h->list_count);
         RECON_HIP_TRY(hipGetLastError(), "diff_integrate_kernel launch");
     }
     return RECON_OK;
