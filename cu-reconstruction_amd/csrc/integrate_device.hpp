@@ -234,33 +234,6 @@ __device__ __forceinline__ uint64_t tile_frames(const VolumeParams& vp, const in
     return live;
 }
 
-// Appends the calling workgroup's surviving tiles (`live` != 0) to `list`
-// with one atomic per workgroup.  Every thread of the workgroup must call.
-__device__ __forceinline__ void append_tile(uint64_t live, uint32_t tile, uint32_t volume,
-                                            ListEntry* __restrict__ list,
-                                            unsigned* __restrict__ list_count, unsigned* s_wave,
-                                            unsigned* s_base) {
-    const unsigned n = live != 0;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned incl = n;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const unsigned o = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += o;
-    }
-    if (lane == 63) s_wave[wave] = incl;
-    __syncthreads();
-    unsigned wave_base = 0, total = 0;
-#pragma unroll
-    for (int i = 0; i < kThreads / 64; ++i) {
-        wave_base += i < wave ? s_wave[i] : 0u;
-        total += s_wave[i];
-    }
-    if (threadIdx.x == 0) *s_base = total ? atomicAdd(list_count, total) : 0u;
-    __syncthreads();
-    if (n) list[*s_base + wave_base + incl - n] = ListEntry{tile, volume, live};
-}
-
 // Appends the tiles of one wavefront (lane l: `tile`, frame mask `live`)
 // that some frame reaches to `list`, with one atomic for the wavefront.
 // Every lane of the calling wavefront must call.
@@ -379,10 +352,11 @@ __device__ __forceinline__ unsigned segment_slot(const unsigned* s_pre, int nseg
 // A wavefront takes a wave-tile; at step j its 64 lanes hold a patch of
 // LW x (64/LW) adjacent voxels of one z layer, so that a depth gather's lanes
 // land on neighbouring pixels, and its D and W accesses are runs of LW voxels
-// of a row (any gx: no vector alignment).  One frame per call is bound by
-// HBM (a 512^3 volume and a VGA frame move 377 MB at 4.5 TB/s, a large copy
-// 5.1): LW = 32, whole 128-byte rows (16 and 8 took 6 and 19 % longer).
-// Several frames are bound by the gathers (16 volumes of up to 40 frames of
+// of a row (any gx).  LW = 0 (one frame, gx % 4 == 0): a lane holds four voxels
+// of a row and moves them as 16 bytes.  One frame per call is bound by
+// HBM (a 512^3 volume and a VGA frame move 377 MB at 4.6 TB/s, a large copy
+// 5.1) and next by the address units (79 % busy with LW = 32; 16 and 8 took 6
+// and 19 % longer than 32).  Several frames are bound by the gathers (16 volumes of up to 40 frames of
 // 1280x720: address units 82 % busy, L2 misses at 6.2 TB/s, since a voxel
 // there spans about 6 pixels): the squarest patch.  Lanes of four voxels of a
 // row each, with its branches per voxel and IEEE divisions, took 818 M
@@ -401,40 +375,47 @@ __device__ __forceinline__ unsigned segment_slot(const unsigned* s_pre, int nseg
 // VARW (WEIGHT_BY_VARIANCE): an observation weighs
 // variance_weight(d) = sigma(1 m)^2 / sigma(d)^2 instead of 1, so
 // d' = ((d * w) + (wo * tsdf)) / (w + wo), w' = min(w + wo, max_weight).
-template <class S, int LW, class Frames, bool COUNT, bool COLOR = false, bool VARW = false>
+//
+// FRESH (several frames): the volume holds (trunc, 0) and is not read.
+template <class S, int LW, class Frames, bool COUNT, bool COLOR = false, bool VARW = false,
+          bool FRESH = false>
 __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Frames& frames,
                                                const uint64_t live, const int x0, const int y0,
                                                const int z0, unsigned& cnt, unsigned& touched) {
-    constexpr int LH = 64 / LW;                                // lanes in y
-    constexpr int NX = S::X / LW, NY = S::Y / LH, NR = S::Z;  // steps in x, y, z
+    constexpr bool kQuad = LW == 0;                           // lanes of four voxels of a row
+    constexpr int LX = kQuad ? S::X / 4 : LW, LH = 64 / LX;   // lanes in x, y
+    constexpr int NX = S::X / LX, NY = S::Y / LH, NR = S::Z;  // steps in x, y, z
     constexpr int NV = NX * NY * NR;                          // voxels per lane
-    static_assert(NX * LW == S::X && NY * LH == S::Y, "lanes must tile the wave-tile");
+    constexpr int XS = kQuad ? 1 : LX;                        // voxels between steps in x
+    static_assert(NX * LX == S::X && NY * LH == S::Y, "lanes must tile the wave-tile");
     constexpr bool kOne = Frames::kMax == 1;
+    static_assert(!kQuad || (kOne && NX == 4 && NY == 1), "quads serve single frames");
     const int lane = threadIdx.x & 63;
-    const int x = x0 + lane % LW, y = y0 + lane / LW;
+    const int xl = (kQuad ? 4 : 1) * (lane % LX);  // the lane's place in the tile's row
+    const int x = x0 + xl, y = y0 + lane / LX;
     if (x >= vp.gx || y >= vp.gy) return;
-    // step j's voxel: (x + LW * jx, y + LH * jy, z0 + jz)
+    // step j's voxel: (x + XS * jx, y + LH * jy, z0 + jz)
     const auto jx = [](int j) { return j % NX; };
     const auto jy = [](int j) { return (j / NX) % NY; };
     const auto jz = [](int j) { return j / (NX * NY); };
     bool in_grid[NV];
     float cxw[NX], cyw[NY], czw[NR];
 #pragma unroll
-    for (int k = 0; k < NX; ++k) cxw[k] = voxel_centre(x + LW * k, vp.vs[0], vp.off[0]);
+    for (int k = 0; k < NX; ++k) cxw[k] = voxel_centre(x + XS * k, vp.vs[0], vp.off[0]);
 #pragma unroll
     for (int k = 0; k < NY; ++k) cyw[k] = voxel_centre(y + LH * k, vp.vs[1], vp.off[1]);
 #pragma unroll
     for (int k = 0; k < NR; ++k) czw[k] = voxel_centre(z0 + k, vp.vs[2], vp.off[2]);
 #pragma unroll
     for (int j = 0; j < NV; ++j)
-        in_grid[j] = (x + LW * jx(j) < vp.gx) & (y + LH * jy(j) < vp.gy) & (z0 + jz(j) < vp.gz);
+        in_grid[j] = (kQuad || x + XS * jx(j) < vp.gx) & (y + LH * jy(j) < vp.gy) & (z0 + jz(j) < vp.gz);
     // offset of step j's voxel from the lane's first, the same for all lanes
     const auto step = [&](int j) {
-        return (int64_t)LW * jx(j) + (int64_t)vp.gx * (LH * jy(j) + (int64_t)vp.gy * jz(j));
+        return (int64_t)XS * jx(j) + (int64_t)vp.gx * (LH * jy(j) + (int64_t)vp.gy * jz(j));
     };
     // the tile's first voxel (uniform) and the lane's place from it
     const int64_t first = x0 + (int64_t)vp.gx * (y0 + (int64_t)vp.gy * z0);
-    const int64_t place = lane % LW + (int64_t)vp.gx * (lane / LW);
+    const int64_t place = xl + (int64_t)vp.gx * (lane / LX);
     GlobalFloat D = (GlobalFloat)vp.D + first, W = (GlobalFloat)vp.W + first;
     // VARW: sigma within [1e-8, 1e8] keeps the weight's quotient normal
     const float reach = vp.maxd + fabsf(vp.noise[2]);
@@ -449,8 +430,9 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         dirty[j] = false;
-        d[j] = w[j] = 0.0f;
-        if (!kOne && in_grid[j]) {
+        d[j] = vp.trunc;
+        w[j] = 0.0f;
+        if (!kOne && !FRESH && in_grid[j]) {
             d[j] = D[place + step(j)];
             w[j] = W[place + step(j)];
         }
@@ -499,8 +481,18 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             if (COLOR) band[j] = sdf <= vp.trunc;
         }
         const uint32_t place4 = 4u * (uint32_t)place;  // below 2^32 unless exact
-        if (kOne) {
-            // read back to back what the frame updates
+        constexpr int G = NX * NY;  // voxels of a layer
+        // read back to back what the frame updates
+        if (kQuad) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+                if (pass[G * r] | pass[G * r + 1] | pass[G * r + 2] | pass[G * r + 3]) {
+                    const Float4 d4 = *(GlobalFloat4)(D + place + step(G * r));
+                    const Float4 w4 = *(GlobalFloat4)(W + place + step(G * r));
+                    d[G * r] = d4.x; d[G * r + 1] = d4.y; d[G * r + 2] = d4.z; d[G * r + 3] = d4.w;
+                    w[G * r] = w4.x; w[G * r + 1] = w4.y; w[G * r + 2] = w4.z; w[G * r + 3] = w4.w;
+                }
+        } else if (kOne) {
 #pragma unroll
             for (int j = 0; j < NV; ++j)
                 if (pass[j]) {
@@ -508,7 +500,6 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                     w[j] = kExact ? W[place + step(j)] : load_float((GlobalBytes)(W + step(j)), place4);
                 }
         }
-        constexpr int G = NX * NY;  // voxels of a layer share the test for the short forms
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             bool any = false;
@@ -528,7 +519,7 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                     nw[i] = w[j] + wo;
                     num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
                     // a quotient near the denormals is left to the division
-                    bad = pass[j] & !(fabsf(num[i]) >= 1e-30f) ? INFINITY : bad;
+                    bad = (pass[j] & !(fabsf(num[i]) >= 1e-30f)) ? INFINITY : bad;
                 } else {
                     nw[i] = w[j] + 1.0f;
                     num[i] = (d[j] * w[j]) + tsdf[j];
@@ -551,20 +542,17 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
                 const float w2 = min_bound(vp.maxw, nw[i]);
-                if (kOne) {
-                    if (pass[j]) {
-                        if (kExact) {
-                            D[place + step(j)] = nd[i];
-                            W[place + step(j)] = w2;
-                        } else {
-                            store_float((GlobalBytes)(D + step(j)), place4, nd[i]);
-                            store_float((GlobalBytes)(W + step(j)), place4, w2);
-                        }
+                d[j] = pass[j] ? nd[i] : d[j];
+                w[j] = pass[j] ? w2 : w[j];
+                dirty[j] |= pass[j];
+                if (kOne && !kQuad && pass[j]) {
+                    if (kExact) {
+                        D[place + step(j)] = d[j];
+                        W[place + step(j)] = w[j];
+                    } else {
+                        store_float((GlobalBytes)(D + step(j)), place4, d[j]);
+                        store_float((GlobalBytes)(W + step(j)), place4, w[j]);
                     }
-                } else {
-                    d[j] = pass[j] ? nd[i] : d[j];
-                    w[j] = pass[j] ? w2 : w[j];
-                    dirty[j] |= pass[j];
                 }
                 if (COUNT && pass[j]) {
                     ++cnt;
@@ -581,6 +569,11 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                     c.w = nwc < vp.maxw ? nwc : vp.maxw;
                     *cp = c;
                 }
+            }
+            if (kQuad) {
+                const int j = G * r;
+                *(GlobalFloat4)(D + place + step(j)) = Float4{d[j], d[j + 1], d[j + 2], d[j + 3]};
+                *(GlobalFloat4)(W + place + step(j)) = Float4{w[j], w[j + 1], w[j + 2], w[j + 3]};
             }
         }
     };

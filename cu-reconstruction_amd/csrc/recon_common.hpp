@@ -285,6 +285,8 @@ __device__ __forceinline__ uint32_t mul24(uint32_t a, uint32_t b) {
 // accesses.  load_float and store_float take a wavefront-uniform base and a
 // 32-bit byte offset per lane (the scalar-base form of the instructions).
 using GlobalFloat = __attribute__((address_space(1))) float*;
+typedef float Float4 __attribute__((ext_vector_type(4)));
+using GlobalFloat4 = __attribute__((address_space(1))) Float4*;
 using GlobalBytes = __attribute__((address_space(1))) char*;
 
 __device__ __forceinline__ float load_float(GlobalBytes base, uint32_t off) {

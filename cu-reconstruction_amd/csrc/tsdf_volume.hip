@@ -8,7 +8,8 @@
 // integrate call is three launches on the caller's stream:
 //   1. depth_bounds_kernel  per 8x8 and 32x32 pixel block, the largest valid
 //                           depth of each frame;
-//   2. cull_kernel          one thread per wave-tile (32 x 8 x 2 voxels):
+//   2. cull_kernel          one thread per wave-tile (32 x 8 x 2 voxels), or
+//                           several frames' tests spread over wavefronts:
 //                           the tile survives a frame if its voxel-centre box
 //                           meets the frame's frustum and the depth bound of
 //                           its image footprint is not closer than the box
@@ -16,11 +17,10 @@
 //                           survivors (with their frame masks) into its own
 //                           segment of the list and writes their count;
 //   3. integrate_list_kernel  a grid sized to the resident wave slots walks
-//                           the list, one wave-tile per wavefront: lane l owns
-//                           voxels x..x+3 of row y for two z, so a wave moves
-//                           aligned 128-byte row segments of D and W with
-//                           dwordx4 accesses, and only lanes with a voxel that
+//                           the list, one wave-tile per wavefront
+//                           (integrate_tile); only lanes with a voxel that
 //                           passes read (and write) D and W.
+// One frame into a small volume is one launch (integrate_direct_kernel).
 // Voxel centres are computed from the index (no table traffic).  Up to
 // kMaxFusedFrames frames can go through one sweep: each voxel sees the frames
 // in order, so the result equals one sweep per frame.  The culling is
@@ -53,12 +53,11 @@ __global__ __launch_bounds__(256) void depth_bounds_kernel(const BoundsJob job, 
 // (the tile is kept after the 32x32 test).
 constexpr int kCullMaxFine = 24;
 
-// Workgroup b tests tiles [b*seg_len, (b+1)*seg_len) (seg_len a multiple of
-// 256, one tile per thread per pass), compacts the survivors into the same
-// slots of the list in tile order and writes their number to counts[b].
-template <int MAXF>
-__global__ __launch_bounds__(256) void cull_kernel(const VolumeParams vp, const int nframes,
-                                                   const FrameBlock<MAXF> fb,
+// One frame.  Workgroup b tests tiles [b*seg_len, (b+1)*seg_len) (seg_len a
+// multiple of 256, one tile per thread per pass), compacts the survivors into
+// the same slots of the list in tile order and writes their number to
+// counts[b].
+__global__ __launch_bounds__(256) void cull_kernel(const VolumeParams vp, const FrameBlock<1> fb,
                                                    ListEntry* __restrict__ list,
                                                    unsigned* __restrict__ counts,
                                                    const unsigned seg_len) {
@@ -70,23 +69,61 @@ __global__ __launch_bounds__(256) void cull_kernel(const VolumeParams vp, const 
     for (uint32_t k = first; k < end; k += kThreads) {
         const uint32_t id = k + threadIdx.x;
         const uint64_t live =
-            id < end ? tile_frames<Shape, FrameBlock<MAXF>, kCullMaxFine>(vp, nframes, fb, id) : 0ull;
+            id < end ? tile_frames<Shape, FrameBlock<1>, kCullMaxFine>(vp, 1, fb, id) : 0ull;
         n += append_local(live, id, 0u, list + first + n, s_wave);
     }
     if (threadIdx.x == 0) counts[blockIdx.x] = n;
 }
 
-// Voxels of a row that a wavefront's lanes hold side by side
-// (integrate_tile's LW).
+// Several frames: the same with seg_len a multiple of 64, 64 tiles per pass
+// and W = blockDim.x / 64 wavefronts (cull_waves), wave g testing frames g,
+// g + W, ... of every tile; wave 0 ORs the tile's masks and compacts.  One
+// thread per tile and 16 frames in a row took 53 us for 26100 tiles (102
+// workgroups), 13 now.
 template <int MAXF>
-constexpr int kLaneRow = MAXF == 1 ? 32 : 8;
+__global__ __launch_bounds__(64 * kCullWaves) void cull_frames_kernel(const VolumeParams vp, const int nframes,
+                                                                      const FrameBlock<MAXF> fb,
+                                                                      ListEntry* __restrict__ list,
+                                                                      unsigned* __restrict__ counts,
+                                                                      const unsigned seg_len) {
+    __shared__ uint64_t s_live[kCullWaves][64];
+    const uint32_t ntiles = (uint32_t)vp.tiles_x * vp.tiles_y * vp.tiles_z;
+    const uint32_t first = blockIdx.x * seg_len;
+    const uint32_t end = min(first + seg_len, ntiles);
+    const int i = threadIdx.x & 63, nw = (int)(blockDim.x >> 6);
+    const int g = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    unsigned n = 0;
+    for (uint32_t k = first; k < end; k += 64) {
+        const uint32_t id = k + i;
+        s_live[g][i] = id < end ? tile_frames<Shape, FrameBlock<MAXF>, kCullMaxFine>(vp, nframes, fb, id, g, nw)
+                                : 0ull;
+        __syncthreads();
+        if (g == 0) {
+            uint64_t live = 0;
+            for (int w = 0; w < nw; ++w) live |= s_live[w][i];
+            const uint64_t ball = __ballot(live != 0);
+            if (live)
+                list[first + n + (unsigned)__popcll(ball & ((1ull << i) - 1ull))] = ListEntry{id, 0u, live};
+            n += (unsigned)__popcll(ball);
+        }
+        __syncthreads();  // s_live is rewritten by the next pass
+    }
+    if (threadIdx.x == 0) counts[blockIdx.x] = n;
+}
+
+// integrate_tile's lane layout (LW): several frames take squares of 8 x 8
+// lanes; one frame takes quads (0) in the list kernel where rows are 16-byte
+// aligned (gx % 4 == 0), which leaves the address units the most time for the
+// gathers, else 32 lanes along a row.  30 VGA frames into 512^3, reset
+// included: 2740 us with quads, 2850 without (2823 before either).
+constexpr int kLanesMany = 8, kLanesOne = 32, kLanesQuad = 0;
 
 // The list's entries in dense order i = 0 .. total-1 (segment by segment):
 // each wavefront takes i = wave, wave + waves, ... (the grid is sized to the
 // resident wave slots, so every wave-tile costs about the same and the device
-// stays full until the list is done); lane j of a wave locates the list slot
-// of the wave's j-th next entry, so one search serves 64 entries.
-template <int MAXF, bool COUNT, bool COLOR = false, bool VARW = false>
+// stays full until the list is done); lane j of a wave locates and reads
+// the wave's j-th next entry, so one search and one load serve 64 entries.
+template <int MAXF, int LW, bool COUNT, bool COLOR, bool VARW>
 __global__ __launch_bounds__(kThreads) void integrate_list_kernel(
     const VolumeParams vp, const int nframes, const FrameBlock<MAXF> fb,
     const ListEntry* __restrict__ list, const unsigned* __restrict__ counts, const int nseg,
@@ -99,16 +136,16 @@ __global__ __launch_bounds__(kThreads) void integrate_list_kernel(
     unsigned cnt = 0, touched = 0;
     for (unsigned i0 = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); i0 < n; i0 += 64 * waves) {
         const unsigned mine = i0 + lane * waves;
-        const unsigned slot = mine < n ? segment_slot(s_pre, nseg, seg_len, mine) : 0u;
+        const ListEntry entry = list[mine < n ? segment_slot(s_pre, nseg, seg_len, mine) : 0u];
         const unsigned m = min(64u, (n - i0 + waves - 1) / waves);
         for (unsigned j = 0; j < m; ++j) {
-            const unsigned e = __builtin_amdgcn_readfirstlane(__shfl(slot, (int)j, 64));
-            const uint32_t tile = __builtin_amdgcn_readfirstlane(list[e].tile);
-            const uint64_t frames = uniform_mask(list[e].frames);
+            const uint32_t tile = __builtin_amdgcn_readlane(entry.tile, (int)j);
+            const uint64_t frames =
+                ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(entry.frames >> 32), (int)j) << 32) |
+                (uint32_t)__builtin_amdgcn_readlane((uint32_t)entry.frames, (int)j);
             int x0, y0, z0;
             tile_origin<Shape>(vp, tile, x0, y0, z0);
-            integrate_tile<Shape, kLaneRow<MAXF>, FrameBlock<MAXF>, COUNT, COLOR, VARW>(
-                vp, fb, frames, x0, y0, z0, cnt, touched);
+            integrate_tile<Shape, LW, FrameBlock<MAXF>, COUNT, COLOR, VARW>(vp, fb, frames, x0, y0, z0, cnt, touched);
         }
     }
     if (COUNT && counter && cnt) atomicAdd(counter, (unsigned long long)cnt);
@@ -133,7 +170,7 @@ __global__ __launch_bounds__(kThreads) void integrate_direct_kernel(const Volume
     for (int k = 0; k < 6; ++k) in = in & (plane_max(fb.f[0].plane[k], lo, hi) >= 0.0f);
     if (!in) return;
     unsigned cnt = 0;
-    integrate_tile<Shape, kLaneRow<1>, FrameBlock<1>, false, COLOR, VARW>(vp, fb, 1ull, x0, y0, z0, cnt,
+    integrate_tile<Shape, kLanesOne, FrameBlock<1>, false, COLOR, VARW>(vp, fb, 1ull, x0, y0, z0, cnt,
                                                                           cnt);
 }
 
@@ -222,11 +259,11 @@ static int ensure_scratch(recon_tsdf* h, const VolumeParams& vp, hipStream_t s) 
     return ensure_cull_list(h, (size_t)vp.tiles_x * vp.tiles_y * vp.tiles_z, sizeof(ListEntry));
 }
 
-// Cull segments: 256 tiles each, or the multiple of 256 that keeps their
+// Cull segments: `pass` tiles each, or the multiple of it that keeps their
 // number within kMaxSegments.
-static void cull_segments(int ntiles, unsigned* seg_len, int* nseg) {
+static void cull_segments(int ntiles, unsigned pass, unsigned* seg_len, int* nseg) {
     const unsigned need = (unsigned)((ntiles + kMaxSegments - 1) / kMaxSegments);
-    *seg_len = std::max<unsigned>(kThreads, (need + kThreads - 1) / kThreads * kThreads);
+    *seg_len = std::max<unsigned>(pass, (need + pass - 1) / pass * pass);
     *nseg = (int)((ntiles + *seg_len - 1) / *seg_len);
 }
 
@@ -246,12 +283,12 @@ constexpr int kListMaxBlocksPerCU = 5;
 // slots (capped).  The grid never exceeds the resident slots, because every
 // wave takes the same share of the list and a workgroup beyond them would
 // start only when another has finished its share.
-template <int MAXF, bool COUNT, bool COLOR, bool VARW>
+template <int MAXF, int LW, bool COUNT, bool COLOR, bool VARW>
 static int list_occupancy() {
     static const int blocks = [] {
         int b = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &b, integrate_list_kernel<MAXF, COUNT, COLOR, VARW>, kThreads, 0) != hipSuccess ||
+                &b, integrate_list_kernel<MAXF, LW, COUNT, COLOR, VARW>, kThreads, 0) != hipSuccess ||
             b < 1)
             b = 1;
         return std::min(b, kListMaxBlocksPerCU);
@@ -259,18 +296,18 @@ static int list_occupancy() {
     return blocks;
 }
 
-template <int MAXF, bool COUNT, bool COLOR>
+template <int MAXF, int LW, bool COUNT, bool COLOR>
 static void launch_list(bool varw, int num_cus, hipStream_t s, const VolumeParams& vp, int nframes,
                         const FrameBlock<MAXF>& fb, const ListArgs& la, unsigned long long* ctr,
                         unsigned long long* tctr) {
     if (varw)
-        hipLaunchKernelGGL((integrate_list_kernel<MAXF, COUNT, COLOR, true>),
-                           dim3(num_cus * list_occupancy<MAXF, COUNT, COLOR, true>()),
+        hipLaunchKernelGGL((integrate_list_kernel<MAXF, LW, COUNT, COLOR, true>),
+                           dim3(num_cus * list_occupancy<MAXF, LW, COUNT, COLOR, true>()),
                            dim3(kThreads), 0, s, vp, nframes, fb, la.list, la.counts, la.nseg,
                            la.seg_len, ctr, tctr);
     else
-        hipLaunchKernelGGL((integrate_list_kernel<MAXF, COUNT, COLOR, false>),
-                           dim3(num_cus * list_occupancy<MAXF, COUNT, COLOR, false>()),
+        hipLaunchKernelGGL((integrate_list_kernel<MAXF, LW, COUNT, COLOR, false>),
+                           dim3(num_cus * list_occupancy<MAXF, LW, COUNT, COLOR, false>()),
                            dim3(kThreads), 0, s, vp, nframes, fb, la.list, la.counts, la.nseg,
                            la.seg_len, ctr, tctr);
 }
@@ -281,7 +318,7 @@ static void launch_list(bool varw, int num_cus, hipStream_t s, const VolumeParam
 template <int MAXF>
 static int launch_prestage(const VolumeParams& vp, const float* depth0, size_t stride_floats,
                            int pitch, int nframes, FrameBlock<MAXF>& fb, float* bounds,
-                           ListEntry* list, unsigned* counts, hipStream_t s, ListArgs* la) {
+                           ListEntry* list, unsigned* counts, int num_cus, hipStream_t s, ListArgs* la) {
     const size_t per = (size_t)vp.b0x * vp.b0y + (size_t)vp.b1x * vp.b1y;
     for (int f = 0; f < nframes; ++f) {
         fb.f[f].bound0 = bounds + per * f;
@@ -307,9 +344,13 @@ static int launch_prestage(const VolumeParams& vp, const float* depth0, size_t s
     const int ntiles = vp.tiles_x * vp.tiles_y * vp.tiles_z;
     la->list = list;
     la->counts = counts;
-    cull_segments(ntiles, &la->seg_len, &la->nseg);
-    hipLaunchKernelGGL((cull_kernel<MAXF>), dim3(la->nseg), dim3(256), 0, s, vp, nframes, fb, list,
-                       counts, la->seg_len);
+    cull_segments(ntiles, MAXF == 1 ? kThreads : 64, &la->seg_len, &la->nseg);
+    if constexpr (MAXF == 1)
+        hipLaunchKernelGGL(cull_kernel, dim3(la->nseg), dim3(256), 0, s, vp, fb, list, counts, la->seg_len);
+    else
+        hipLaunchKernelGGL((cull_frames_kernel<MAXF>), dim3(la->nseg),
+                           dim3(64 * cull_waves(la->nseg, nframes, num_cus)), 0, s, vp, nframes, fb, list,
+                           counts, la->seg_len);
     RECON_HIP_TRY(hipGetLastError(), "cull_kernel launch");
     return RECON_OK;
 }
@@ -323,13 +364,28 @@ static int launch_liststage(recon_tsdf* h, const VolumeParams& vp, int nframes,
     unsigned long long* tctr = h->touch_counter;
     bool color = false;
     if constexpr (MAXF == 1) color = fb.f[0].rgb && vp.C;  // colour integrate (no counting)
-    if (color) {
-        if constexpr (MAXF == 1)
-            launch_list<1, false, true>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
-    } else if (ctr || tctr) {
-        launch_list<MAXF, true, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
+    const auto launch = [&](auto layout, auto count, auto with_color) {
+        launch_list<MAXF, decltype(layout)::value, decltype(count)::value, decltype(with_color)::value>(
+            varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using Quad = std::integral_constant<int, kLanesQuad>;
+    using Row = std::integral_constant<int, MAXF == 1 ? kLanesOne : kLanesMany>;
+    if constexpr (MAXF == 1) {
+        const bool quad = vp.gx % 4 == 0;
+        if (color) {
+            if (quad) launch(Quad{}, No{}, Yes{});
+            else launch(Row{}, No{}, Yes{});
+        } else if (ctr || tctr) {
+            launch(Row{}, Yes{}, No{});
+        } else {
+            if (quad) launch(Quad{}, No{}, No{});
+            else launch(Row{}, No{}, No{});
+        }
     } else {
-        launch_list<MAXF, false, false>(varw, h->num_cus, s, vp, nframes, fb, la, ctr, tctr);
+        if (ctr || tctr) launch(Row{}, Yes{}, No{});
+        else launch(Row{}, No{}, No{});
     }
     RECON_HIP_TRY(hipGetLastError(), "integrate_list_kernel launch");
     return RECON_OK;
@@ -359,7 +415,7 @@ static int launch_integrate(recon_tsdf* h, const VolumeParams& vp, const float* 
     if (rc) return rc;
     ListArgs la;
     rc = launch_prestage<MAXF>(vp, depth0, stride_floats, pitch, nframes, fb, h->bounds,
-                               static_cast<ListEntry*>(h->list), h->list_count, s, &la);
+                               static_cast<ListEntry*>(h->list), h->list_count, h->num_cus, s, &la);
     if (rc) return rc;
     return launch_liststage<MAXF>(h, vp, nframes, fb, la, s);
 }

@@ -34,7 +34,7 @@ HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
     "-ffp-contract=off", "-fno-fast-math",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wall", "-Wno-unused-function",
+    "-Wall", "-Wno-unused-function", "-Wno-bitwise-instead-of-logical",
     f"-I{INCLUDE}", f"-I{PKG / 'csrc'}",
 ]
 CXX = os.environ.get("CXX", "g++")
