@@ -19,14 +19,26 @@ __all__ = ["TSDFVolume", "Batch", "make_config", "depth_view", "depth_to_points"
            "mc_class_histogram", "ReconError", "TsdfConfig", "TsdfInfo", "ffi"]
 
 
+_torch_module = None
+
+
 def _torch():
-    import torch  # noqa: F401  (imported before librecon.so so one HIP runtime is shared)
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch  # (imported before librecon.so so one HIP runtime is shared)
+        _torch_module = torch
+    return _torch_module
 
 
 def _stream(stream) -> int:
+    """The hipStream_t of `stream` (a torch stream or a number), None: the
+    current stream of the current device."""
     if stream is None:
-        return _torch().cuda.current_stream().cuda_stream
+        torch = _torch()
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:  # without the Stream object around it
+            return raw(torch.cuda.current_device())
+        return torch.cuda.current_stream().cuda_stream
     return int(getattr(stream, "cuda_stream", stream))
 
 
@@ -63,8 +75,7 @@ def _device_tensor(t, name, dtype):
     """Raises ValueError unless `t` is a torch tensor of `dtype` in GPU
     memory: the kernels read raw device addresses, so a host tensor or a
     wrong element type must be refused before any call."""
-    torch = _torch()
-    if not isinstance(t, torch.Tensor):
+    if not isinstance(t, _torch().Tensor):
         raise ValueError(f"{name} must be a torch tensor")
     if not t.is_cuda:
         raise ValueError(f"{name} must be in GPU memory")
@@ -75,11 +86,11 @@ def _device_tensor(t, name, dtype):
 
 def depth_view(t) -> DepthView:
     """View of a 2-D float32 device tensor (row stride may exceed cols)."""
-    torch = _torch()
-    _device_tensor(t, "depth", torch.float32)
-    if t.dim() != 2 or t.stride(1) != 1 or t.stride(0) < t.shape[1]:
+    _device_tensor(t, "depth", _torch().float32)
+    shape, strides = t.shape, t.stride()
+    if len(shape) != 2 or strides[1] != 1 or strides[0] < shape[1]:
         raise ValueError("depth must be a 2-D float32 tensor with unit column stride")
-    return DepthView(t.data_ptr(), t.stride(0) * 4, t.shape[0], t.shape[1])
+    return DepthView(t.data_ptr(), strides[0] * 4, shape[0], shape[1])
 
 
 def _frames_view(depths, name="depths"):

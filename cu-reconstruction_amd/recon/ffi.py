@@ -11,6 +11,8 @@ import ctypes as C
 import os
 from pathlib import Path
 
+import numpy as np
+
 PKG = Path(__file__).resolve().parents[1]
 LIB_DIR = PKG / "lib"
 
@@ -214,8 +216,17 @@ def check(status: int) -> int:
     return status
 
 
+_Pose = C.c_double * 7
+
+
 def pose_array(pose) -> C.Array:
-    vals = [float(v) for v in pose]
+    # a row of float64 converts in one call; anything else value by value
+    if type(pose) is np.ndarray and pose.dtype == np.float64 and pose.ndim == 1:
+        vals = pose.tolist()
+    else:
+        vals = [float(v) for v in pose]
+    if len(vals) == 7:
+        return _Pose(*vals)
     if len(vals) % 7:
         raise ValueError("poses are 7-vectors {qw,qx,qy,qz,tx,ty,tz}")
     return (C.c_double * len(vals))(*vals)
