@@ -68,6 +68,21 @@ def test_random_fields(cuda, grid):
     _compare(cuda, f, grid, (0.01, 0.02, 0.03), (0.1, -0.2, 0.3), f"random {grid}")
 
 
+# a row of 1, 4 and 5 chunks and of several windows; values inside and outside
+# the range of the short quotients, mixed in one wavefront
+@pytest.mark.parametrize("grid", [(64, 3, 3), (255, 3, 4), (256, 2, 3), (257, 5, 2), (321, 3, 3),
+                                  (577, 4, 3)])
+@pytest.mark.parametrize("scale", [1.0, 1e-36, 1e30])
+def test_windows_and_quotient_ranges(cuda, grid, scale):
+    rng = np.random.default_rng(sum(grid))
+    gx, gy, gz = grid
+    f = rng.standard_normal((gz, gy, gx)).astype(np.float32)
+    f[rng.random(f.shape) < 0.3] *= np.float32(scale)
+    f[..., gx // 3: gx // 2] = np.abs(f[..., gx // 3: gx // 2])  # a stretch without vertices
+    print(f"welded windows {grid} scale {scale}", flush=True)
+    _compare(cuda, f, grid, (0.01, 0.02, 0.03), (0.1, -0.2, 0.3), f"windows {grid} {scale}")
+
+
 def test_counts_capacity_and_degenerate(cuda):
     lib = ffi.load()
     f = np.random.default_rng(3).standard_normal((6, 7, 8)).astype(np.float32)
