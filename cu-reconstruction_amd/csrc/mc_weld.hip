@@ -15,11 +15,11 @@
 // totals gives each chunk's first vertex.  The index of edge (voxel, axis) is
 //   base[chunk] + popc of the three masks below the voxel's lane
 //               + the voxel's own set bits of the axes before `axis`,
-// which the vertex writer and the triangle writer both evaluate: 32 B of
-// signs, counts and bases per 64 voxels.  The field is read whole once, by
-// weld_count_kernel (signs, vertex and triangle counts); after two exclusive
-// scans weld_write_kernel classifies cubes from the signs alone and reads the
-// field at the vertices.
+// which the vertex writer and the triangle writer both evaluate: 16 B of
+// signs and counts per 64 voxels.  The field is read whole once, by
+// weld_sign_kernel; weld_count_kernel counts vertices and triangles from the
+// signs, and after a scan of its block sums weld_write_kernel classifies the
+// cubes from the signs again and reads the field at the vertices.
 //
 // Vertex: from the negative end N to the other end M, r = (-dN)/(dM - dN),
 // p = sN + r*(sM - sN) per component.  This is the soup's own formula
@@ -33,17 +33,44 @@
 
 #include "mc_device.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace recon {
 
-constexpr int kWeldWaves = 4;  // one wavefront per voxel row, 256 threads
+// A group is 16 consecutive chunks (of one voxel row or several): the unit of
+// a wavefront in the count and write passes, lane 4i + q holding voxels and
+// cubes 16q .. 16q+15 of chunk i.  kBlockGroups groups are a workgroup of the
+// count pass; a chunk's first vertex is its block's plus its place in it.
+constexpr int kGroupChunks = 16;
+constexpr int kBlockGroups = 16, kBlockChunks = kBlockGroups * kGroupChunks;
+// A unit of the write pass is up to kUnitRounds rounds of 64 elements of a
+// group: its vertices first, then its triangles (<= 48 + 80 rounds, so <= 32
+// units).  The list holds group << kUnitBits | unit (group < 2^31 / 16).
+constexpr int kUnitRounds = 4, kUnitBits = 5;
+static_assert((16 * 64 * 3 + 16 * 64 * 5) / 64 <= kUnitRounds << kUnitBits, "a group's units fit the bits");
+constexpr int kSignChunks = 8;  // chunks per wavefront of the sign pass
+constexpr int kWeldWaves = 4;   // wavefronts per workgroup of the other passes
 
 struct WeldParams {
     McParams mc;
     int32_t cpr;      // 64-voxel chunks per x-row
     int32_t nchunks;  // cpr * gy * gz
+    uint32_t mul_cpr, mul_gy;  // div31's of cpr and gy
+    int32_t sh_cpr, sh_gy;
 };
+
+// n / d for n < 2^31: ceil(2^(31 + l) / d), l = ceil(log2 d), errs by less
+// than 2^-31 of n / d, too little to reach the next whole number.
+static void div31_make(uint32_t d, uint32_t& mul, int32_t& sh) {
+    int l = 0;
+    while ((1ull << l) < d) ++l;
+    mul = (uint32_t)((((1ull << 31) << l) + d - 1) / d);
+    sh = l;
+}
+__device__ __forceinline__ uint32_t div31(uint32_t n, uint32_t mul, int32_t sh) {
+    return (uint32_t)(((uint64_t)n * mul) >> 31) >> sh;
+}
 
 // Bits 0 .. n-1 (none for n <= 0, all for n >= 64).
 __device__ __forceinline__ unsigned long long low_bits(int n) {
@@ -63,105 +90,238 @@ __device__ __forceinline__ void weld_edges(const McParams& p, int j, int y, int 
     m[2] = z + 1 < p.gz ? (s ^ sz) & in : 0ull;
 }
 
-// Count pass: one wavefront per four voxel rows (y..y+3, z), streaming the
-// ten voxel rows (y+i, z) and (y+i, z+1), i = 0..4, 64 voxels a step (the
-// marching-cubes count's walk): each voxel's sign bit (v < 0) for the ten
-// rows packs into one word, bit 2j the lane's voxel of row j and bit 2j+1
-// the next lane's (a DPP wave shift; lane 63 takes the next step's lane 0).
-// A row's sign word is a ballot of its bit; the cube byte of cube row i is
-// bits 4i .. 4i+7 (corner order 0, 1, 3, 2, 4, 5, 7, 6, the count table
-// mc_ntab_qbyte); lane i of the wave stores row i's signs and counts.
-// Loads past a row's end read its last voxel, and rows past the grid (y+i
-// >= gy, z+1 >= gz) read the last row (in bounds); their edges and cubes
-// do not count.
-constexpr int kWeldRows = 4;
-constexpr int kWeldLoadRows = 2 * (kWeldRows + 1);
-
-__global__ __launch_bounds__(256) void weld_count_kernel(const WeldParams w,
-                                                         unsigned long long* __restrict__ signs,
-                                                         int32_t* __restrict__ vcount,
-                                                         int32_t* __restrict__ tcount) {
-    __shared__ uint8_t ntab[256];
-    ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
-    __syncthreads();
+// Signs of every chunk: eight chunks a wavefront, one 4-byte load a lane and
+// chunk, all in flight together.  It is the one pass over the whole field:
+// 250 x 333 x 287 voxels in 18 us, 5.3 TB/s.  A count kernel that read the
+// field itself took ten loads per four voxel rows (each row two and a half
+// times) and was bound by their addresses: 41 us, against 32 for this kernel
+// and the count of the signs.
+__global__ __launch_bounds__(256) void weld_sign_kernel(const WeldParams w,
+                                                        unsigned long long* __restrict__ signs,
+                                                        uint32_t* __restrict__ nunits) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nunits = 0;  // for the count kernel
     const McParams& p = w.mc;
     const int lane = threadIdx.x & 63;
-    const int gpl = (p.gy + kWeldRows - 1) / kWeldRows;
-    const int q = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWeldWaves + (threadIdx.x >> 6)));
-    const int z = q / gpl, y = kWeldRows * (q - z * gpl);
-    if (z >= p.gz) return;
-    const int k = min(kWeldRows, p.gy - y);         // voxel rows of the wave
-    const int z1 = min(z + 1, p.gz - 1);
-    const bool zin = z + 1 < p.gz;
-    const char* rowp[kWeldLoadRows];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t c0 = kSignChunks * (blockIdx.x * kWeldWaves + (uint32_t)wave);
+    if (c0 >= (uint32_t)w.nchunks) return;
+    // lane k (of every eight): chunk c0 + k (the last one past the end), its
+    // first voxel and the voxels after that in its row
+    const uint32_t cl = min(c0 + (uint32_t)(lane & 7), (uint32_t)w.nchunks - 1u);
+    const uint32_t row = div31(cl, w.mul_cpr, w.sh_cpr), j = cl - row * (uint32_t)w.cpr;
+    const unsigned long long start = (unsigned long long)row * (uint32_t)p.gx + 64ull * j;
+    const int lo = (int)(uint32_t)start, hi = (int)(uint32_t)(start >> 32), last = p.gx - 1 - 64 * (int)j;
+    float v[kSignChunks];
 #pragma unroll
-    for (int i = 0; i <= kWeldRows; ++i) {
-        const int yy = min(y + i, p.gy - 1);
-        rowp[2 * i] = reinterpret_cast<const char*>(p.f + (size_t)p.gx * ((size_t)yy + (size_t)p.gy * z));
-        rowp[2 * i + 1] =
-            reinterpret_cast<const char*>(p.f + (size_t)p.gx * ((size_t)yy + (size_t)p.gy * z1));
+    for (int k = 0; k < kSignChunks; ++k) {
+        const unsigned long long s = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readlane(lo, k);
+        const float* base = p.f + s;
+        v[k] = base[(uint32_t)min(lane, __builtin_amdgcn_readlane(last, k))];
     }
-    const uint32_t xlast = (uint32_t)(p.gx - 1);
-    auto load = [&](int chunk, float v[kWeldLoadRows]) {
-        const uint32_t off = min((uint32_t)(64 * chunk + lane), xlast) << 2;
+    unsigned long long out = 0;
 #pragma unroll
-        for (int j = 0; j < kWeldLoadRows; ++j) v[j] = *reinterpret_cast<const float*>(rowp[j] + off);
-    };
-    auto sign_bits = [&](const float v[kWeldLoadRows]) {
-        uint32_t m = 0;
+    for (int k = 0; k < kSignChunks; ++k) {
+        const unsigned long long b = __ballot(v[k] < 0.0f);
+        out = lane == k ? b : out;
+    }
+    if (lane < kSignChunks && c0 + lane < (uint32_t)w.nchunks) signs[c0 + lane] = out;
+}
+
+// Chunk c's place: chunk j of voxel row (y, z).
+struct ChunkPlace {
+    int j, y, z;
+};
+__device__ __forceinline__ ChunkPlace chunk_place(const WeldParams& w, uint32_t c) {
+    const uint32_t row = div31(c, w.mul_cpr, w.sh_cpr), z = div31(row, w.mul_gy, w.sh_gy);
+    return {(int)(c - row * (uint32_t)w.cpr), (int)(row - z * (uint32_t)w.mc.gy), (int)z};
+}
+
+// Triangle counts of 16 cubes of a chunk from voxel x on, 4 bits each, from
+// the signs q of their rows (y,z), (y,z+1), (y+1,z), (y+1,z+1), 17 voxels
+// each; `in`: the cubes' rows are in the grid.  A cube's byte holds the rows'
+// bits in this order (corner order 0, 1, 3, 2, 4, 5, 7, 6).
+struct CubeCounts {
+    uint32_t w[2];
+};
+__device__ __forceinline__ uint32_t cube_byte(const uint32_t q[4], int j) {
+    return ((q[0] >> j) & 3u) | (((q[1] >> j) & 3u) << 2) | (((q[2] >> j) & 3u) << 4) |
+           (((q[3] >> j) & 3u) << 6);
+}
+__device__ __forceinline__ CubeCounts cube_counts(const McParams& p, const uint8_t* ntab,
+                                                  const uint32_t q[4], bool in, int x) {
+    CubeCounts n = {{0u, 0u}};
 #pragma unroll
-        for (int j = 0; j < kWeldLoadRows; ++j) m |= (v[j] < 0.0f ? 1u : 0u) << (2 * j);
-        return m;
-    };
-    const int cpr = w.cpr;
-    auto emit = [&](int c, uint32_t pc, uint32_t pn) {
-        const uint32_t sh = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)pc, 0x130, 0xF, 0xF, false);
-        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)pn, 0);
-        const uint32_t word = pc | ((lane == 63 ? first : sh) << 1);
-        const int x = 64 * c + lane;
-        const bool xin1 = x + 1 < p.gx;
-        int n[kWeldRows];
-        unsigned long long s[kWeldRows + 1];
-        int nv[kWeldRows];
-#pragma unroll
-        for (int i = 0; i <= kWeldRows; ++i) s[i] = __ballot((pc >> (4 * i)) & 1u);
-#pragma unroll
-        for (int i = 0; i < kWeldRows; ++i) {
+    for (int j = 0; j < 16; ++j) n.w[j >> 3] |= (uint32_t)ntab[cube_byte(q, j)] << (4 * (j & 7));
+    const int left = in ? min(max(p.gx - 1 - x, 0), 16) : 0;
+    const unsigned long long keep = low_bits(4 * left);
+    n.w[0] &= (uint32_t)keep;
+    n.w[1] &= (uint32_t)(keep >> 32);
+    return n;
+}
+// Sum of the low 8, 4 or 2 of the 4-bit counts in w.
+__device__ __forceinline__ int sum8(uint32_t w) {
+    const uint32_t b = (w & 0x0F0F0F0Fu) + ((w >> 4) & 0x0F0F0F0Fu);
+    return (int)((b * 0x01010101u) >> 24);
+}
+
+// Counts: one wavefront a group.  Lane 16 rr + i reads the signs of chunk i
+// in row (y + (rr >> 1), z + (rr & 1)); the edges follow from the words, the
+// triangles from the table, 16 cubes a lane, where any cube of the group has
+// both signs.  A workgroup appends its groups' units of work to the write
+// pass's list, in any order between workgroups (what a unit writes and where
+// does not depend on it).  14 us for 24 000 groups, two thirds of them without
+// a negative value: latency, of the loads and of the workgroup's two steps.
+__global__ __launch_bounds__(64 * kBlockGroups) void weld_count_kernel(
+    const WeldParams w, const unsigned long long* __restrict__ signs, int32_t* __restrict__ voff,
+    int32_t* __restrict__ toff, int2* __restrict__ group, long long* __restrict__ vsums,
+    long long* __restrict__ tsums, bool want_v, bool want_t, uint32_t* __restrict__ units,
+    uint32_t* __restrict__ nunits) {
+    __shared__ uint8_t ntab[256];
+    __shared__ unsigned long long sl[kBlockGroups][64];
+    __shared__ uint8_t nl[kBlockGroups][64];
+    __shared__ int vc[kBlockChunks], tc[kBlockChunks];
+    __shared__ int wv[kBlockChunks / 64], wt[kBlockChunks / 64], gu[kBlockGroups];
+    const McParams& p = w.mc;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t nchunks = (uint32_t)w.nchunks;
+    const uint32_t c0 = kGroupChunks * (blockIdx.x * kBlockGroups + (uint32_t)wave);
+    const int rr = lane >> 4;
+    const uint32_t c = c0 + (lane & 15);
+    const ChunkPlace at = chunk_place(w, c < nchunks ? c : nchunks - 1u);
+    const bool here = (c < nchunks) & (at.y + (rr >> 1) < p.gy) & (at.z + (rr & 1) < p.gz);
+    const size_t cc = (size_t)c + (rr >> 1 ? (size_t)w.cpr : 0) + (rr & 1 ? (size_t)w.cpr * p.gy : 0);
+    unsigned long long s = 0, sn = 0;
+    if (here) {
+        s = signs[cc];
+        if (at.j + 1 < w.cpr) sn = signs[cc + 1];
+    }
+    if (threadIdx.x < 256) ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
+    __syncthreads();
+    int nv = 0;
+    bool mixed = false;
+    if (__ballot((s | sn) != 0ull)) {  // any negative value in reach
+        const unsigned long long sz = __shfl_down(s, 16, 64), sy = __shfl_down(s, 32, 64);
+        if (rr == 0 && here) {
             unsigned long long m[3];
-            weld_edges(p, c, y + i, z, s[i], (first >> (4 * i)) & 1u, s[i + 1],
-                       __ballot((pc >> (4 * i + 2)) & 1u), m);
-            nv[i] = __popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]);
-            const bool cube = xin1 && zin && y + i + 1 < p.gy;
-            n[i] = cube ? (int)ntab[(word >> (4 * i)) & 0xFFu] : 0;
+            weld_edges(p, at.j, at.y, at.z, s, sn, sy, sz, m);
+            nv = __popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]);
         }
-        const int s01 = wave_inclusive_scan(n[0] | (n[1] << 16), lane);
-        const int s23 = wave_inclusive_scan(n[2] | (n[3] << 16), lane);
-        const int t01 = __builtin_amdgcn_readlane(s01, 63), t23 = __builtin_amdgcn_readlane(s23, 63);
-        if (lane < k) {
-            const int i = lane;
-            const int tw = i < 2 ? t01 : t23;
-            const int64_t cc = (int64_t)(y + i + p.gy * z) * cpr + c;
-            signs[cc] = i == 0 ? s[0] : (i == 1 ? s[1] : (i == 2 ? s[2] : s[3]));
-            vcount[cc] = i == 0 ? nv[0] : (i == 1 ? nv[1] : (i == 2 ? nv[2] : nv[3]));
-            tcount[cc] = (i & 1) ? (tw >> 16) : (tw & 0xFFFF);
-        }
-    };
-    float va[kWeldLoadRows], vb[kWeldLoadRows];
-    load(0, va);
-    load(1, vb);
-    uint32_t pc = sign_bits(va);
-    load(2, va);
-    for (int c = 0; c < cpr; c += 2) {
-        uint32_t pn = sign_bits(vb);  // chunk c+1
-        load(c + 3, vb);
-        emit(c, pc, pn);
-        if (c + 1 >= cpr) break;
-        pc = pn;
-        pn = sign_bits(va);  // chunk c+2
-        load(c + 4, va);
-        emit(c + 1, pc, pn);
-        pc = pn;
+        // a cube has both signs where the eight words' AND and OR differ
+        const unsigned long long sx = (s >> 1) | (sn << 63);
+        unsigned long long all = s & sx, any = s | sx;
+        all &= __shfl_xor(all, 16, 64);
+        any |= __shfl_xor(any, 16, 64);
+        all &= __shfl_xor(all, 32, 64);
+        any |= __shfl_xor(any, 32, 64);
+        const bool cubes = (c < nchunks) & (at.y + 1 < p.gy) & (at.z + 1 < p.gz);
+        mixed = cubes & (((any & ~all) & low_bits(p.gx - 1 - 64 * at.j)) != 0);
     }
+    if (rr == 0) vc[kGroupChunks * wave + lane] = nv;
+    const int nvg = __builtin_amdgcn_readlane(wave_inclusive_scan(nv, lane), 63);
+    int ntg = 0;
+    if (__ballot(mixed)) {
+        sl[wave][lane] = s;
+        nl[wave][lane] = (uint8_t)(sn & 1ull);
+        __builtin_amdgcn_wave_barrier();
+        const int i = lane >> 2, b = 16 * (lane & 3);
+        const ChunkPlace mine = chunk_place(w, min(c0 + (uint32_t)i, nchunks - 1u));
+        uint32_t q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            q[k] = (uint32_t)(sl[wave][16 * k + i] >> b);
+            if (b == 48) q[k] |= (uint32_t)nl[wave][16 * k + i] << 16;
+        }
+        const bool in = (c0 + (uint32_t)i < nchunks) & (mine.y + 1 < p.gy) & (mine.z + 1 < p.gz);
+        const CubeCounts n = cube_counts(p, ntab, q, in, 64 * mine.j + b);
+        const int incl = wave_inclusive_scan(sum8(n.w[0]) + sum8(n.w[1]), lane);
+        ntg = __builtin_amdgcn_readlane(incl, 63);
+        const int before = __shfl(incl, 4 * (lane & 15) - 1, 64);  // lanes 0..15: chunk lane's
+        const int upto = __shfl(incl, 4 * (lane & 15) + 3, 64);
+        if (lane < 16) tc[kGroupChunks * wave + lane] = upto - (lane ? before : 0);
+    } else if (lane < 16) {
+        tc[kGroupChunks * wave + lane] = 0;
+    }
+    if (lane == 0) {
+        const int rounds = (want_v ? (nvg + 63) / 64 : 0) + (want_t ? (ntg + 63) / 64 : 0);
+        gu[wave] = (rounds + kUnitRounds - 1) / kUnitRounds;
+        if (c0 < nchunks) group[c0 / kGroupChunks] = make_int2(nvg, ntg);
+    }
+    __syncthreads();
+    if (wave == kBlockGroups - 1) {
+        const int mine = lane < kBlockGroups ? gu[lane] : 0;
+        const int incl = wave_inclusive_scan(mine, lane);
+        const int all_units = __builtin_amdgcn_readlane(incl, 63);
+        if (all_units) {
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(nunits, (uint32_t)all_units);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + (uint32_t)(incl - mine);
+            const uint32_t g = kBlockGroups * blockIdx.x + (uint32_t)lane;
+            for (int k = 0; k < mine; ++k) units[base + k] = (g << kUnitBits) | (uint32_t)k;
+        }
+    }
+    const bool scan = wave < kBlockChunks / 64;
+    int v = 0, t = 0, iv = 0, it = 0;
+    if (scan) {
+        v = vc[threadIdx.x];
+        t = tc[threadIdx.x];
+        iv = wave_inclusive_scan(v, lane);
+        it = wave_inclusive_scan(t, lane);
+        if (lane == 63) {
+            wv[wave] = iv;
+            wt[wave] = it;
+        }
+    }
+    __syncthreads();
+    if (scan) {
+        int bv = 0, bt = 0, av = 0, at_ = 0;
+#pragma unroll
+        for (int k = 0; k < kBlockChunks / 64; ++k) {
+            bv += k < wave ? wv[k] : 0;
+            bt += k < wave ? wt[k] : 0;
+            av += wv[k];
+            at_ += wt[k];
+        }
+        const uint32_t ct = kBlockChunks * blockIdx.x + threadIdx.x;
+        if (ct < nchunks) {
+            voff[ct] = bv + iv - v;
+            toff[ct] = bt + it - t;
+        }
+        if (threadIdx.x == 0) {
+            vsums[blockIdx.x] = av;
+            tsums[blockIdx.x] = at_;
+        }
+    }
+}
+
+// Block sums to first indices in place, the totals to total[0] (vertices) and
+// total[1] (triangles): a workgroup an array.
+__global__ __launch_bounds__(256) void weld_scan_kernel(long long* __restrict__ vsums,
+                                                        long long* __restrict__ tsums, int nb,
+                                                        long long* __restrict__ total) {
+    constexpr int kItems = 8;
+    __shared__ long long sh[4];
+    long long* __restrict__ sums = blockIdx.x ? tsums : vsums;
+    long long carry = 0;
+    for (int base = 0; base < nb; base += 256 * kItems) {
+        const int i0 = base + (int)threadIdx.x * kItems;
+        long long v[kItems], s = 0;
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) {
+            v[k] = i0 + k < nb ? sums[i0 + k] : 0;
+            s += v[k];
+        }
+        long long all;
+        long long e = carry + block_exclusive_scan(s, sh, &all);
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) {
+            if (i0 + k < nb) sums[i0 + k] = e;
+            e += v[k];
+        }
+        carry += all;
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
 // Gradient component `a` of the field at voxel (x, y, z).
@@ -315,37 +475,37 @@ __device__ __forceinline__ void weld_vertex(const WeldParams& w, const WeldSteps
     }
 }
 
-// A window is up to four consecutive chunks of a voxel row; one wavefront
-// writes it, lane l holding voxels and cubes 4l .. 4l+3 of its 256.  For the
-// four rows (y + dy, z + dz) its cubes reach and its own chunks and the next,
-// LDS holds the signs, edge masks and first vertex: entry 5 (2 dy + dz) + j.
-constexpr int kWinChunks = 4, kWinEntries = 4 * (kWinChunks + 1);
-struct WeldWindow {
-    unsigned long long s[kWinEntries];
-    unsigned long long m[kWinEntries][3];
-    uint32_t base[kWinEntries];
+// A group's neighbourhood in LDS, for the four rows (y + dy, z + dz) that its
+// cubes reach: entry 17 (2 dy + dz) + i is chunk i's (16: the next one's) word
+// of signs, edge masks and first vertex.
+constexpr int kGroupEntries = kGroupChunks + 1;
+struct WeldGroup {
+    unsigned long long s[4 * kGroupEntries];
+    unsigned long long m[4 * kGroupEntries][3];
+    uint32_t base[4 * kGroupEntries];
+    int x[kGroupChunks], y[kGroupChunks], z[kGroupChunks];
     int mark[64];
 };
 
 // The lane whose elements include element k0 + lane of the lanes' elements
-// (first element excl, count n per lane; carry: the round before's last
-// owner): marks at the first elements and a max-scan.  Every lane calls.
-__device__ __forceinline__ int weld_owner(int* mark, int excl, int n, int k0, int lane, int& carry) {
+// (first element excl, count n per lane; k0 below their total): marks at the
+// first elements, a max-scan, and the lane that element k0 is in before the
+// first mark.  Every lane calls.
+__device__ __forceinline__ int weld_owner(int* mark, int excl, int n, int k0, int lane) {
     mark[lane] = 0;
     if (n > 0 && excl >= k0 && excl < k0 + 64) mark[excl - k0] = lane + 1;
     __builtin_amdgcn_wave_barrier();
     const int mx = wave_inclusive_max(mark[lane]);
-    const int owner = mx > 0 ? mx - 1 : carry;
-    carry = __builtin_amdgcn_readlane(owner, 63);
+    const int first = 63 - __builtin_clzll(__ballot(n > 0 && excl <= k0) | 1ull);
     __builtin_amdgcn_wave_barrier();
-    return owner;
+    return mx > 0 ? mx - 1 : first;
 }
 
-// Vertex index of local edge e (table word et: axis, lower end's dx, dy, dz)
-// of the window's cube at voxel place xl.
-__device__ __forceinline__ int32_t weld_index(const WeldWindow& nb, int xl, unsigned et) {
+// Vertex index of the local edge of table word et (axis, lower end's dx, dy,
+// dz) of the cube at voxel place xl of the group's chunks.
+__device__ __forceinline__ int32_t weld_index(const WeldGroup& nb, int xl, unsigned et) {
     const int a = (int)(et & 3u), X = xl + (int)((et >> 2) & 1u), l = X & 63;
-    const int n = 5 * (int)(et >> 3) + (X >> 6);
+    const int n = kGroupEntries * (int)(et >> 3) + (X >> 6);
     const unsigned long long below = (1ull << l) - 1ull;
     const unsigned long long m0 = nb.m[n][0], m1 = nb.m[n][1], m2 = nb.m[n][2];
     int idx = (int)nb.base[n] + __popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below);
@@ -354,142 +514,171 @@ __device__ __forceinline__ int32_t weld_index(const WeldWindow& nb, int xl, unsi
     return idx;
 }
 
-__device__ __forceinline__ void weld_write_window(const WeldParams& w, const WeldSteps& st, int row, int j0,
-                                                  int lane, const unsigned long long* __restrict__ signs,
-                                                  const long long* __restrict__ vbase, long long v0,
-                                                  long long t0, bool want_v, bool want_t, WeldWindow& nb,
-                                                  const uint64_t* tri, const uint8_t* ntab,
-                                                  const uint32_t* edges, float* __restrict__ verts,
-                                                  float* __restrict__ normals, int32_t* __restrict__ tris) {
+// Entry of chunk c (place at; of the grid) in row rr of the neighbourhood.
+__device__ __forceinline__ void weld_entry_load(const WeldParams& w, uint32_t c, const ChunkPlace& at, int rr,
+                                                const unsigned long long* __restrict__ signs,
+                                                const int32_t* __restrict__ voff,
+                                                const long long* __restrict__ vsums, bool in,
+                                                WeldGroup& nb, int entry) {
     const McParams& p = w.mc;
-    const int z = row / p.gy, y = row - z * p.gy;
-    if (lane < kWinEntries) {
-        const int rr = lane / 5, j = j0 + lane - 5 * rr;
-        const int Y = y + (rr >> 1), Z = z + (rr & 1);
-        unsigned long long s = 0, m[3] = {0, 0, 0};
-        uint32_t base = 0;
-        if (Y < p.gy && Z < p.gz && j < w.cpr) {
-            const int64_t c = (int64_t)(Y + p.gy * Z) * w.cpr + j;
-            s = signs[c];
-            const unsigned long long sn = j + 1 < w.cpr ? signs[c + 1] : 0ull;
-            const unsigned long long sy = Y + 1 < p.gy ? signs[c + w.cpr] : 0ull;
-            const unsigned long long sz = Z + 1 < p.gz ? signs[c + (int64_t)w.cpr * p.gy] : 0ull;
-            weld_edges(p, j, Y, Z, s, sn, sy, sz, m);
-            base = (uint32_t)vbase[c];
+    const int Y = at.y + (rr >> 1), Z = at.z + (rr & 1);
+    unsigned long long s = 0, m[3] = {0, 0, 0};
+    uint32_t base = 0;
+    if (in & (Y < p.gy) & (Z < p.gz)) {
+        const size_t cc = (size_t)c + (rr >> 1 ? (size_t)w.cpr : 0) + (rr & 1 ? (size_t)w.cpr * p.gy : 0);
+        s = signs[cc];
+        const unsigned long long sn = at.j + 1 < w.cpr ? signs[cc + 1] : 0ull;
+        const unsigned long long sy = Y + 1 < p.gy ? signs[cc + w.cpr] : 0ull;
+        const unsigned long long sz = Z + 1 < p.gz ? signs[cc + (size_t)w.cpr * p.gy] : 0ull;
+        weld_edges(p, at.j, Y, Z, s, sn, sy, sz, m);
+        base = (uint32_t)vsums[cc / kBlockChunks] + (uint32_t)voff[cc];
+    }
+    nb.s[entry] = s;
+    nb.m[entry][0] = m[0];
+    nb.m[entry][1] = m[1];
+    nb.m[entry][2] = m[2];
+    nb.base[entry] = base;
+}
+
+// Elements [first, first + 64 kUnitRounds) of the group of chunks from c0 on:
+// its nv vertices rounded up to whole rounds, then its nt triangles.
+__device__ __forceinline__ void weld_write_unit(
+    const WeldParams& w, const WeldSteps& st, uint32_t c0, int lane, int first, int nv, int nt,
+    const unsigned long long* __restrict__ signs, const int32_t* __restrict__ voff,
+    const int32_t* __restrict__ toff, const long long* __restrict__ vsums,
+    const long long* __restrict__ tsums, WeldGroup& nb, const uint64_t* tri, const uint8_t* ntab,
+    const uint32_t* edges, float* __restrict__ verts, float* __restrict__ normals,
+    int32_t* __restrict__ tris) {
+    const McParams& p = w.mc;
+    const uint32_t nchunks = (uint32_t)w.nchunks;
+    {
+        const uint32_t c = c0 + (lane & 15);
+        const ChunkPlace at = chunk_place(w, min(c, nchunks - 1u));
+        weld_entry_load(w, c, at, lane >> 4, signs, voff, vsums, c < nchunks, nb,
+                        kGroupEntries * (lane >> 4) + (lane & 15));
+        if (lane < kGroupChunks) {
+            nb.x[lane] = 64 * at.j;
+            nb.y[lane] = at.y;
+            nb.z[lane] = at.z;
         }
-        nb.s[lane] = s;
-        nb.m[lane][0] = m[0];
-        nb.m[lane][1] = m[1];
-        nb.m[lane][2] = m[2];
-        nb.base[lane] = base;
+    }
+    const uint32_t cn = c0 + kGroupChunks;  // the next chunk, where it goes on with the row
+    if (cn < nchunks && cn % (uint32_t)w.cpr) {
+        const ChunkPlace at = chunk_place(w, cn);
+        if (lane < 4)
+            weld_entry_load(w, cn, at, lane, signs, voff, vsums, true, nb,
+                            kGroupEntries * lane + kGroupChunks);
     }
     __builtin_amdgcn_wave_barrier();
-    const int slot = lane >> 4, b = 4 * (lane & 15);
-    const int x0 = 64 * j0;
-    if (want_v) {
-        // the lane's edges, bit 3 v + axis of voxel 4 lane + v
-        unsigned own = 0;
-        if (j0 + slot < w.cpr) {
+    const int i = lane >> 2, b = 16 * (lane & 3);
+    // rounds [first, first + kUnitRounds) of the vertices' and then the
+    // triangles'
+    const int nv64 = (nv + 63) & ~63, end = first + 64 * kUnitRounds;
+    if (first < nv64) {
+        const uint32_t own01 = (uint32_t)((nb.m[i][0] >> b) & 0xFFFFull) |
+                               ((uint32_t)((nb.m[i][1] >> b) & 0xFFFFull) << 16);
+        const uint32_t own2 = (uint32_t)((nb.m[i][2] >> b) & 0xFFFFull);
+        const int mine = __popc(own01) + __popc(own2);
+        const int excl = wave_inclusive_scan(mine, lane) - mine;
+        const long long v0 = (long long)nb.base[0];
+        for (int k0 = first; k0 < min(end, nv); k0 += 64) {
+            const int owner = weld_owner(nb.mark, excl, mine, k0, lane);
+            uint32_t o01 = (uint32_t)__shfl((int)own01, owner, 64), o2 = (uint32_t)__shfl((int)own2, owner, 64);
+            int r = k0 + lane - __shfl(excl, owner, 64), v = 0;
+            // edge r of the 16 voxels', in the order voxel, axis: halve the
+            // voxels (bits shifted in from o01's upper half stay above the
+            // bits that are left to look at)
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const unsigned q = (unsigned)(nb.m[slot][a] >> b) & 0xFu;
-                own |= ((q & 1u) | ((q & 2u) << 2) | ((q & 4u) << 4) | ((q & 8u) << 6)) << a;
+            for (int h = 8; h >= 1; h >>= 1) {
+                const uint32_t msk = (1u << h) - 1u;
+                const int c = __popc(o01 & (msk | (msk << 16))) + __popc(o2 & msk);
+                const bool up = r >= c;
+                r -= up ? c : 0;
+                v += up ? h : 0;
+                o01 >>= up ? h : 0;
+                o2 >>= up ? h : 0;
             }
-        }
-        const int n = __popc(own);
-        const int incl = wave_inclusive_scan(n, lane);
-        const int excl = incl - n, total = __builtin_amdgcn_readlane(incl, 63);
-        int carry = 0;
-        for (int k0 = 0; k0 < total; k0 += 64) {
-            const int owner = weld_owner(nb.mark, excl, n, k0, lane, carry);
-            unsigned left = (unsigned)__shfl((int)own, owner, 64);
-            const int r = k0 + lane - __shfl(excl, owner, 64);
-            // the r-th set bit (r < 12), three at a time: a voxel's
-            int v = 0, rr = r;
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const int c = __popc((left >> (3 * v)) & 7u);
-                if (v == q && rr >= c) {
-                    rr -= c;
-                    ++v;
-                }
-            }
-            left = (left >> (3 * v)) & 7u;
-            const unsigned l1 = left & (left - 1u), l2 = l1 & (l1 - 1u);
-            const unsigned bit = rr == 0 ? left : (rr == 1 ? l1 : l2);
-            const int a = bit ? __builtin_ctz(bit) : 0;
-            weld_vertex(w, st, k0 + lane < total, x0 + 4 * owner + v, y, z, a, v0 + k0 + lane, verts, normals);
+            const bool ex = o01 & 1u, ey = (o01 >> 16) & 1u;
+            const int a = r == 0 ? (ex ? 0 : (ey ? 1 : 2)) : (r == 1 && ex && ey ? 1 : 2);
+            const int oi = owner >> 2;
+            weld_vertex(w, st, k0 + lane < nv, nb.x[oi] + 16 * (owner & 3) + v, nb.y[oi], nb.z[oi], a,
+                        v0 + k0 + lane, verts, normals);
         }
     }
-    if (!want_t) return;
-    // the lane's cubes from the signs of their rows (y,z), (y,z+1), (y+1,z),
-    // (y+1,z+1), five voxels from bit b
-    unsigned q[4];
+    if (end <= nv64) return;
+    uint32_t q[4];
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        const unsigned long long s = nb.s[5 * rr + slot];
-        q[rr] = (unsigned)(s >> b) & 0x1Fu;
-        if (b == 60) q[rr] |= ((unsigned)nb.s[5 * rr + slot + 1] & 1u) << 4;
+    for (int k = 0; k < 4; ++k) {
+        q[k] = (uint32_t)(nb.s[kGroupEntries * k + i] >> b) & 0x1FFFFu;
+        // the next chunk's first voxel (of another row past the last: no cube)
+        if (b == 48) q[k] |= ((uint32_t)nb.s[kGroupEntries * k + i + 1] & 1u) << 16;
     }
-    int nt[4], cls = 0;
+    const bool in = (c0 + (uint32_t)i < nchunks) & (nb.y[i] + 1 < p.gy) & (nb.z[i] + 1 < p.gz);
+    const CubeCounts cn4 = cube_counts(p, ntab, q, in, nb.x[i] + b);
+    const int mine = sum8(cn4.w[0]) + sum8(cn4.w[1]);
+    const int excl = wave_inclusive_scan(mine, lane) - mine;
+    const long long t0 = tsums[c0 / kBlockChunks] + toff[c0];
+    for (int k0 = max(first - nv64, 0); k0 < min(end - nv64, nt); k0 += 64) {
+        const int owner = weld_owner(nb.mark, excl, mine, k0, lane);
+        const uint32_t w0 = (uint32_t)__shfl((int)cn4.w[0], owner, 64);
+        const uint32_t w1 = (uint32_t)__shfl((int)cn4.w[1], owner, 64);
+        uint32_t oq[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const unsigned byte = ((q[0] >> j) & 3u) | (((q[1] >> j) & 3u) << 2) | (((q[2] >> j) & 3u) << 4) |
-                              (((q[3] >> j) & 3u) << 6);
-        const bool cube = (x0 + 4 * lane + j + 1 < p.gx) & (y + 1 < p.gy) & (z + 1 < p.gz);
-        nt[j] = cube ? (int)ntab[byte] : 0;
-        cls |= (int)(byte << (8 * j));
-    }
-    const int c1 = nt[0], c2 = c1 + nt[1], c3 = c2 + nt[2], n = c3 + nt[3];
-    const int cp = c1 | (c2 << 8) | (c3 << 16);  // each <= 15
-    const int incl = wave_inclusive_scan(n, lane);
-    const int excl = incl - n, total = __builtin_amdgcn_readlane(incl, 63);
-    int carry = 0;
-    for (int k0 = 0; k0 < total; k0 += 64) {
-        const int owner = weld_owner(nb.mark, excl, n, k0, lane, carry);
-        const int ocls = __shfl(cls, owner, 64), ocp = __shfl(cp, owner, 64);
-        const int local = k0 + lane - __shfl(excl, owner, 64);
-        const int o1 = ocp & 0xFF, o2 = (ocp >> 8) & 0xFF, o3 = (ocp >> 16) & 0xFF;
-        const int j = (local >= o1 ? 1 : 0) + (local >= o2 ? 1 : 0) + (local >= o3 ? 1 : 0);
-        const int slot3 = local - (j == 0 ? 0 : (j == 1 ? o1 : (j == 2 ? o2 : o3)));
-        if (k0 + lane < total) {
-            const uint64_t word = tri[(ocls >> (8 * j)) & 0xFF] >> (4 + 12 * slot3);
+        for (int k = 0; k < 4; ++k) oq[k] = (uint32_t)__shfl((int)q[k], owner, 64);
+        int r = k0 + lane - __shfl(excl, owner, 64);
+        // triangle r of the 16 cubes': halve the cubes
+        int j = 0;
+        const int c8 = sum8(w0);
+        uint32_t left = r >= c8 ? w1 : w0;
+        j += r >= c8 ? 8 : 0;
+        r -= r >= c8 ? c8 : 0;
+#pragma unroll
+        for (int h = 4; h >= 1; h >>= 1) {
+            const int c = sum8(left & ((1u << (4 * h)) - 1u));
+            const bool up = r >= c;
+            r -= up ? c : 0;
+            j += up ? h : 0;
+            left >>= up ? 4 * h : 0;
+        }
+        if (k0 + lane < nt) {
+            const uint64_t word = tri[cube_byte(oq, j)] >> (4 + 12 * r);
             const long long t = t0 + k0 + lane;
 #pragma unroll
             for (int e = 0; e < 3; ++e)
-                tris[3 * t + e] = weld_index(nb, 4 * owner + j, edges[(word >> (4 * e)) & 0xFull]);
+                tris[3 * t + e] = weld_index(nb, 64 * (owner >> 2) + 16 * (owner & 3) + j,
+                                             edges[(word >> (4 * e)) & 0xFull]);
         }
     }
 }
 
-// One wavefront per four windows: one load of their chunks' counts (most of a
-// volume's windows hold neither vertices nor triangles), then each busy
-// window.  A row's few vertices and triangles fill the lanes of one or two
-// rounds; chunk by chunk, with the field's corners read again, the pass was
-// bound by instruction issue (96 % VALU busy, ten vertices a round): 250 x
-// 333 x 287 voxels and 0.6 M vertices took 106 us, 59 this way.  Nothing is
-// written when the totals (*vtotal, *ttotal, from the scans) exceed int32
-// indices or a requested output's capacity: the host reports that after the
-// call.
-__global__ __launch_bounds__(256) void weld_write_kernel(const WeldParams w,
-                                                         const unsigned long long* __restrict__ signs,
-                                                         const int32_t* __restrict__ vcount,
-                                                         const long long* __restrict__ vbase,
-                                                         const int32_t* __restrict__ tcount,
-                                                         const long long* __restrict__ tbase,
-                                                         const long long* __restrict__ vtotal,
-                                                         const long long* __restrict__ ttotal,
-                                                         long long vcap, long long tcap,
-                                                         float* __restrict__ verts,
-                                                         float* __restrict__ normals,
-                                                         int32_t* __restrict__ tris) {
-    __shared__ WeldWindow windows[kWeldWaves];
+// The units of the list, strided over as many wavefronts as are resident: a
+// unit's vertices, then its triangles, are spread over the lanes 64 at a time.
+// The pass is bound by instruction issue and by its longest wavefront: lanes
+// without work and groups that a surface runs along (48 rounds) are its cost.
+// 250 x 333 x 287 voxels with 0.6 M vertices: chunk by chunk, with the field's
+// corners read again for the classes, 106 us (ten vertices a round); in units
+// of four chunks 59; a group a wavefront 52; units 34.
+// Nothing is written when the totals (from the scan) exceed int32 indices or
+// a requested output's capacity: the host reports that after the call.
+constexpr int kWriteBlocks = 256 * 8;  // 8 workgroups a CU by registers
+__global__ __launch_bounds__(64 * kWeldWaves) void weld_write_kernel(
+    const WeldParams w, const unsigned long long* __restrict__ signs, const int32_t* __restrict__ voff,
+    const int32_t* __restrict__ toff, const int2* __restrict__ group, const long long* __restrict__ vsums,
+    const long long* __restrict__ tsums, const long long* __restrict__ total,
+    const uint32_t* __restrict__ units, const uint32_t* __restrict__ nunits, long long vcap,
+    long long tcap, float* __restrict__ verts, float* __restrict__ normals, int32_t* __restrict__ tris) {
+    __shared__ WeldGroup groups[kWeldWaves];
     __shared__ uint64_t tri[256];    // triangle table by the signs' byte
     __shared__ uint8_t ntab[256];    // its triangle counts
     __shared__ uint32_t edges[16];   // axis | dx << 2 | (2 dy + dz) << 3 of an edge's lower end
-    const long long nvt = *vtotal, ntt = *ttotal;
-    const bool want_v = verts || normals;
-    if (nvt > INT32_MAX || (want_v && nvt > vcap) || (tris && ntt > tcap)) return;
+    const McParams& p = w.mc;
+    const bool want_v = verts || normals, want_t = tris != nullptr;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t nu = *nunits;
+    const long long nvt = total[0], ntt = total[1];
+    if (kWeldWaves * blockIdx.x >= nu || nvt > INT32_MAX || (want_v && nvt > vcap) || (want_t && ntt > tcap))
+        return;
     tri[threadIdx.x] = c_tri[qbyte_class((int)threadIdx.x)];
     ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
     if (threadIdx.x < 12) {
@@ -504,7 +693,6 @@ __global__ __launch_bounds__(256) void weld_write_kernel(const WeldParams w,
         edges[e] = (unsigned)__builtin_ctz(oa ^ ob) | ((lo & 1u) << 2) | (((lo & 2u) | (lo >> 2)) << 3);
     }
     __syncthreads();
-    const McParams& p = w.mc;
     WeldSteps st;
     st.ok = true;
 #pragma unroll
@@ -514,35 +702,19 @@ __global__ __launch_bounds__(256) void weld_write_kernel(const WeldParams w,
         st.r2[k] = recip_sum(p.vs[k] + p.vs[k], bad);
         st.ok = st.ok && bad < kRecipBad && p.vs[k] >= 1e-6f && p.vs[k] <= 1e6f;
     }
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int wpr = (w.cpr + kWinChunks - 1) / kWinChunks;  // windows per row
-    const uint32_t nwin = (uint32_t)wpr * (uint32_t)(p.gy * p.gz);  // <= nchunks
-    const uint32_t win0 = 4u * (blockIdx.x * kWeldWaves + (uint32_t)wave);
-    int n = 0;
-    if (lane < 16 && win0 + (lane >> 2) < nwin) {
-        const uint32_t win = win0 + (lane >> 2);
-        const int row = (int)(win / (uint32_t)wpr);
-        const int j = kWinChunks * ((int)win - row * wpr) + (lane & 3);
-        if (j < w.cpr) {
-            const int64_t c = (int64_t)row * w.cpr + j;
-            n = (want_v ? vcount[c] : 0) + (tris ? tcount[c] : 0);
-        }
-    }
-    const unsigned long long busy = __ballot(n > 0);
-    for (int k = 0; k < 4; ++k) {
-        if (!((busy >> (4 * k)) & 15ull)) continue;
-        const uint32_t win = win0 + k;
-        const int row = (int)(win / (uint32_t)wpr), j0 = kWinChunks * ((int)win - row * wpr);
-        const int64_t c = (int64_t)row * w.cpr + j0;
-        weld_write_window(w, st, row, j0, lane, signs, vbase, vbase[c], tbase[c], want_v, tris != nullptr,
-                          windows[wave], tri, ntab, edges, verts, normals, tris);
+    for (uint32_t u = kWeldWaves * blockIdx.x + (uint32_t)wave; u < nu; u += kWeldWaves * gridDim.x) {
+        const uint32_t unit = (uint32_t)__builtin_amdgcn_readfirstlane((int)units[u]);
+        const uint32_t g = unit >> kUnitBits;
+        const int2 n = group[g];
+        weld_write_unit(w, st, g * kGroupChunks, lane,
+                        64 * kUnitRounds * (int)(unit & ((1u << kUnitBits) - 1u)), want_v ? n.x : 0,
+                        want_t ? n.y : 0, signs, voff, toff, vsums, tsums, groups[wave], tri, ntab, edges,
+                        verts, normals, tris);
         __builtin_amdgcn_wave_barrier();
     }
 }
 
 static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-
 
 // Counts (always), then writes what is asked for when it fits.
 static int weld_run(const float* field, const int32_t grid[3], const float vs[3], const float off[3],
@@ -567,15 +739,19 @@ static int weld_run(const float* field, const int32_t grid[3], const float vs[3]
     }
     w.cpr = (grid[0] + 63) / 64;
     w.nchunks = w.cpr * grid[1] * grid[2];
-    const int nb = (w.nchunks + kScanBlock - 1) / kScanBlock;
+    div31_make((uint32_t)w.cpr, w.mul_cpr, w.sh_cpr);
+    div31_make((uint32_t)grid[1], w.mul_gy, w.sh_gy);
+    const int nb = (w.nchunks + kBlockChunks - 1) / kBlockChunks;
     const size_t o_signs = 0;
-    const size_t o_vcount = o_signs + align256(8 * (size_t)w.nchunks);
-    const size_t o_tcount = o_vcount + align256(4 * (size_t)w.nchunks);
-    const size_t o_vbase = o_tcount + align256(4 * (size_t)w.nchunks);
-    const size_t o_tbase = o_vbase + align256(8 * (size_t)w.nchunks);
-    const size_t o_vsums = o_tbase + align256(8 * (size_t)w.nchunks);
-    const size_t o_tsums = o_vsums + align256(8 * (size_t)(nb + 1));
-    const size_t need = o_tsums + align256(8 * (size_t)(nb + 1));
+    const size_t o_voff = o_signs + align256(8 * (size_t)w.nchunks);
+    const size_t o_toff = o_voff + align256(4 * (size_t)w.nchunks);
+    const size_t o_group = o_toff + align256(4 * (size_t)w.nchunks);
+    const size_t o_vsums = o_group + align256(8 * (size_t)nb * kBlockGroups);
+    const size_t o_tsums = o_vsums + align256(8 * (size_t)nb);
+    const size_t o_total = o_tsums + align256(8 * (size_t)nb);
+    const size_t o_nunits = o_total + 256;
+    const size_t o_units = o_nunits + 256;
+    const size_t need = o_units + align256((sizeof(uint32_t) << kUnitBits) * nb * kBlockGroups);
     if (*scratch_bytes < need) {
         if (*scratch) (void)hipFree(*scratch);
         *scratch = nullptr;
@@ -585,41 +761,37 @@ static int weld_run(const float* field, const int32_t grid[3], const float vs[3]
     }
     char* sb = static_cast<char*>(*scratch);
     auto* signs = reinterpret_cast<unsigned long long*>(sb + o_signs);
-    auto* vcount = reinterpret_cast<int32_t*>(sb + o_vcount);
-    auto* tcount = reinterpret_cast<int32_t*>(sb + o_tcount);
-    auto* vbase = reinterpret_cast<long long*>(sb + o_vbase);
-    auto* tbase = reinterpret_cast<long long*>(sb + o_tbase);
+    auto* voff = reinterpret_cast<int32_t*>(sb + o_voff);
+    auto* toff = reinterpret_cast<int32_t*>(sb + o_toff);
+    auto* group = reinterpret_cast<int2*>(sb + o_group);
     auto* vsums = reinterpret_cast<long long*>(sb + o_vsums);
     auto* tsums = reinterpret_cast<long long*>(sb + o_tsums);
-    const int count_blocks =
-        (((grid[1] + kWeldRows - 1) / kWeldRows) * grid[2] + kWeldWaves - 1) / kWeldWaves;
-    hipLaunchKernelGGL(weld_count_kernel, dim3(count_blocks), dim3(256), 0, s, w, signs, vcount,
-                       tcount);
-    RECON_HIP_TRY(hipGetLastError(), "weld_count_kernel launch");
-    ScanJobs jobs;
-    jobs.in[0] = vcount;
-    jobs.in[1] = tcount;
-    jobs.sums[0] = vsums;
-    jobs.sums[1] = tsums;
-    jobs.out[0] = vbase;
-    jobs.out[1] = tbase;
-    const int rc = launch_exclusive_scans(jobs, 2, w.nchunks, s);
-    if (rc) return rc;
-    // The write pass checks the totals on the device, so it is queued before
-    // the host waits; the copies of the totals to pageable memory come last,
-    // since each returns only when the stream has reached it.
+    auto* total = reinterpret_cast<long long*>(sb + o_total);
+    auto* nunits = reinterpret_cast<uint32_t*>(sb + o_nunits);
+    auto* units = reinterpret_cast<uint32_t*>(sb + o_units);
     const bool write = verts || normals || tris;
+    constexpr int kSignBlock = kSignChunks * kWeldWaves;
+    hipLaunchKernelGGL(weld_sign_kernel, dim3((w.nchunks + kSignBlock - 1) / kSignBlock),
+                       dim3(64 * kWeldWaves), 0, s, w, signs, nunits);
+    RECON_HIP_TRY(hipGetLastError(), "weld_sign_kernel launch");
+    hipLaunchKernelGGL(weld_count_kernel, dim3(nb), dim3(64 * kBlockGroups), 0, s, w, signs, voff, toff,
+                       group, vsums, tsums, verts || normals, tris != nullptr, units, nunits);
+    RECON_HIP_TRY(hipGetLastError(), "weld_count_kernel launch");
+    hipLaunchKernelGGL(weld_scan_kernel, dim3(2), dim3(256), 0, s, vsums, tsums, nb, total);
+    RECON_HIP_TRY(hipGetLastError(), "weld_scan_kernel launch");
+    // The write pass checks the totals on the device, so it is queued before
+    // the host waits; the copy of the totals to pageable memory comes last,
+    // since it returns only when the stream has reached it.
     if (write) {
-        const long long windows = (long long)((w.cpr + kWinChunks - 1) / kWinChunks) * grid[1] * grid[2];
-        const unsigned blocks = (unsigned)((windows + 4 * kWeldWaves - 1) / (4 * kWeldWaves));
-        hipLaunchKernelGGL(weld_write_kernel, dim3(blocks), dim3(256), 0, s, w, signs, vcount,
-                           vbase, tcount, tbase, vsums + nb, tsums + nb, (long long)vcap,
+        // most groups are empty and a busy one is one or two units
+        const int blocks = std::min(kWriteBlocks, nb * kBlockGroups);
+        hipLaunchKernelGGL(weld_write_kernel, dim3(blocks), dim3(64 * kWeldWaves), 0, s, w, signs, voff,
+                           toff, group, vsums, tsums, total, units, nunits, (long long)vcap,
                            (long long)tcap, verts, normals, tris);
         RECON_HIP_TRY(hipGetLastError(), "weld_write_kernel launch");
     }
     long long totals[2] = {0, 0};
-    RECON_HIP_TRY(hipMemcpyAsync(&totals[0], vsums + nb, 8, hipMemcpyDeviceToHost, s), "vertex total");
-    RECON_HIP_TRY(hipMemcpyAsync(&totals[1], tsums + nb, 8, hipMemcpyDeviceToHost, s), "triangle total");
+    RECON_HIP_TRY(hipMemcpyAsync(totals, total, 16, hipMemcpyDeviceToHost, s), "totals");
     RECON_HIP_TRY(hipStreamSynchronize(s), "welded marching cubes");
     *nv_out = totals[0];
     *nt_out = totals[1];
