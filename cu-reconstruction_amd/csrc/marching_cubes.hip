@@ -5,40 +5,34 @@
 // kernel per z layer, synchronises, and compacts each layer on the host from
 // managed memory.  Here the whole volume is done on the device in four
 // launches with a fixed, deterministic output order:
+//   1-3. signs, counts, scan (mc_signs.hip): a word of signs per 64 voxels,
+//        the triangles per 64-cube chunk from the words, each chunk's first
+//        triangle, and a list of units of up to 256 triangles;
+//   4.   emit - the resident wavefronts stride over the units: a unit's cubes
+//        are classified from the signs (16 a lane), its triangles spread over
+//        the lanes 64 at a time, a lane reading the six field values of its
+//        triangle's edges (marching_cubes.cu:23-74).
+// The allocation-free entry, whose static scratch has no room for the words
+// and the list, keeps to a smaller one (2 B per 64 cubes):
 //   1. chunk count - one wavefront per 4 cube rows (y..y+3, z), streaming
 //                    their 10 voxel rows once, 256 cubes a step (16-byte
 //                    loads; 64 with 4-byte loads where rows are not 16-byte
-//                    aligned): every
-//                    cube's class (marching_cubes.cu:76-84,118-130) from
-//                    the corners' sign bits, its triangle count from a
-//                    table, and per 64-cube chunk of each row the chunk's
-//                    triangle count; per workgroup ("tile", 16 cube rows)
-//                    the tile's total and its number of chunks with
-//                    triangles;
-//   2. tile scan   - one workgroup: exclusive scans of the tile totals
-//                    (each tile's first triangle and the volume's total)
-//                    and of the tiles' groups of four chunks with
-//                    triangles;
-//   3. group prep  - one wavefront per tile: a 16-byte record per group of
-//                    four chunks with triangles (its tile, first triangle
-//                    and chunks);
-//   4. emit        - a grid sized to the resident workgroups: each
-//                    wavefront takes groups gi = wave, wave + waves, ...,
-//                    reads each group's record and spreads its triangles
-//                    (16 lanes per chunk, 4 cubes per lane) over its 64
-//                    lanes to compute the vertices (marching_cubes.cu:23-74),
-//                    staged in LDS and written in consecutive dwords.  A tile
-//                    dense with triangles (a floor along a cube layer) is
-//                    thus shared by many wavefronts.  The allocation-free
-//                    entry skips step 3 (its static scratch has no room for
-//                    the records) and finds each group's tile and chunks by
-//                    a search and a walk instead.
+//                    aligned): every cube's class from the corners' sign
+//                    bits, and per 64-cube chunk of each row its triangle
+//                    count; per workgroup ("tile", 16 cube rows) the tile's
+//                    total and its number of chunks with triangles;
+//   2. tile scan   - one workgroup: exclusive scans of the tile totals and of
+//                    the tiles' groups of four chunks with triangles;
+//   3. emit        - each wavefront takes groups gi = wave, wave + waves, ...,
+//                    finds the group's tile and chunks by a search and a walk,
+//                    and spreads its triangles over its 64 lanes
+//                    (mc_emit_group, also the batch's).
 // Output order is cube z, y, x, table slot -- the order the reference's host
 // loop produces (marching_cubes.cu:163-188 inside :213-225) -- as a triangle
 // soup: triangle t owns vertices 3t, 3t+1, 3t+2 (marching_cubes.cu:171).
 #pragma clang fp contract(off)
 
-#include "mc_device.hpp"
+#include "mc_signs.hpp"
 
 #include <algorithm>
 #include <mutex>
@@ -182,44 +176,180 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
     mc_count_tile4(p, tl, blockIdx.x, cc, ntab, wtot, tile_sum + blockIdx.x, tile_nne + blockIdx.x);
 }
 
-// One wavefront per tile: the records of the tile's groups (mc_group_prep).
-__global__ __launch_bounds__(256) void mc_group_prep_kernel(const McParams p, const McTiling tl,
-                                                            const uint16_t* __restrict__ cc,
-                                                            const long long* __restrict__ tile_off,
-                                                            const int32_t* __restrict__ tile_nne,
-                                                            const int32_t* __restrict__ group_off,
-                                                            McGroupRec* __restrict__ rec) {
-    const int b = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (b < tl.tiles)
-        mc_group_prep(p, tl, b, cc, tile_off, tile_nne, group_off, rec, (int)(threadIdx.x & 63));
+// ---- emit from signs -------------------------------------------------------------
+// LDS of a wavefront: the words of its unit's chunks (a lane each), of rows
+// (y,z), (y,z+1), (y+1,z), (y+1,z+1).
+struct UnitEmitLds {
+    unsigned long long s[4][64];
+    int mark[64];
+    float stage[64 * 9];  // 64 triangles' vertices
+};
+
+// The place of set bit r of m.
+__device__ __forceinline__ int set_bit(unsigned long long m, int r) {
+    const uint32_t lo = (uint32_t)m;
+    const int c32 = __popc(lo);
+    uint32_t v = r >= c32 ? (uint32_t)(m >> 32) : lo;
+    int k = r >= c32 ? 32 : 0;
+    r -= r >= c32 ? c32 : 0;
+#pragma unroll
+    for (int h = 16; h >= 1; h >>= 1) {
+        const int c = __popc(v & ((1u << h) - 1u));
+        const bool up = r >= c;
+        r -= up ? c : 0;
+        k += up ? h : 0;
+        v >>= up ? h : 0;
+    }
+    return k;
 }
 
-// A grid sized to the resident workgroups walks the volume's groups of four
-// chunks with triangles, wavefront by wavefront (gi = wave, wave + waves,
-// ...), each from its record (one scalar load, which unlike a vector load
-// does not wait for the wavefront's earlier stores): the groups of a tile
-// dense with triangles (a floor along a cube layer) go to as many
-// wavefronts.
-__global__ __launch_bounds__(256) void mc_chunk_emit_kernel(const McParams p, const McTiling tl,
-                                                            const McGroupRec* __restrict__ rec,
-                                                            const int32_t* __restrict__ group_off,
-                                                            float* __restrict__ verts,
-                                                            int32_t* __restrict__ tris,
-                                                            long long capacity) {
-    __shared__ McEmitLds lds;
-    mc_emit_lds_init(lds);
-    __syncthreads();
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+// One wavefront per unit, strided over as many as are resident: the cubes with
+// both signs of its chunks, 64 at a time, and their triangles, 64 at a time;
+// triangles below the capacity are written.  The lanes fill whether a surface
+// crosses a row once (a wall) or runs along it (a floor): 512^3 voxels
+// with 3.3 M triangles 70 us, 2.9 TB/s of field values and output, half of it
+// instruction issue; by groups of four 64-cube chunks, their voxel values
+// passed between the lanes, it took 116 and 5 for the groups' records.  Units
+// of 64 cubes instead of 256 take 9 us off a mesh of 64^3 voxels (fewer
+// rounds one after the other) and 1 us off this one.
+constexpr int kEmitBlocks = 256 * 7;  // 7 workgroups a CU by LDS
+__global__ __launch_bounds__(64 * kUnitWaves) void mc_unit_emit_kernel(
+    const SignParams w, const unsigned long long* __restrict__ signs, const int32_t* __restrict__ toff,
+    const long long* __restrict__ tsums, const unsigned long long* __restrict__ units,
+    const uint32_t* __restrict__ nunits, float* __restrict__ verts, int32_t* __restrict__ tris,
+    long long capacity) {
+    __shared__ UnitEmitLds lds[kUnitWaves];
+    __shared__ uint64_t tri[256];   // triangle table by the signs' byte
+    __shared__ uint8_t ntab[256];   // its triangle counts
+    __shared__ int4 ends[12];       // an edge's ends: voxel offsets a, b; dx | dy << 1 | dz << 2 of a, b
+    const McParams& p = w.mc;
     const int lane = threadIdx.x & 63;
-    const int ngroups = group_off[tl.tiles];
-    const int waves = (int)gridDim.x * 4;
-    for (int gi = (int)blockIdx.x * 4 + wave; gi < ngroups; gi += waves)
-        mc_emit_group_rec(p, tl, rec[gi], lds, wave, lane, verts, tris, capacity);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t nu = *nunits;
+    if (kUnitWaves * blockIdx.x >= nu) return;
+    tri[threadIdx.x] = c_tri[qbyte_class((int)threadIdx.x)];
+    ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
+    if (threadIdx.x < 12) {
+        // corner offsets packed as bits: dx = bit0, dy = bit1, dz = bit2
+        // (0:000 1:001 2:101 3:100 4:010 5:011 6:111 7:110)
+        constexpr unsigned k_off = (0u << 0) | (1u << 3) | (5u << 6) | (4u << 9) | (2u << 12) |
+                                   (3u << 15) | (7u << 18) | (6u << 21);
+        const int e = (int)threadIdx.x;
+        const int ca = (int)((kEdgeA >> (4 * e)) & 0xFull), cb = (int)((kEdgeB >> (4 * e)) & 0xFull);
+        const int oa = (int)((k_off >> (3 * ca)) & 7u), ob = (int)((k_off >> (3 * cb)) & 7u);
+        auto place = [&](int o) {
+            return (o & 1) + ((o >> 1) & 1) * p.gx + (o >> 2) * p.gx * p.gy;
+        };
+        ends[e] = make_int4(place(oa), place(ob), oa, ob);
+    }
+    __syncthreads();
+    UnitEmitLds& l = lds[wave];
+    for (uint32_t u = kUnitWaves * blockIdx.x + (uint32_t)wave; u < nu; u += kUnitWaves * gridDim.x) {
+        const unsigned long long unit = units[u];
+        const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(unit >> 6));
+        const int len = 1 + __builtin_amdgcn_readfirstlane((int)(unit & 63ull));
+        long long t0 = tsums[c0 / kBlockChunks] + toff[c0];
+        const uint32_t c = c0 + (uint32_t)(lane < len ? lane : 0);
+        const ChunkPlace at = chunk_place(w, c);
+        const ChunkWords v = chunk_words(w, signs, c, at, lane < len);
+        const unsigned long long mixed = mixed_cubes(p, v, at, lane < len);
+        const uint32_t nb = next_bits(v);
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) l.s[rr][lane] = v.s[rr];
+        const int cubes = __popcll(mixed), incl = wave_inclusive_scan(cubes, lane);
+        const int excl = incl - cubes, all = __builtin_amdgcn_readlane(incl, 63);
+        for (int q0 = 0; q0 < all; q0 += 64) {
+            // the lane's cube
+            const int chunk = unit_owner(l.mark, excl, cubes, q0, lane);
+            const unsigned long long om =
+                ((unsigned long long)(uint32_t)__shfl((int)(mixed >> 32), chunk, 64) << 32) |
+                (uint32_t)__shfl((int)mixed, chunk, 64);
+            const int k = set_bit(om, q0 + lane - __shfl(excl, chunk, 64));
+            const unsigned long long s[4] = {l.s[0][chunk], l.s[1][chunk], l.s[2][chunk], l.s[3][chunk]};
+            const uint32_t byte = cube_byte64(s, (uint32_t)__shfl((int)nb, chunk, 64), k & 63) & 0xFFu;
+            const ChunkPlace cat = chunk_place(w, c0 + (uint32_t)chunk);
+            const int cx = 64 * cat.j + k;
+            const int n = q0 + lane < all ? (int)ntab[byte] : 0;
+            const int tincl = wave_inclusive_scan(n, lane), texcl = tincl - n;
+            const int nt = __builtin_amdgcn_readlane(tincl, 63);
+            const int pk = (int)byte | (texcl << 8);
+            for (int k0 = 0; k0 < nt; k0 += 64) {
+                const int owner = unit_owner(l.mark, texcl, n, k0, lane);
+                const int opk = __shfl(pk, owner, 64);
+                const int x = __shfl(cx, owner, 64), y = __shfl(cat.y, owner, 64), z = __shfl(cat.z, owner, 64);
+                const int r = k0 + lane - (opk >> 8);
+                if (k0 + lane < nt) {
+                    const float* __restrict__ f = p.f + ((size_t)x + (size_t)p.gx * ((size_t)y + (size_t)p.gy * z));
+                    const uint64_t word3 = tri[opk & 0xFF] >> (4 + 12 * r);
+                    float wa[3], wb[3];
+                    int da[3], db[3];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        const int4 d = ends[(word3 >> (4 * e)) & 0xFull];
+                        wa[e] = f[d.x];
+                        wb[e] = f[d.y];
+                        da[e] = d.z;
+                        db[e] = d.w;
+                    }
+                    const int cube[3] = {x, y, z};
+                    float ctr[3][2];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        ctr[k][0] = voxel_centre(cube[k], p.vs[k], p.off[k]);
+                        ctr[k][1] = voxel_centre(cube[k] + 1, p.vs[k], p.off[k]);
+                    }
+                    float out[9];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        // from the negative end when the first is above zero and
+                        // the second below (marching_cubes.cu:23-51)
+                        const bool swap = (wa[e] > 0.0f) & (wb[e] < 0.0f);
+                        const float s = swap ? wb[e] : wa[e], en = swap ? wa[e] : wb[e];
+                        const int os = swap ? db[e] : da[e], oe = swap ? da[e] : db[e];
+                        const float den = en - s;
+                        float res = 0.0f;
+                        const float y_den = recip_sum(den, res);
+                        bool bad = !(res < kRecipBad) | !(fabsf(den) <= 1e7f);
+                        float ratio = short_quotient(-s, den, y_den, bad);
+                        if (__builtin_expect(bad, 0)) ratio = (-s) / den;
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            const float cs = (os >> k) & 1 ? ctr[k][1] : ctr[k][0];
+                            const float ce = (oe >> k) & 1 ? ctr[k][1] : ctr[k][0];
+                            const float edge = ce - cs;
+                            const float o = ratio * edge;
+                            out[3 * e + k] = cs + o;
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) l.stage[9 * lane + q] = out[q];
+                }
+                __builtin_amdgcn_wave_barrier();
+                const long long tb = t0 + k0;
+                const int m = (int)min((long long)min(64, nt - k0), max(capacity - tb, 0ll));
+                float* __restrict__ dst = verts + 9 * tb;
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    if (64 * q + lane < 9 * m) dst[64 * q + lane] = l.stage[64 * q + lane];
+                if (tris) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        if (64 * q + lane < 3 * m)
+                            tris[3 * tb + 64 * q + lane] = (int32_t)(3 * tb + 64 * q + lane);
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+            t0 += nt;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
 }
 
-// The same walk for the allocation-free entry (no room for records): each
-// wavefront finds its group's tile by a search over group_off and its
-// chunks by a walk over the tile's chunk counts (mc_emit_group_at).
+// The emit of the allocation-free entry: a grid sized to the resident
+// workgroups walks the volume's groups of four chunks with triangles,
+// wavefront by wavefront; each finds its group's tile by a search over
+// group_off and its chunks by a walk over the tile's chunk counts
+// (mc_emit_group_at).
 __global__ __launch_bounds__(256) void mc_chunk_emit_search_kernel(const McParams p, const McTiling tl,
                                                             const uint16_t* __restrict__ cc,
                                                             const long long* __restrict__ tile_off,
@@ -390,20 +520,14 @@ static int check_grid(const float* field, const int32_t grid[3], const float vs[
     return RECON_OK;
 }
 
-// Tiling of a grid (host side) and the scratch layout: chunk counts
-// uint16[rows * nch] | tile sums int32[tiles] | tile chunks with triangles
-// int32[tiles] | tile offsets int64[tiles+1] | tile first groups
-// int32[tiles+1] (need bytes, the search emit's) | group records
-// McGroupRec[4 * nch per tile] (need_rec bytes in all, the record emit's),
-// each part 256-byte aligned.  Records fit their fields when the tile index
-// stays below 2^24, the triangle count below 2^40 (at most 5 per cube) and a
-// tile's chunks below kNoChunk.
+// Tiling of a grid (host side) and the scratch layout of the allocation-free
+// entry: chunk counts uint16[rows * nch] | tile sums int32[tiles] | tile chunks
+// with triangles int32[tiles] | tile offsets int64[tiles+1] | tile first groups
+// int32[tiles+1], each part 256-byte aligned.
 struct McScratchLayout {
     McTiling t{0, 0, 0, 0};
     int gpl = 0, groups = 0, tiles = 0, nch = 0;
     size_t off_sum = 0, off_nne = 0, off_off = 0, off_goff = 0, need = 0;
-    size_t off_rec = 0, need_rec = 0;
-    bool rec_ok = false;
     explicit McScratchLayout(const int32_t grid[3]) {
         if (grid[0] < 2 || grid[1] < 2 || grid[2] < 2) return;
         t = mc_tiling(grid[0], grid[1], grid[2]);
@@ -418,56 +542,90 @@ struct McScratchLayout {
         off_off = off_nne + a256(4 * (size_t)tiles);
         off_goff = off_off + a256(8 * ((size_t)tiles + 1));
         need = off_goff + 4 * ((size_t)tiles + 1);
-        off_rec = a256(need);
-        need_rec = off_rec + sizeof(McGroupRec) * (size_t)tiles * 4 * (size_t)nch;
-        const double cubes = (double)(grid[0] - 1) * (double)rows;
-        rec_ok = tiles < (1 << 24) && 5.0 * cubes < 0x1p40 && 16 * (size_t)nch < kNoChunk;
     }
 };
 
-// Workgroups of an emit pass: its resident slots on every CU of the current
-// device (looked up once per device and kernel; which = 0 the record emit,
-// 1 the search emit).
-static int emit_grid(int which) {
+// Workgroups of the search emit: its resident slots on every CU of the current
+// device (looked up once per device).
+static int emit_grid() {
     static std::mutex mu;
-    static int grid[2][64] = {{0}};
+    static int grid[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1024;
     std::lock_guard<std::mutex> lk(mu);
-    if (!grid[which][dev]) {
+    if (!grid[dev]) {
         int cus = 0, occ = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             cus < 1)
             cus = 256;
-        const hipError_t e =
-            which == 0
-                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, mc_chunk_emit_kernel, 256, 0)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, mc_chunk_emit_search_kernel,
-                                                               256, 0);
-        if (e != hipSuccess || occ < 1) occ = 1;
-        grid[which][dev] = cus * occ;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, mc_chunk_emit_search_kernel, 256, 0) !=
+                hipSuccess ||
+            occ < 1)
+            occ = 1;
+        grid[dev] = cus * occ;
     }
-    return grid[which][dev];
+    return grid[dev];
 }
 
 size_t mc_scratch_need(const int32_t grid[3]) { return McScratchLayout(grid).need; }
+
+// The total of a run whose launches are all queued (the emit checks the
+// capacity on the device): the copy to pageable memory comes last, since it
+// returns only when the stream has reached it.
+static int read_total(const long long* dev, int64_t* total, hipStream_t s) {
+    long long host_total = 0;
+    RECON_HIP_TRY(hipMemcpyAsync(&host_total, dev, sizeof(long long), hipMemcpyDeviceToHost, s),
+                  "marching cubes total");
+    RECON_HIP_TRY(hipStreamSynchronize(s), "marching cubes synchronize");
+    *total = host_total;
+    return RECON_OK;
+}
+
+// The allocation-free entry's passes.
+static int mc_run_noalloc(const McParams& p, const int32_t grid[3], float* verts, int32_t* tris,
+                          int64_t capacity, int64_t* total, bool count_only, void* scratch,
+                          size_t scratch_bytes, hipStream_t s) {
+    const McScratchLayout L(grid);
+    if ((int64_t)(grid[1] - 1) * (grid[2] - 1) * L.nch >= (int64_t(1) << 31))
+        return fail(RECON_ERR_RANGE, "marching cubes: more than 2^31 64-cube chunks");
+    if (scratch_bytes < L.need)
+        return fail(RECON_ERR_RANGE, "marching cubes needs %zu bytes of scratch, %zu available",
+                    L.need, scratch_bytes);
+    char* sb = static_cast<char*>(scratch);
+    uint16_t* cc = reinterpret_cast<uint16_t*>(sb);
+    int32_t* tile_sum = reinterpret_cast<int32_t*>(sb + L.off_sum);
+    int32_t* tile_nne = reinterpret_cast<int32_t*>(sb + L.off_nne);
+    long long* tile_off = reinterpret_cast<long long*>(sb + L.off_off);
+    int32_t* group_off = reinterpret_cast<int32_t*>(sb + L.off_goff);
+    if (grid[0] % 4 == 0 && reinterpret_cast<uintptr_t>(p.f) % 16 == 0)
+        hipLaunchKernelGGL(mc_chunk_count4_kernel, dim3(L.tiles), dim3(256), 0, s, p, L.t, cc,
+                           tile_sum, tile_nne);
+    else
+        hipLaunchKernelGGL(mc_chunk_count_kernel, dim3(L.tiles), dim3(256), 0, s, p, L.t, cc,
+                           tile_sum, tile_nne);
+    RECON_HIP_TRY(hipGetLastError(), "mc_chunk_count_kernel launch");
+    const int rc = launch_tile_scan(tile_sum, L.tiles, tile_off, s, tile_nne, group_off);
+    if (rc) return rc;
+    if (!count_only && capacity > 0 && verts) {
+        hipLaunchKernelGGL(mc_chunk_emit_search_kernel, dim3(emit_grid()), dim3(256), 0, s, p,
+                           L.t, cc, tile_off, tile_nne, group_off, verts, tris,
+                           (long long)capacity);
+        RECON_HIP_TRY(hipGetLastError(), "mc_chunk_emit_search_kernel launch");
+    }
+    return read_total(tile_off + L.tiles, total, s);
+}
 
 int mc_run(const float* field, const int32_t grid[3], const float vs[3], const float off[3],
            float* verts, int32_t* tris, int64_t capacity, int64_t* total, bool count_only,
            void** scratch, size_t* scratch_bytes, hipStream_t s, bool may_allocate) {
     *total = 0;
     if (grid[0] < 2 || grid[1] < 2 || grid[2] < 2) return RECON_OK;
-    const McParams p = make_params(field, grid, vs, off);
-    const McScratchLayout L(grid);
-    if ((int64_t)(grid[1] - 1) * (grid[2] - 1) * L.nch >= (int64_t(1) << 31))
-        return fail(RECON_ERR_RANGE, "marching cubes: more than 2^31 64-cube chunks");
-    if (*scratch_bytes < L.need && !may_allocate)
-        return fail(RECON_ERR_RANGE, "marching cubes needs %zu bytes of scratch, %zu available",
-                    L.need, *scratch_bytes);
-    // the record emit when allocating; the allocation-free entry keeps to the
-    // search emit's smaller scratch
-    const bool use_rec = L.rec_ok && may_allocate;
-    const size_t need = use_rec ? L.need_rec : L.need;
+    if (!may_allocate)
+        return mc_run_noalloc(make_params(field, grid, vs, off), grid, verts, tris, capacity, total,
+                              count_only, *scratch, *scratch_bytes, s);
+    SignParams w;
+    SignScratch sc;
+    const size_t need = sign_layout(field, grid, vs, off, false, nullptr, w, sc);
     if (*scratch_bytes < need) {
         if (*scratch) (void)hipFree(*scratch);
         *scratch = nullptr;
@@ -475,47 +633,18 @@ int mc_run(const float* field, const int32_t grid[3], const float vs[3], const f
         RECON_HIP_TRY(hipMalloc(scratch, need), "marching cubes scratch");
         *scratch_bytes = need;
     }
-    char* sb = static_cast<char*>(*scratch);
-    uint16_t* cc = reinterpret_cast<uint16_t*>(sb);
-    int32_t* tile_sum = reinterpret_cast<int32_t*>(sb + L.off_sum);
-    int32_t* tile_nne = reinterpret_cast<int32_t*>(sb + L.off_nne);
-    long long* tile_off = reinterpret_cast<long long*>(sb + L.off_off);
-    int32_t* group_off = reinterpret_cast<int32_t*>(sb + L.off_goff);
-    McGroupRec* rec = reinterpret_cast<McGroupRec*>(sb + L.off_rec);
-    if (grid[0] % 4 == 0 && reinterpret_cast<uintptr_t>(field) % 16 == 0)
-        hipLaunchKernelGGL(mc_chunk_count4_kernel, dim3(L.tiles), dim3(256), 0, s, p, L.t, cc,
-                           tile_sum, tile_nne);
-    else
-        hipLaunchKernelGGL(mc_chunk_count_kernel, dim3(L.tiles), dim3(256), 0, s, p, L.t, cc,
-                           tile_sum, tile_nne);
-    RECON_HIP_TRY(hipGetLastError(), "mc_chunk_count_kernel launch");
-    int rc = launch_tile_scan(tile_sum, L.tiles, tile_off, s, tile_nne, group_off);
+    sign_layout(field, grid, vs, off, false, static_cast<char*>(*scratch), w, sc);
+    const bool write = !count_only && capacity > 0 && verts;
+    const int rc = launch_signs(w, sc, false, false, write, s);
     if (rc) return rc;
-    // The emit checks the capacity on the device, so every launch is queued
-    // before the host waits: the copy of the total to pageable memory comes
-    // last, since it returns only when the stream has reached it.
-    if (!count_only && capacity > 0 && verts) {
-        if (use_rec) {
-            hipLaunchKernelGGL(mc_group_prep_kernel, dim3((L.tiles + 3) / 4), dim3(256), 0, s, p,
-                               L.t, cc, tile_off, tile_nne, group_off, rec);
-            RECON_HIP_TRY(hipGetLastError(), "mc_group_prep_kernel launch");
-            hipLaunchKernelGGL(mc_chunk_emit_kernel, dim3(emit_grid(0)), dim3(256), 0, s, p, L.t,
-                               rec, group_off, verts, tris, (long long)capacity);
-            RECON_HIP_TRY(hipGetLastError(), "mc_chunk_emit_kernel launch");
-        } else {
-            hipLaunchKernelGGL(mc_chunk_emit_search_kernel, dim3(emit_grid(1)), dim3(256), 0, s, p,
-                               L.t, cc, tile_off, tile_nne, group_off, verts, tris,
-                               (long long)capacity);
-            RECON_HIP_TRY(hipGetLastError(), "mc_chunk_emit_search_kernel launch");
-        }
+    if (write) {
+        const int blocks = std::min(kEmitBlocks, w.nchunks / 16 + 1);
+        hipLaunchKernelGGL(mc_unit_emit_kernel, dim3(blocks), dim3(64 * kUnitWaves), 0, s, w, sc.signs, sc.toff,
+                           sc.tsums, static_cast<const unsigned long long*>(sc.units), sc.nunits, verts, tris,
+                           (long long)capacity);
+        RECON_HIP_TRY(hipGetLastError(), "mc_unit_emit_kernel launch");
     }
-    long long host_total = 0;
-    RECON_HIP_TRY(hipMemcpyAsync(&host_total, tile_off + L.tiles, sizeof(long long),
-                                 hipMemcpyDeviceToHost, s),
-                  "marching cubes total");
-    RECON_HIP_TRY(hipStreamSynchronize(s), "marching cubes synchronize");
-    *total = host_total;
-    return RECON_OK;
+    return read_total(sc.total + 1, total, s);
 }
 
 }  // namespace recon

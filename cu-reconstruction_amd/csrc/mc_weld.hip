@@ -16,10 +16,10 @@
 //   base[chunk] + popc of the three masks below the voxel's lane
 //               + the voxel's own set bits of the axes before `axis`,
 // which the vertex writer and the triangle writer both evaluate: 16 B of
-// signs and counts per 64 voxels.  The field is read whole once, by
-// weld_sign_kernel; weld_count_kernel counts vertices and triangles from the
-// signs, and after a scan of its block sums weld_write_kernel classifies the
-// cubes from the signs again and reads the field at the vertices.
+// signs and counts per 64 voxels.  The field is read whole once, by the sign
+// pass (mc_signs.hip); after the counts and their scan weld_write_kernel
+// classifies the cubes from the signs again and reads the field at the
+// vertices.
 //
 // Vertex: from the negative end N to the other end M, r = (-dN)/(dM - dN),
 // p = sN + r*(sM - sN) per component.  This is the soup's own formula
@@ -31,298 +31,12 @@
 // normalised; (0,0,0) where the gradient vanishes.
 #pragma clang fp contract(off)
 
-#include "mc_device.hpp"
+#include "mc_signs.hpp"
 
 #include <algorithm>
 #include <cmath>
 
 namespace recon {
-
-// A group is 16 consecutive chunks (of one voxel row or several): the unit of
-// a wavefront in the count and write passes, lane 4i + q holding voxels and
-// cubes 16q .. 16q+15 of chunk i.  kBlockGroups groups are a workgroup of the
-// count pass; a chunk's first vertex is its block's plus its place in it.
-constexpr int kGroupChunks = 16;
-constexpr int kBlockGroups = 16, kBlockChunks = kBlockGroups * kGroupChunks;
-// A unit of the write pass is up to kUnitRounds rounds of 64 elements of a
-// group: its vertices first, then its triangles (<= 48 + 80 rounds, so <= 32
-// units).  The list holds group << kUnitBits | unit (group < 2^31 / 16).
-constexpr int kUnitRounds = 4, kUnitBits = 5;
-static_assert((16 * 64 * 3 + 16 * 64 * 5) / 64 <= kUnitRounds << kUnitBits, "a group's units fit the bits");
-constexpr int kSignChunks = 8;  // chunks per wavefront of the sign pass
-constexpr int kWeldWaves = 4;   // wavefronts per workgroup of the other passes
-
-struct WeldParams {
-    McParams mc;
-    int32_t cpr;      // 64-voxel chunks per x-row
-    int32_t nchunks;  // cpr * gy * gz
-    uint32_t mul_cpr, mul_gy;  // div31's of cpr and gy
-    int32_t sh_cpr, sh_gy;
-};
-
-// n / d for n < 2^31: ceil(2^(31 + l) / d), l = ceil(log2 d), errs by less
-// than 2^-31 of n / d, too little to reach the next whole number.
-static void div31_make(uint32_t d, uint32_t& mul, int32_t& sh) {
-    int l = 0;
-    while ((1ull << l) < d) ++l;
-    mul = (uint32_t)((((1ull << 31) << l) + d - 1) / d);
-    sh = l;
-}
-__device__ __forceinline__ uint32_t div31(uint32_t n, uint32_t mul, int32_t sh) {
-    return (uint32_t)(((uint64_t)n * mul) >> 31) >> sh;
-}
-
-// Bits 0 .. n-1 (none for n <= 0, all for n >= 64).
-__device__ __forceinline__ unsigned long long low_bits(int n) {
-    return n <= 0 ? 0ull : (n >= 64 ? ~0ull : (1ull << n) - 1ull);
-}
-
-// Masks of the sign-changing x, y, z edges owned by the voxels of chunk j of
-// row (y, z), from its signs s and those after it (sn: the next chunk's), in
-// the next row (sy) and in the next layer (sz); a neighbour past the grid may
-// hold anything.
-__device__ __forceinline__ void weld_edges(const McParams& p, int j, int y, int z, unsigned long long s,
-                                           unsigned long long sn, unsigned long long sy,
-                                           unsigned long long sz, unsigned long long m[3]) {
-    const unsigned long long in = low_bits(p.gx - 64 * j);
-    m[0] = (s ^ ((s >> 1) | (sn << 63))) & low_bits(p.gx - 1 - 64 * j);
-    m[1] = y + 1 < p.gy ? (s ^ sy) & in : 0ull;
-    m[2] = z + 1 < p.gz ? (s ^ sz) & in : 0ull;
-}
-
-// Signs of every chunk: eight chunks a wavefront, one 4-byte load a lane and
-// chunk, all in flight together.  It is the one pass over the whole field:
-// 250 x 333 x 287 voxels in 18 us, 5.3 TB/s.  A count kernel that read the
-// field itself took ten loads per four voxel rows (each row two and a half
-// times) and was bound by their addresses: 41 us, against 32 for this kernel
-// and the count of the signs.
-__global__ __launch_bounds__(256) void weld_sign_kernel(const WeldParams w,
-                                                        unsigned long long* __restrict__ signs,
-                                                        uint32_t* __restrict__ nunits) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nunits = 0;  // for the count kernel
-    const McParams& p = w.mc;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t c0 = kSignChunks * (blockIdx.x * kWeldWaves + (uint32_t)wave);
-    if (c0 >= (uint32_t)w.nchunks) return;
-    // lane k (of every eight): chunk c0 + k (the last one past the end), its
-    // first voxel and the voxels after that in its row
-    const uint32_t cl = min(c0 + (uint32_t)(lane & 7), (uint32_t)w.nchunks - 1u);
-    const uint32_t row = div31(cl, w.mul_cpr, w.sh_cpr), j = cl - row * (uint32_t)w.cpr;
-    const unsigned long long start = (unsigned long long)row * (uint32_t)p.gx + 64ull * j;
-    const int lo = (int)(uint32_t)start, hi = (int)(uint32_t)(start >> 32), last = p.gx - 1 - 64 * (int)j;
-    float v[kSignChunks];
-#pragma unroll
-    for (int k = 0; k < kSignChunks; ++k) {
-        const unsigned long long s = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32) |
-                                     (uint32_t)__builtin_amdgcn_readlane(lo, k);
-        const float* base = p.f + s;
-        v[k] = base[(uint32_t)min(lane, __builtin_amdgcn_readlane(last, k))];
-    }
-    unsigned long long out = 0;
-#pragma unroll
-    for (int k = 0; k < kSignChunks; ++k) {
-        const unsigned long long b = __ballot(v[k] < 0.0f);
-        out = lane == k ? b : out;
-    }
-    if (lane < kSignChunks && c0 + lane < (uint32_t)w.nchunks) signs[c0 + lane] = out;
-}
-
-// Chunk c's place: chunk j of voxel row (y, z).
-struct ChunkPlace {
-    int j, y, z;
-};
-__device__ __forceinline__ ChunkPlace chunk_place(const WeldParams& w, uint32_t c) {
-    const uint32_t row = div31(c, w.mul_cpr, w.sh_cpr), z = div31(row, w.mul_gy, w.sh_gy);
-    return {(int)(c - row * (uint32_t)w.cpr), (int)(row - z * (uint32_t)w.mc.gy), (int)z};
-}
-
-// Triangle counts of 16 cubes of a chunk from voxel x on, 4 bits each, from
-// the signs q of their rows (y,z), (y,z+1), (y+1,z), (y+1,z+1), 17 voxels
-// each; `in`: the cubes' rows are in the grid.  A cube's byte holds the rows'
-// bits in this order (corner order 0, 1, 3, 2, 4, 5, 7, 6).
-struct CubeCounts {
-    uint32_t w[2];
-};
-__device__ __forceinline__ uint32_t cube_byte(const uint32_t q[4], int j) {
-    return ((q[0] >> j) & 3u) | (((q[1] >> j) & 3u) << 2) | (((q[2] >> j) & 3u) << 4) |
-           (((q[3] >> j) & 3u) << 6);
-}
-__device__ __forceinline__ CubeCounts cube_counts(const McParams& p, const uint8_t* ntab,
-                                                  const uint32_t q[4], bool in, int x) {
-    CubeCounts n = {{0u, 0u}};
-#pragma unroll
-    for (int j = 0; j < 16; ++j) n.w[j >> 3] |= (uint32_t)ntab[cube_byte(q, j)] << (4 * (j & 7));
-    const int left = in ? min(max(p.gx - 1 - x, 0), 16) : 0;
-    const unsigned long long keep = low_bits(4 * left);
-    n.w[0] &= (uint32_t)keep;
-    n.w[1] &= (uint32_t)(keep >> 32);
-    return n;
-}
-// Sum of the low 8, 4 or 2 of the 4-bit counts in w.
-__device__ __forceinline__ int sum8(uint32_t w) {
-    const uint32_t b = (w & 0x0F0F0F0Fu) + ((w >> 4) & 0x0F0F0F0Fu);
-    return (int)((b * 0x01010101u) >> 24);
-}
-
-// Counts: one wavefront a group.  Lane 16 rr + i reads the signs of chunk i
-// in row (y + (rr >> 1), z + (rr & 1)); the edges follow from the words, the
-// triangles from the table, 16 cubes a lane, where any cube of the group has
-// both signs.  A workgroup appends its groups' units of work to the write
-// pass's list, in any order between workgroups (what a unit writes and where
-// does not depend on it).  14 us for 24 000 groups, two thirds of them without
-// a negative value: latency, of the loads and of the workgroup's two steps.
-__global__ __launch_bounds__(64 * kBlockGroups) void weld_count_kernel(
-    const WeldParams w, const unsigned long long* __restrict__ signs, int32_t* __restrict__ voff,
-    int32_t* __restrict__ toff, int2* __restrict__ group, long long* __restrict__ vsums,
-    long long* __restrict__ tsums, bool want_v, bool want_t, uint32_t* __restrict__ units,
-    uint32_t* __restrict__ nunits) {
-    __shared__ uint8_t ntab[256];
-    __shared__ unsigned long long sl[kBlockGroups][64];
-    __shared__ uint8_t nl[kBlockGroups][64];
-    __shared__ int vc[kBlockChunks], tc[kBlockChunks];
-    __shared__ int wv[kBlockChunks / 64], wt[kBlockChunks / 64], gu[kBlockGroups];
-    const McParams& p = w.mc;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t nchunks = (uint32_t)w.nchunks;
-    const uint32_t c0 = kGroupChunks * (blockIdx.x * kBlockGroups + (uint32_t)wave);
-    const int rr = lane >> 4;
-    const uint32_t c = c0 + (lane & 15);
-    const ChunkPlace at = chunk_place(w, c < nchunks ? c : nchunks - 1u);
-    const bool here = (c < nchunks) & (at.y + (rr >> 1) < p.gy) & (at.z + (rr & 1) < p.gz);
-    const size_t cc = (size_t)c + (rr >> 1 ? (size_t)w.cpr : 0) + (rr & 1 ? (size_t)w.cpr * p.gy : 0);
-    unsigned long long s = 0, sn = 0;
-    if (here) {
-        s = signs[cc];
-        if (at.j + 1 < w.cpr) sn = signs[cc + 1];
-    }
-    if (threadIdx.x < 256) ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
-    __syncthreads();
-    int nv = 0;
-    bool mixed = false;
-    if (__ballot((s | sn) != 0ull)) {  // any negative value in reach
-        const unsigned long long sz = __shfl_down(s, 16, 64), sy = __shfl_down(s, 32, 64);
-        if (rr == 0 && here) {
-            unsigned long long m[3];
-            weld_edges(p, at.j, at.y, at.z, s, sn, sy, sz, m);
-            nv = __popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]);
-        }
-        // a cube has both signs where the eight words' AND and OR differ
-        const unsigned long long sx = (s >> 1) | (sn << 63);
-        unsigned long long all = s & sx, any = s | sx;
-        all &= __shfl_xor(all, 16, 64);
-        any |= __shfl_xor(any, 16, 64);
-        all &= __shfl_xor(all, 32, 64);
-        any |= __shfl_xor(any, 32, 64);
-        const bool cubes = (c < nchunks) & (at.y + 1 < p.gy) & (at.z + 1 < p.gz);
-        mixed = cubes & (((any & ~all) & low_bits(p.gx - 1 - 64 * at.j)) != 0);
-    }
-    if (rr == 0) vc[kGroupChunks * wave + lane] = nv;
-    const int nvg = __builtin_amdgcn_readlane(wave_inclusive_scan(nv, lane), 63);
-    int ntg = 0;
-    if (__ballot(mixed)) {
-        sl[wave][lane] = s;
-        nl[wave][lane] = (uint8_t)(sn & 1ull);
-        __builtin_amdgcn_wave_barrier();
-        const int i = lane >> 2, b = 16 * (lane & 3);
-        const ChunkPlace mine = chunk_place(w, min(c0 + (uint32_t)i, nchunks - 1u));
-        uint32_t q[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            q[k] = (uint32_t)(sl[wave][16 * k + i] >> b);
-            if (b == 48) q[k] |= (uint32_t)nl[wave][16 * k + i] << 16;
-        }
-        const bool in = (c0 + (uint32_t)i < nchunks) & (mine.y + 1 < p.gy) & (mine.z + 1 < p.gz);
-        const CubeCounts n = cube_counts(p, ntab, q, in, 64 * mine.j + b);
-        const int incl = wave_inclusive_scan(sum8(n.w[0]) + sum8(n.w[1]), lane);
-        ntg = __builtin_amdgcn_readlane(incl, 63);
-        const int before = __shfl(incl, 4 * (lane & 15) - 1, 64);  // lanes 0..15: chunk lane's
-        const int upto = __shfl(incl, 4 * (lane & 15) + 3, 64);
-        if (lane < 16) tc[kGroupChunks * wave + lane] = upto - (lane ? before : 0);
-    } else if (lane < 16) {
-        tc[kGroupChunks * wave + lane] = 0;
-    }
-    if (lane == 0) {
-        const int rounds = (want_v ? (nvg + 63) / 64 : 0) + (want_t ? (ntg + 63) / 64 : 0);
-        gu[wave] = (rounds + kUnitRounds - 1) / kUnitRounds;
-        if (c0 < nchunks) group[c0 / kGroupChunks] = make_int2(nvg, ntg);
-    }
-    __syncthreads();
-    if (wave == kBlockGroups - 1) {
-        const int mine = lane < kBlockGroups ? gu[lane] : 0;
-        const int incl = wave_inclusive_scan(mine, lane);
-        const int all_units = __builtin_amdgcn_readlane(incl, 63);
-        if (all_units) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(nunits, (uint32_t)all_units);
-            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + (uint32_t)(incl - mine);
-            const uint32_t g = kBlockGroups * blockIdx.x + (uint32_t)lane;
-            for (int k = 0; k < mine; ++k) units[base + k] = (g << kUnitBits) | (uint32_t)k;
-        }
-    }
-    const bool scan = wave < kBlockChunks / 64;
-    int v = 0, t = 0, iv = 0, it = 0;
-    if (scan) {
-        v = vc[threadIdx.x];
-        t = tc[threadIdx.x];
-        iv = wave_inclusive_scan(v, lane);
-        it = wave_inclusive_scan(t, lane);
-        if (lane == 63) {
-            wv[wave] = iv;
-            wt[wave] = it;
-        }
-    }
-    __syncthreads();
-    if (scan) {
-        int bv = 0, bt = 0, av = 0, at_ = 0;
-#pragma unroll
-        for (int k = 0; k < kBlockChunks / 64; ++k) {
-            bv += k < wave ? wv[k] : 0;
-            bt += k < wave ? wt[k] : 0;
-            av += wv[k];
-            at_ += wt[k];
-        }
-        const uint32_t ct = kBlockChunks * blockIdx.x + threadIdx.x;
-        if (ct < nchunks) {
-            voff[ct] = bv + iv - v;
-            toff[ct] = bt + it - t;
-        }
-        if (threadIdx.x == 0) {
-            vsums[blockIdx.x] = av;
-            tsums[blockIdx.x] = at_;
-        }
-    }
-}
-
-// Block sums to first indices in place, the totals to total[0] (vertices) and
-// total[1] (triangles): a workgroup an array.
-__global__ __launch_bounds__(256) void weld_scan_kernel(long long* __restrict__ vsums,
-                                                        long long* __restrict__ tsums, int nb,
-                                                        long long* __restrict__ total) {
-    constexpr int kItems = 8;
-    __shared__ long long sh[4];
-    long long* __restrict__ sums = blockIdx.x ? tsums : vsums;
-    long long carry = 0;
-    for (int base = 0; base < nb; base += 256 * kItems) {
-        const int i0 = base + (int)threadIdx.x * kItems;
-        long long v[kItems], s = 0;
-#pragma unroll
-        for (int k = 0; k < kItems; ++k) {
-            v[k] = i0 + k < nb ? sums[i0 + k] : 0;
-            s += v[k];
-        }
-        long long all;
-        long long e = carry + block_exclusive_scan(s, sh, &all);
-#pragma unroll
-        for (int k = 0; k < kItems; ++k) {
-            if (i0 + k < nb) sums[i0 + k] = e;
-            e += v[k];
-        }
-        carry += all;
-    }
-    if (threadIdx.x == 0) total[blockIdx.x] = carry;
-}
 
 // Gradient component `a` of the field at voxel (x, y, z).
 __device__ __forceinline__ float weld_grad(const McParams& p, int x, int y, int z, int a) {
@@ -337,7 +51,7 @@ __device__ __forceinline__ float weld_grad(const McParams& p, int x, int y, int 
 
 // Vertex (and normal) `idx` on the edge from voxel (x, y, z) along axis a, by
 // the divisions.
-__device__ __forceinline__ void weld_vertex_exact(const WeldParams& w, int x, int y, int z, int a,
+__device__ __forceinline__ void weld_vertex_exact(const SignParams& w, int x, int y, int z, int a,
                                                   long long idx, float* __restrict__ verts,
                                                   float* __restrict__ normals) {
     const McParams& p = w.mc;
@@ -383,15 +97,7 @@ __device__ __forceinline__ void weld_vertex_exact(const WeldParams& w, int x, in
     }
 }
 
-// num / den by y = RN(1/den) and div_by_rcp; `bad` is set where that might not
-// be the division's bits (a quotient near the denormals or out of range, -0).
-__device__ __forceinline__ float weld_quotient(float num, float den, float y, bool& bad) {
-    const float an = fabsf(num);
-    bad |= !((an >= 1e-30f) & (an <= 1e30f)) & (__float_as_uint(num) != 0u);
-    return div_by_rcp(num, den, y);
-}
-
-// 1/vs and 1/(vs + vs) per axis, and whether weld_quotient covers them.
+// 1/vs and 1/(vs + vs) per axis, and whether short_quotient covers them.
 struct WeldSteps {
     float r1[3], r2[3];
     bool ok;
@@ -399,7 +105,7 @@ struct WeldSteps {
 
 // Every lane with `on` writes vertex (and normal) `idx` of edge (x, y, z, a):
 // weld_vertex_exact's bits.
-__device__ __forceinline__ void weld_vertex(const WeldParams& w, const WeldSteps& st, bool on, int x, int y,
+__device__ __forceinline__ void weld_vertex(const SignParams& w, const WeldSteps& st, bool on, int x, int y,
                                             int z, int a, long long idx, float* __restrict__ verts,
                                             float* __restrict__ normals) {
     const McParams& p = w.mc;
@@ -417,7 +123,7 @@ __device__ __forceinline__ void weld_vertex(const WeldParams& w, const WeldSteps
         float res = 0.0f;
         const float y_den = recip_sum(den, res);
         bad |= !(res < kRecipBad) | !(fabsf(den) <= 1e7f);
-        const float r = weld_quotient(-dn, den, y_den, bad);
+        const float r = short_quotient(-dn, den, y_den, bad);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const float s0 = voxel_centre(c[k], p.vs[k], p.off[k]);
@@ -440,7 +146,7 @@ __device__ __forceinline__ void weld_vertex(const WeldParams& w, const WeldSteps
                     const bool lo = ck > 0, hi = ck < g[k] - 1;
                     const float num = p.f[hi ? iq + sx[k] : iq] - p.f[lo ? iq - sx[k] : iq];
                     const bool both = lo & hi;
-                    ge[q] = weld_quotient(num, both ? p.vs[k] + p.vs[k] : p.vs[k],
+                    ge[q] = short_quotient(num, both ? p.vs[k] + p.vs[k] : p.vs[k],
                                           both ? st.r2[k] : st.r1[k], bad);
                 }
                 const float gn = first ? ge[0] : ge[1], gm = first ? ge[1] : ge[0];
@@ -455,7 +161,7 @@ __device__ __forceinline__ void weld_vertex(const WeldParams& w, const WeldSteps
                 float rl = 0.0f;
                 const float y_len = recip_sum(len, rl);
 #pragma unroll
-                for (int k = 0; k < 3; ++k) nrm[k] = weld_quotient(gr[k], len, y_len, bad);
+                for (int k = 0; k < 3; ++k) nrm[k] = short_quotient(gr[k], len, y_len, bad);
             } else {
                 bad |= !(len2 == 0.0f);
             }
@@ -487,20 +193,6 @@ struct WeldGroup {
     int mark[64];
 };
 
-// The lane whose elements include element k0 + lane of the lanes' elements
-// (first element excl, count n per lane; k0 below their total): marks at the
-// first elements, a max-scan, and the lane that element k0 is in before the
-// first mark.  Every lane calls.
-__device__ __forceinline__ int weld_owner(int* mark, int excl, int n, int k0, int lane) {
-    mark[lane] = 0;
-    if (n > 0 && excl >= k0 && excl < k0 + 64) mark[excl - k0] = lane + 1;
-    __builtin_amdgcn_wave_barrier();
-    const int mx = wave_inclusive_max(mark[lane]);
-    const int first = 63 - __builtin_clzll(__ballot(n > 0 && excl <= k0) | 1ull);
-    __builtin_amdgcn_wave_barrier();
-    return mx > 0 ? mx - 1 : first;
-}
-
 // Vertex index of the local edge of table word et (axis, lower end's dx, dy,
 // dz) of the cube at voxel place xl of the group's chunks.
 __device__ __forceinline__ int32_t weld_index(const WeldGroup& nb, int xl, unsigned et) {
@@ -515,7 +207,7 @@ __device__ __forceinline__ int32_t weld_index(const WeldGroup& nb, int xl, unsig
 }
 
 // Entry of chunk c (place at; of the grid) in row rr of the neighbourhood.
-__device__ __forceinline__ void weld_entry_load(const WeldParams& w, uint32_t c, const ChunkPlace& at, int rr,
+__device__ __forceinline__ void weld_entry_load(const SignParams& w, uint32_t c, const ChunkPlace& at, int rr,
                                                 const unsigned long long* __restrict__ signs,
                                                 const int32_t* __restrict__ voff,
                                                 const long long* __restrict__ vsums, bool in,
@@ -530,7 +222,7 @@ __device__ __forceinline__ void weld_entry_load(const WeldParams& w, uint32_t c,
         const unsigned long long sn = at.j + 1 < w.cpr ? signs[cc + 1] : 0ull;
         const unsigned long long sy = Y + 1 < p.gy ? signs[cc + w.cpr] : 0ull;
         const unsigned long long sz = Z + 1 < p.gz ? signs[cc + (size_t)w.cpr * p.gy] : 0ull;
-        weld_edges(p, at.j, Y, Z, s, sn, sy, sz, m);
+        sign_edges(p, at.j, Y, Z, s, sn, sy, sz, m);
         base = (uint32_t)vsums[cc / kBlockChunks] + (uint32_t)voff[cc];
     }
     nb.s[entry] = s;
@@ -543,7 +235,7 @@ __device__ __forceinline__ void weld_entry_load(const WeldParams& w, uint32_t c,
 // Elements [first, first + 64 kUnitRounds) of the group of chunks from c0 on:
 // its nv vertices rounded up to whole rounds, then its nt triangles.
 __device__ __forceinline__ void weld_write_unit(
-    const WeldParams& w, const WeldSteps& st, uint32_t c0, int lane, int first, int nv, int nt,
+    const SignParams& w, const WeldSteps& st, uint32_t c0, int lane, int first, int nv, int nt,
     const unsigned long long* __restrict__ signs, const int32_t* __restrict__ voff,
     const int32_t* __restrict__ toff, const long long* __restrict__ vsums,
     const long long* __restrict__ tsums, WeldGroup& nb, const uint64_t* tri, const uint8_t* ntab,
@@ -582,7 +274,7 @@ __device__ __forceinline__ void weld_write_unit(
         const int excl = wave_inclusive_scan(mine, lane) - mine;
         const long long v0 = (long long)nb.base[0];
         for (int k0 = first; k0 < min(end, nv); k0 += 64) {
-            const int owner = weld_owner(nb.mark, excl, mine, k0, lane);
+            const int owner = unit_owner(nb.mark, excl, mine, k0, lane);
             uint32_t o01 = (uint32_t)__shfl((int)own01, owner, 64), o2 = (uint32_t)__shfl((int)own2, owner, 64);
             int r = k0 + lane - __shfl(excl, owner, 64), v = 0;
             // edge r of the 16 voxels', in the order voxel, axis: halve the
@@ -619,27 +311,13 @@ __device__ __forceinline__ void weld_write_unit(
     const int excl = wave_inclusive_scan(mine, lane) - mine;
     const long long t0 = tsums[c0 / kBlockChunks] + toff[c0];
     for (int k0 = max(first - nv64, 0); k0 < min(end - nv64, nt); k0 += 64) {
-        const int owner = weld_owner(nb.mark, excl, mine, k0, lane);
-        const uint32_t w0 = (uint32_t)__shfl((int)cn4.w[0], owner, 64);
-        const uint32_t w1 = (uint32_t)__shfl((int)cn4.w[1], owner, 64);
+        const int owner = unit_owner(nb.mark, excl, mine, k0, lane);
+        int r = k0 + lane - __shfl(excl, owner, 64);
+        const int j = cube_of((uint32_t)__shfl((int)cn4.w[0], owner, 64),
+                              (uint32_t)__shfl((int)cn4.w[1], owner, 64), r);
         uint32_t oq[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) oq[k] = (uint32_t)__shfl((int)q[k], owner, 64);
-        int r = k0 + lane - __shfl(excl, owner, 64);
-        // triangle r of the 16 cubes': halve the cubes
-        int j = 0;
-        const int c8 = sum8(w0);
-        uint32_t left = r >= c8 ? w1 : w0;
-        j += r >= c8 ? 8 : 0;
-        r -= r >= c8 ? c8 : 0;
-#pragma unroll
-        for (int h = 4; h >= 1; h >>= 1) {
-            const int c = sum8(left & ((1u << (4 * h)) - 1u));
-            const bool up = r >= c;
-            r -= up ? c : 0;
-            j += up ? h : 0;
-            left >>= up ? 4 * h : 0;
-        }
         if (k0 + lane < nt) {
             const uint64_t word = tri[cube_byte(oq, j)] >> (4 + 12 * r);
             const long long t = t0 + k0 + lane;
@@ -660,14 +338,14 @@ __device__ __forceinline__ void weld_write_unit(
 // of four chunks 59; a group a wavefront 52; units 34.
 // Nothing is written when the totals (from the scan) exceed int32 indices or
 // a requested output's capacity: the host reports that after the call.
-constexpr int kWriteBlocks = 256 * 8;  // 8 workgroups a CU by registers
-__global__ __launch_bounds__(64 * kWeldWaves) void weld_write_kernel(
-    const WeldParams w, const unsigned long long* __restrict__ signs, const int32_t* __restrict__ voff,
+constexpr int kWriteBlocks = 256 * 5;  // 5 workgroups a CU by registers (bound to 80 for 6: 4 % slower)
+__global__ __launch_bounds__(64 * kUnitWaves) void weld_write_kernel(
+    const SignParams w, const unsigned long long* __restrict__ signs, const int32_t* __restrict__ voff,
     const int32_t* __restrict__ toff, const int2* __restrict__ group, const long long* __restrict__ vsums,
     const long long* __restrict__ tsums, const long long* __restrict__ total,
     const uint32_t* __restrict__ units, const uint32_t* __restrict__ nunits, long long vcap,
     long long tcap, float* __restrict__ verts, float* __restrict__ normals, int32_t* __restrict__ tris) {
-    __shared__ WeldGroup groups[kWeldWaves];
+    __shared__ WeldGroup groups[kUnitWaves];
     __shared__ uint64_t tri[256];    // triangle table by the signs' byte
     __shared__ uint8_t ntab[256];    // its triangle counts
     __shared__ uint32_t edges[16];   // axis | dx << 2 | (2 dy + dz) << 3 of an edge's lower end
@@ -677,7 +355,7 @@ __global__ __launch_bounds__(64 * kWeldWaves) void weld_write_kernel(
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t nu = *nunits;
     const long long nvt = total[0], ntt = total[1];
-    if (kWeldWaves * blockIdx.x >= nu || nvt > INT32_MAX || (want_v && nvt > vcap) || (want_t && ntt > tcap))
+    if (kUnitWaves * blockIdx.x >= nu || nvt > INT32_MAX || (want_v && nvt > vcap) || (want_t && ntt > tcap))
         return;
     tri[threadIdx.x] = c_tri[qbyte_class((int)threadIdx.x)];
     ntab[threadIdx.x] = mc_ntab_qbyte((int)threadIdx.x);
@@ -702,7 +380,7 @@ __global__ __launch_bounds__(64 * kWeldWaves) void weld_write_kernel(
         st.r2[k] = recip_sum(p.vs[k] + p.vs[k], bad);
         st.ok = st.ok && bad < kRecipBad && p.vs[k] >= 1e-6f && p.vs[k] <= 1e6f;
     }
-    for (uint32_t u = kWeldWaves * blockIdx.x + (uint32_t)wave; u < nu; u += kWeldWaves * gridDim.x) {
+    for (uint32_t u = kUnitWaves * blockIdx.x + (uint32_t)wave; u < nu; u += kUnitWaves * gridDim.x) {
         const uint32_t unit = (uint32_t)__builtin_amdgcn_readfirstlane((int)units[u]);
         const uint32_t g = unit >> kUnitBits;
         const int2 n = group[g];
@@ -714,8 +392,6 @@ __global__ __launch_bounds__(64 * kWeldWaves) void weld_write_kernel(
     }
 }
 
-static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-
 // Counts (always), then writes what is asked for when it fits.
 static int weld_run(const float* field, const int32_t grid[3], const float vs[3], const float off[3],
                     float* verts, float* normals, int64_t vcap, int32_t* tris, int64_t tcap,
@@ -724,34 +400,9 @@ static int weld_run(const float* field, const int32_t grid[3], const float vs[3]
     *nv_out = 0;
     *nt_out = 0;
     if (grid[0] < 2 || grid[1] < 2 || grid[2] < 2) return RECON_OK;
-    WeldParams w;
-    McParams& p = w.mc;
-    p.f = field;
-    p.gx = grid[0];
-    p.gy = grid[1];
-    p.gz = grid[2];
-    p.cx = grid[0] - 1;
-    p.cyr = grid[1] - 1;
-    p.rows = (grid[1] - 1) * (grid[2] - 1);
-    for (int i = 0; i < 3; ++i) {
-        p.vs[i] = vs[i];
-        p.off[i] = off[i];
-    }
-    w.cpr = (grid[0] + 63) / 64;
-    w.nchunks = w.cpr * grid[1] * grid[2];
-    div31_make((uint32_t)w.cpr, w.mul_cpr, w.sh_cpr);
-    div31_make((uint32_t)grid[1], w.mul_gy, w.sh_gy);
-    const int nb = (w.nchunks + kBlockChunks - 1) / kBlockChunks;
-    const size_t o_signs = 0;
-    const size_t o_voff = o_signs + align256(8 * (size_t)w.nchunks);
-    const size_t o_toff = o_voff + align256(4 * (size_t)w.nchunks);
-    const size_t o_group = o_toff + align256(4 * (size_t)w.nchunks);
-    const size_t o_vsums = o_group + align256(8 * (size_t)nb * kBlockGroups);
-    const size_t o_tsums = o_vsums + align256(8 * (size_t)nb);
-    const size_t o_total = o_tsums + align256(8 * (size_t)nb);
-    const size_t o_nunits = o_total + 256;
-    const size_t o_units = o_nunits + 256;
-    const size_t need = o_units + align256((sizeof(uint32_t) << kUnitBits) * nb * kBlockGroups);
+    SignParams w;
+    SignScratch sc;
+    const size_t need = sign_layout(field, grid, vs, off, true, nullptr, w, sc);
     if (*scratch_bytes < need) {
         if (*scratch) (void)hipFree(*scratch);
         *scratch = nullptr;
@@ -759,39 +410,23 @@ static int weld_run(const float* field, const int32_t grid[3], const float vs[3]
         RECON_HIP_TRY(hipMalloc(scratch, need), "welded marching cubes scratch");
         *scratch_bytes = need;
     }
-    char* sb = static_cast<char*>(*scratch);
-    auto* signs = reinterpret_cast<unsigned long long*>(sb + o_signs);
-    auto* voff = reinterpret_cast<int32_t*>(sb + o_voff);
-    auto* toff = reinterpret_cast<int32_t*>(sb + o_toff);
-    auto* group = reinterpret_cast<int2*>(sb + o_group);
-    auto* vsums = reinterpret_cast<long long*>(sb + o_vsums);
-    auto* tsums = reinterpret_cast<long long*>(sb + o_tsums);
-    auto* total = reinterpret_cast<long long*>(sb + o_total);
-    auto* nunits = reinterpret_cast<uint32_t*>(sb + o_nunits);
-    auto* units = reinterpret_cast<uint32_t*>(sb + o_units);
+    sign_layout(field, grid, vs, off, true, static_cast<char*>(*scratch), w, sc);
     const bool write = verts || normals || tris;
-    constexpr int kSignBlock = kSignChunks * kWeldWaves;
-    hipLaunchKernelGGL(weld_sign_kernel, dim3((w.nchunks + kSignBlock - 1) / kSignBlock),
-                       dim3(64 * kWeldWaves), 0, s, w, signs, nunits);
-    RECON_HIP_TRY(hipGetLastError(), "weld_sign_kernel launch");
-    hipLaunchKernelGGL(weld_count_kernel, dim3(nb), dim3(64 * kBlockGroups), 0, s, w, signs, voff, toff,
-                       group, vsums, tsums, verts || normals, tris != nullptr, units, nunits);
-    RECON_HIP_TRY(hipGetLastError(), "weld_count_kernel launch");
-    hipLaunchKernelGGL(weld_scan_kernel, dim3(2), dim3(256), 0, s, vsums, tsums, nb, total);
-    RECON_HIP_TRY(hipGetLastError(), "weld_scan_kernel launch");
+    const int rc = launch_signs(w, sc, true, verts || normals, tris != nullptr, s);
+    if (rc) return rc;
     // The write pass checks the totals on the device, so it is queued before
     // the host waits; the copy of the totals to pageable memory comes last,
     // since it returns only when the stream has reached it.
     if (write) {
         // most groups are empty and a busy one is one or two units
-        const int blocks = std::min(kWriteBlocks, nb * kBlockGroups);
-        hipLaunchKernelGGL(weld_write_kernel, dim3(blocks), dim3(64 * kWeldWaves), 0, s, w, signs, voff,
-                           toff, group, vsums, tsums, total, units, nunits, (long long)vcap,
-                           (long long)tcap, verts, normals, tris);
+        const int blocks = std::min(kWriteBlocks, w.nchunks / kGroupChunks + 1);
+        hipLaunchKernelGGL(weld_write_kernel, dim3(blocks), dim3(64 * kUnitWaves), 0, s, w, sc.signs, sc.voff,
+                           sc.toff, sc.group, sc.vsums, sc.tsums, sc.total, static_cast<const uint32_t*>(sc.units), sc.nunits,
+                           (long long)vcap, (long long)tcap, verts, normals, tris);
         RECON_HIP_TRY(hipGetLastError(), "weld_write_kernel launch");
     }
     long long totals[2] = {0, 0};
-    RECON_HIP_TRY(hipMemcpyAsync(totals, total, 16, hipMemcpyDeviceToHost, s), "totals");
+    RECON_HIP_TRY(hipMemcpyAsync(totals, sc.total, 16, hipMemcpyDeviceToHost, s), "totals");
     RECON_HIP_TRY(hipStreamSynchronize(s), "welded marching cubes");
     *nv_out = totals[0];
     *nt_out = totals[1];

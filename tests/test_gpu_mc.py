@@ -62,6 +62,24 @@ def test_random_fields(cuda, grid):
     _mc_compare(cuda, f, grid, (0.01, 0.02, 0.03), (0.1, -0.2, 0.3))
 
 
+# fields that a row crosses once (a wall), runs along (a floor) and at random:
+# units of one chunk and of 64, rows of 1, 4 and 6 chunks; values inside and
+# outside the range of the short quotients, mixed in one wavefront
+@pytest.mark.parametrize("grid", [(64, 3, 3), (65, 9, 3), (64, 40, 6), (256, 5, 4), (321, 6, 3)])
+@pytest.mark.parametrize("scale", [1.0, 1e-36, 1e30])
+def test_units_and_quotient_ranges(cuda, grid, scale):
+    rng = np.random.default_rng(sum(grid))
+    gx, gy, gz = grid
+    big = rng.random((gz, gy, gx)) < 0.3
+    noise = rng.random((gz, gy, gx), dtype=np.float32) * np.float32(0.2)
+    wall = np.arange(gx, dtype=np.float32)[None, None, :] - np.float32(gx / 3 + 0.1) + noise
+    floor = np.arange(gz, dtype=np.float32)[:, None, None] - np.float32(0.5) + noise
+    for f in (wall, floor, noise - np.float32(0.1)):
+        f = np.ascontiguousarray(f, np.float32)
+        f[big] *= np.float32(scale)
+        _mc_compare(cuda, f, grid, (0.01, 0.02, 0.03), (0.1, -0.2, 0.3))
+
+
 def test_unaligned_field_takes_4_byte_loads(cuda):
     # a field one float past a 16-byte boundary: rows of 68 voxels, but the
     # 4-byte loads; the same results as the aligned copy
