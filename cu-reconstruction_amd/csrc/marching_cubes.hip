@@ -214,7 +214,7 @@ __device__ __forceinline__ int set_bit(unsigned long long m, int r) {
 // rounds one after the other) and 1 us off this one.
 constexpr int kEmitBlocks = 256 * 7;  // 7 workgroups a CU by LDS
 __global__ __launch_bounds__(64 * kUnitWaves) void mc_unit_emit_kernel(
-    const SignParams w, const unsigned long long* __restrict__ signs, const int32_t* __restrict__ toff,
+    const SignParams w, const unsigned long long* __restrict__ signs,
     const long long* __restrict__ tsums, const unsigned long long* __restrict__ units,
     const uint32_t* __restrict__ nunits, float* __restrict__ verts, int32_t* __restrict__ tris,
     long long capacity) {
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * kUnitWaves) void mc_unit_emit_kernel(
         const unsigned long long unit = units[u];
         const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(unit >> 6));
         const int len = 1 + __builtin_amdgcn_readfirstlane((int)(unit & 63ull));
-        long long t0 = tsums[c0 / kBlockChunks] + toff[c0];
+        long long t0 = tsums[c0 / kBlockChunks] + (long long)(unit >> kSoupTriShift);
         const uint32_t c = c0 + (uint32_t)(lane < len ? lane : 0);
         const ChunkPlace at = chunk_place(w, c);
         const ChunkWords v = chunk_words(w, signs, c, at, lane < len);
@@ -639,7 +639,7 @@ int mc_run(const float* field, const int32_t grid[3], const float vs[3], const f
     if (rc) return rc;
     if (write) {
         const int blocks = std::min(kEmitBlocks, w.nchunks / 16 + 1);
-        hipLaunchKernelGGL(mc_unit_emit_kernel, dim3(blocks), dim3(64 * kUnitWaves), 0, s, w, sc.signs, sc.toff,
+        hipLaunchKernelGGL(mc_unit_emit_kernel, dim3(blocks), dim3(64 * kUnitWaves), 0, s, w, sc.signs,
                            sc.tsums, static_cast<const unsigned long long*>(sc.units), sc.nunits, verts, tris,
                            (long long)capacity);
         RECON_HIP_TRY(hipGetLastError(), "mc_unit_emit_kernel launch");

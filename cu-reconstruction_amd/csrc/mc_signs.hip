@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kBlockChunks) void sign_count_kernel(
     }
     if (in) {
         if (VERTS) voff[c] = bv + iv - nv;
-        toff[c] = bt + it - nt;
+        if (VERTS) toff[c] = bt + it - nt;
     }
     if (threadIdx.x == 0) {
         if (VERTS) vsums[blockIdx.x] = av;
@@ -170,7 +170,8 @@ __global__ __launch_bounds__(kBlockChunks) void sign_count_kernel(
     } else if (mine) {
         const unsigned long long after = lane < 63 ? starts >> (lane + 1) : 0ull;
         const int len = after ? 1 + __builtin_ctzll(after) : 64 - lane;
-        static_cast<unsigned long long*>(units)[base] = ((unsigned long long)c << 6) | (unsigned)(len - 1);
+        static_cast<unsigned long long*>(units)[base] = ((unsigned long long)(unsigned)(bt + it - nt) << kSoupTriShift) |
+                                                        ((unsigned long long)c << 6) | (unsigned)(len - 1);
     }
 }
 
@@ -233,7 +234,7 @@ size_t sign_layout(const float* field, const int32_t grid[3], const float vs[3],
     };
     sc.signs = reinterpret_cast<unsigned long long*>(take(8 * n));
     sc.voff = reinterpret_cast<int32_t*>(take(verts ? 4 * n : 0));
-    sc.toff = reinterpret_cast<int32_t*>(take(4 * n));
+    sc.toff = reinterpret_cast<int32_t*>(take(verts ? 4 * n : 0));
     sc.group = reinterpret_cast<int2*>(take(8 * ng));
     sc.vsums = reinterpret_cast<long long*>(take(verts ? 8 * nb : 0));
     sc.tsums = reinterpret_cast<long long*>(take(8 * nb));

@@ -22,8 +22,9 @@ constexpr int kGroupChunks = 16;
 constexpr int kBlockChunks = 512, kBlockGroups = kBlockChunks / kGroupChunks;
 // A unit of the soup's emit is a run of at most 64 consecutive chunks, within
 // one of the count pass's wavefronts, whose cubes with both signs number at
-// most kUnitCubes + 63; the list holds chunk << 6 | (chunks - 1).
-constexpr int kUnitCubes = 64, kWaveUnits = 64 * 64 / kUnitCubes;
+// most kUnitCubes + 63; the list holds its first triangle in its count block
+// (< 2^18) << kSoupTriShift | chunk << 6 | (chunks - 1).
+constexpr int kUnitCubes = 64, kWaveUnits = 64 * 64 / kUnitCubes, kSoupTriShift = 38;
 // A unit of the welded write pass is up to kUnitRounds rounds of 64 elements of a
 // group: its vertices first, then its triangles (<= 48 + 80 rounds, so <= 32
 // units).  The list holds group << kUnitBits | unit (group < 2^31 / 16).
@@ -193,10 +194,10 @@ __device__ __forceinline__ int unit_owner(int* mark, int excl, int n, int k0, in
     return mx > 0 ? mx - 1 : first;
 }
 
-// Scratch of the passes: signs and places of every chunk (voff only with
-// `verts`), per group its vertices and triangles, per count block its sums,
-// the totals, and the list of units.
-// (uint32 with `verts`, else 64-bit words).
+// Scratch of the passes: the signs of every chunk; with `verts` its first
+// vertex and triangle in its count block and every group's numbers of both;
+// per count block its sums, the totals, and the list of units (uint32 with
+// `verts`, else 64-bit words).
 struct SignScratch {
     unsigned long long* signs;
     int32_t *voff, *toff;
@@ -209,7 +210,7 @@ struct SignScratch {
 // bytes of its scratch, laid out from base.
 size_t sign_layout(const float* field, const int32_t grid[3], const float vs[3], const float off[3],
                    bool verts, char* base, SignParams& w, SignScratch& sc);
-// Signs, counts and scan: voff, vsums and total[0] only with `verts`; the list
+// Signs, counts and scan: vertices and total[0] only with `verts`; the list
 // holds the units of the outputs that are wanted.
 int launch_signs(const SignParams& w, const SignScratch& sc, bool verts, bool want_v, bool want_t,
                  hipStream_t s);
