@@ -388,9 +388,9 @@ __global__ __launch_bounds__(256) void mc_class_hist_kernel(const McParams p,
     if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)h[threadIdx.x]);
 }
 
-__global__ __launch_bounds__(256) void scan_block_sums_kernel(const ScanJobs j, int n) {
+__global__ __launch_bounds__(256) void scan_block_sums_kernel(const int32_t* __restrict__ in, int n,
+                                                              long long* __restrict__ sums) {
     __shared__ long long sh[256];
-    const int32_t* __restrict__ in = blockIdx.y ? j.in[1] : j.in[0];
     const int b0 = blockIdx.x * kScanBlock + threadIdx.x * kScanItems;
     long long s = 0;
     if (b0 + kScanItems <= n && (reinterpret_cast<uintptr_t>(in) & 15) == 0) {
@@ -403,16 +403,14 @@ __global__ __launch_bounds__(256) void scan_block_sums_kernel(const ScanJobs j, 
     }
     long long total;
     block_exclusive_scan(s, sh, &total);
-    if (threadIdx.x == 0) (blockIdx.y ? j.sums[1] : j.sums[0])[blockIdx.x] = total;
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// One workgroup per array: exclusive scan of its block sums in place, total
-// at [nb]; each thread takes kTopItems consecutive sums per pass, so up to
+// One workgroup: exclusive scan of the block sums in place, total at [nb]; each thread takes kTopItems consecutive sums per pass, so up to
 // 256 * kTopItems sums need one workgroup scan.
 constexpr int kTopItems = 8;
-__global__ __launch_bounds__(256) void scan_top_kernel(const ScanJobs j, int nb) {
+__global__ __launch_bounds__(256) void scan_top_kernel(long long* __restrict__ sums, int nb) {
     __shared__ long long sh[256];
-    long long* __restrict__ sums = blockIdx.y ? j.sums[1] : j.sums[0];
     long long carry = 0;
     for (int base = 0; base < nb; base += 256 * kTopItems) {
         const int i0 = base + threadIdx.x * kTopItems;
@@ -434,10 +432,10 @@ __global__ __launch_bounds__(256) void scan_top_kernel(const ScanJobs j, int nb)
     if (threadIdx.x == 0) sums[nb] = carry;
 }
 
-__global__ __launch_bounds__(256) void scan_apply_kernel(const ScanJobs j, int n) {
+__global__ __launch_bounds__(256) void scan_apply_kernel(const int32_t* __restrict__ in, int n,
+                                                         const long long* __restrict__ sums,
+                                                         long long* __restrict__ out) {
     __shared__ long long sh[256];
-    const int32_t* __restrict__ in = blockIdx.y ? j.in[1] : j.in[0];
-    long long* __restrict__ out = blockIdx.y ? j.out[1] : j.out[0];
     const int b0 = blockIdx.x * kScanBlock + threadIdx.x * kScanItems;
     const bool vec = b0 + kScanItems <= n && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(out) & 15) == 0;
@@ -451,8 +449,7 @@ __global__ __launch_bounds__(256) void scan_apply_kernel(const ScanJobs j, int n
     }
     const long long s = (vals[0] + vals[1]) + (vals[2] + vals[3]);
     long long total;
-    const long long e0 =
-        block_exclusive_scan(s, sh, &total) + (blockIdx.y ? j.sums[1] : j.sums[0])[blockIdx.x];
+    const long long e0 = block_exclusive_scan(s, sh, &total) + sums[blockIdx.x];
     const long long e1 = e0 + vals[0], e2 = e1 + vals[1], e3 = e2 + vals[2];
     if (vec) {
         longlong2* o2 = reinterpret_cast<longlong2*>(out + b0);
@@ -466,29 +463,18 @@ __global__ __launch_bounds__(256) void scan_apply_kernel(const ScanJobs j, int n
     }
 }
 
-int launch_exclusive_scans(const ScanJobs& j, int count, int n, hipStream_t s) {
-    if (count < 1 || count > 2) return fail(RECON_ERR_SIZE, "launch_exclusive_scans: %d arrays", count);
+int launch_exclusive_scan(const int32_t* counts, int n, long long* offsets, long long* sums,
+                          hipStream_t s) {
     const int nb = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(scan_block_sums_kernel, dim3(nb, count), dim3(256), 0, s, j, n);
+    hipLaunchKernelGGL(scan_block_sums_kernel, dim3(nb), dim3(256), 0, s, counts, n, sums);
     RECON_HIP_TRY(hipGetLastError(), "scan_block_sums_kernel launch");
-    hipLaunchKernelGGL(scan_top_kernel, dim3(1, count), dim3(256), 0, s, j, nb);
+    hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(256), 0, s, sums, nb);
     RECON_HIP_TRY(hipGetLastError(), "scan_top_kernel launch");
-    bool apply = true;
-    for (int i = 0; i < count; ++i) apply = apply && j.out[i];
-    if (apply) {
-        hipLaunchKernelGGL(scan_apply_kernel, dim3(nb, count), dim3(256), 0, s, j, n);
+    if (offsets) {
+        hipLaunchKernelGGL(scan_apply_kernel, dim3(nb), dim3(256), 0, s, counts, n, sums, offsets);
         RECON_HIP_TRY(hipGetLastError(), "scan_apply_kernel launch");
     }
     return RECON_OK;
-}
-
-int launch_exclusive_scan(const int32_t* counts, int n, long long* offsets, long long* sums,
-                          hipStream_t s) {
-    ScanJobs j;
-    j.in[0] = j.in[1] = counts;
-    j.sums[0] = j.sums[1] = sums;
-    j.out[0] = j.out[1] = offsets;
-    return launch_exclusive_scans(j, 1, n, s);
 }
 
 static McParams make_params(const float* field, const int32_t grid[3], const float vs[3],

@@ -64,123 +64,6 @@ __device__ __forceinline__ void load_corners(const McParams& p, int x, int y, in
     v[7] = p.f[i0 + sy + sz];
 }
 
-// The corners of the cubes of one cube row, 64 at a time, for a wavefront
-// walking the row (every lane calls every step).  Each of the row's four
-// voxel rows is read once, two steps ahead (the step at x0 issues the loads
-// of x0+128 .. x0+191), so a step never waits on a load it has just issued.
-// A cube's x+1 corners come from the next lane (a DPP wave shift) and lane
-// 63's from lane 0 of the following 64 voxels.  The values are
-// load_corners'.
-struct CornerStream {
-    const float* f;
-    int gx;
-    int rows[4];  // voxel rows (y,z), (y,z+1), (y+1,z), (y+1,z+1)
-    float cur[4];
-    float nx[4];
-
-    __device__ __forceinline__ CornerStream(const McParams& p, int y, int z, int lane) {
-        f = p.f;
-        gx = p.gx;
-        const int r0 = p.gx * y + p.gx * p.gy * z;
-        rows[0] = r0;
-        rows[1] = r0 + p.gx * p.gy;
-        rows[2] = r0 + p.gx;
-        rows[3] = r0 + p.gx + p.gx * p.gy;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cur[k] = lane < gx ? f[rows[k] + lane] : 0.0f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nx[k] = lane + 64 < gx ? f[rows[k] + lane + 64] : 0.0f;
-    }
-
-    // Corners of cube (x0 + lane, y, z), x0 = 0, 64, 128, ... in turn;
-    // defined for lanes with x0 + lane < gx - 1.
-    __device__ __forceinline__ void step(int x0, int lane, float v[8]) {
-        const int xn = x0 + 128 + lane;
-        float nn[4], hi[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nn[k] = xn < gx ? f[rows[k] + xn] : 0.0f;
-        float nxt[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nxt[k] = nx[k];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            // wave_shl:1 -- lane i receives lane i+1
-            const float sh = __int_as_float(
-                __builtin_amdgcn_update_dpp(0, __float_as_int(cur[k]), 0x130, 0xF, 0xF, false));
-            const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nxt[k]), 0));
-            hi[k] = lane == 63 ? first : sh;
-        }
-        v[0] = cur[0];
-        v[1] = hi[0];
-        v[2] = hi[1];
-        v[3] = cur[1];
-        v[4] = cur[2];
-        v[5] = hi[2];
-        v[6] = hi[3];
-        v[7] = cur[3];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            cur[k] = nxt[k];
-            nx[k] = nn[k];
-        }
-    }
-};
-
-// K consecutive cube rows (y .. y+K-1, z) of one wavefront: their 2(K+1)
-// voxel rows, each read once, streamed like CornerStream (instead of 4 per
-// cube row).
-template <int K>
-struct CornerStreamK {
-    static constexpr int R = 2 * (K + 1);  // voxel rows: (y+i, z) and (y+i, z+1)
-    const float* f;
-    int gx;
-    int rows[R];
-    float cur[R];
-    float nx[R];
-
-    __device__ __forceinline__ CornerStreamK(const McParams& p, int y, int z, int lane) {
-        f = p.f;
-        gx = p.gx;
-        const int sz = p.gx * p.gy;
-        const int r0 = p.gx * y + sz * z;
-#pragma unroll
-        for (int i = 0; i <= K; ++i) {
-            rows[2 * i] = r0 + i * p.gx;
-            rows[2 * i + 1] = r0 + i * p.gx + sz;
-        }
-#pragma unroll
-        for (int k = 0; k < R; ++k) cur[k] = lane < gx ? f[rows[k] + lane] : 0.0f;
-#pragma unroll
-        for (int k = 0; k < R; ++k) nx[k] = lane + 64 < gx ? f[rows[k] + lane + 64] : 0.0f;
-    }
-
-    // v[i] = corners of cube (x0 + lane, y + i, z), i < K
-    __device__ __forceinline__ void step(int x0, int lane, float v[K][8]) {
-        const int xn = x0 + 128 + lane;
-        float nn[R], hi[R];
-#pragma unroll
-        for (int k = 0; k < R; ++k) nn[k] = xn < gx ? f[rows[k] + xn] : 0.0f;
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const float sh = __int_as_float(
-                __builtin_amdgcn_update_dpp(0, __float_as_int(cur[k]), 0x130, 0xF, 0xF, false));
-            const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nx[k]), 0));
-            hi[k] = lane == 63 ? first : sh;
-        }
-#pragma unroll
-        for (int i = 0; i < K; ++i) {
-            const int a = 2 * i, b = 2 * i + 2;  // rows y+i and y+i+1 at z (z+1 at +1)
-            v[i][0] = cur[a]; v[i][1] = hi[a]; v[i][2] = hi[a + 1]; v[i][3] = cur[a + 1];
-            v[i][4] = cur[b]; v[i][5] = hi[b]; v[i][6] = hi[b + 1]; v[i][7] = cur[b + 1];
-        }
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            cur[k] = nx[k];
-            nx[k] = nn[k];
-        }
-    }
-};
-
 // define_voxel_type (marching_cubes.cu:76-84)
 __device__ __forceinline__ int cube_class(const float v[8]) {
     int c = 0;
@@ -214,14 +97,6 @@ __device__ __forceinline__ int wave_inclusive_max(int v) {
     t = max(t, __builtin_amdgcn_update_dpp(0, t, 0x142, 0xA, 0xF, false));  // row_bcast:15
     t = max(t, __builtin_amdgcn_update_dpp(0, t, 0x143, 0xC, 0xF, false));  // row_bcast:31
     return t;
-}
-
-__device__ __forceinline__ int wave_owner(int incl, int k) {
-    int pos = 0;
-#pragma unroll
-    for (int st = 32; st >= 1; st >>= 1)
-        if (__shfl(incl, pos + st - 1, 64) <= k) pos += st;
-    return min(pos, 63);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wavefront, by DPP moves
@@ -596,7 +471,7 @@ __device__ __forceinline__ void mc_emit_lds_init(McEmitLds& l) {
 // one wavefront: lane l takes cubes 4(l%16) .. +3 of chunk l/16, so the
 // lanes' cubes are in output order; a wave-level prefix sum places each
 // lane's triangles, and triangle k of the group is computed by lane k % 64,
-// which finds its cube (wave_owner, then among the owner's four), takes the
+// which finds its cube (LDS marks and a max-scan, then among the owner's four), takes the
 // owner's 20 voxel values (wave shuffles; the cube's 8 corners are among
 // them) and computes the vertices (edge_vertex) into an LDS stage; each 64
 // triangles' vertices and indices then leave in consecutive dwords.
