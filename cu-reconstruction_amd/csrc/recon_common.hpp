@@ -194,7 +194,7 @@ int describe(const recon_tsdf_config* cfg, recon_tsdf_info* info);
 // the count words) on first use.
 int ensure_cull_list(recon_tsdf* h, size_t ntiles, size_t entry_bytes);
 
-// Device scratch bytes marching cubes needs for `grid`.
+// Device scratch bytes that marching cubes without allocation needs for `grid`.
 size_t mc_scratch_need(const int32_t grid[3]);
 
 // Marching cubes over a dense field; `scratch` / `scratch_bytes` may point
