@@ -583,13 +583,14 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
         rest &= rest - 1;
         const FrameParams& F = frames.f[f];
         float pz[NV], rz[NV];
-        float bad = F.guard;
+        float bad = F.guard, most = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             pz[j] = ((F.R[6] * cxw[jx(j)] + F.R[7] * cyw[jy(j)]) + F.R[8] * czw[jz(j)]) + F.t[2];
             rz[j] = recip(pz[j], bad);  // serves both axes
+            most = fmaxf(most, rz[j]);
         }
-        if (__builtin_expect(__ballot(bad > kRecipBad) == 0, 1))
+        if (__builtin_expect(__ballot((bad > kRecipBad) | (most > kRecipMax)) == 0, 1))
             observe(std::false_type{}, F, pz, rz);
         else
             observe(std::true_type{}, F, pz, rz);

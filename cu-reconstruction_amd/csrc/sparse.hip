@@ -325,14 +325,15 @@ __global__ __launch_bounds__(256) void sparse_integrate_kernel(const SparseParam
         for (int z0 = 0; z0 < kBrick; z0 += kHalf, Db += 64 * kHalf, Wb += 64 * kHalf) {
             float pz[kHalf], rz[kHalf], cz[kHalf], dep[kHalf];
             bool ok[kHalf];
-            float bad = F.guard;
+            float bad = F.guard, most = 0.0f;
 #pragma unroll
             for (int j = 0; j < kHalf; ++j) {
                 cz[j] = voxel_centre(bc.z * kBrick + z0 + j, p.vs[2], p.off[2]);
                 pz[j] = ((F.R[6] * cx + F.R[7] * cy) + F.R[8] * cz[j]) + F.t[2];
                 rz[j] = recip(pz[j], bad);
+                most = fmaxf(most, rz[j]);
             }
-            const bool exact = __builtin_expect(__ballot(bad > kRecipBad) != 0, 0);
+            const bool exact = __builtin_expect(__ballot((bad > kRecipBad) | (most > kRecipMax)) != 0, 0);
             uint32_t at[kHalf];
 #pragma unroll
             for (int j = 0; j < kHalf; ++j) {
@@ -568,7 +569,7 @@ extern "C" int recon_sparse_integrate(recon_sparse* h, const recon_depth_view* d
         tabs += std::fabs(F.t[k]);
     }
     for (int k = 0; k < 9; ++k) rabs += std::fabs(F.R[k]);
-    const bool easy = (rabs * coord + tabs) * ((double)h->p.fx + h->p.fy + 1.0) < 1e30 &&
+    const bool easy = (rabs * coord + tabs) * ((double)h->p.fx + h->p.fy + 1.0) < kProductMax &&
                       std::fabs(h->p.cx) + std::fabs(h->p.cy) < 1e30 && F.pitch < (1 << 22) &&
                       depth->cols < (1 << 24) && 4.0 * (double)F.pitch * depth->rows < 4294967296.0;
     F.guard = easy ? 0.0f : INFINITY;

@@ -233,3 +233,41 @@ def test_direct_and_list_kernels_agree(cuda, grid, weight_type):
         v.close()
     assert_bitexact(got[0][0], got[1][0], "D")
     assert_bitexact(got[0][1], got[1][1], "W")
+
+
+# Poses turned by 4e-36 about an axis of the image: the camera z of a layer
+# through the camera centre is 4e-36 x or y, a normal number, and x * f / z
+# overflows.  Such a voxel projects to no pixel.  The grids have a wave-tile
+# (32 x 8 x 2) across the optical axis, which the frustum test keeps.
+GRAZING_POSES = np.array([[1, 0, -2e-36, 0, 0, 0, 0], [1, 2e-36, 0, 0, 0, 0, 0],
+                          [1, 0, 2e-36, 0, 0, 0, 0]], np.float64)
+
+
+def _grazing_workload(grid):
+    w = scenes.tiny(grid=grid, voxel_size=1 / 64, image=(640, 480), num_frames=3)
+    # voxel centres of layer gz / 2 at z = 0 exactly
+    w.offset = (-grid[0] / 128, -grid[1] / 128, -(grid[2] // 2 + 0.5) / 64)
+    w.intrinsics = (2000.0, 2000.0, 319.5, 239.5)
+    w.poses = GRAZING_POSES
+    return w, np.full((3, 480, 640), 1.0, np.float32)
+
+
+@pytest.mark.parametrize("path", ["single", "counted", "fused", "batch"])
+@pytest.mark.parametrize("grid", [(96, 40, 32), (63, 40, 32), (288, 248, 257), (287, 248, 257)])
+def test_layer_through_the_camera_centre(cuda, grid, path):
+    w, depth = _grazing_workload(grid)
+    cfg = w.config()
+    o = oracle_run(cfg, depth, w.poses)
+    assert (o["W"] > 0).any() and (o["W"][grid[2] // 2] == 0).all()
+    if path == "batch":
+        b = recon.Batch([(cfg, cuda.from_numpy(depth).cuda(), w.poses)])
+        b.run()
+        cuda.cuda.synchronize()
+        D, W = b.download(0)
+        b.close()
+    else:
+        g = gpu_run(cfg, depth, w.poses, fused=path == "fused", count=path == "counted")
+        D, W = g["D"], g["W"]
+        g["vol"].close()
+    assert_bitexact(W, o["W"], "W")
+    assert_bitexact(D, o["D"], "D")

@@ -124,3 +124,29 @@ def test_full_pool_is_flagged(cuda):
     cuda.cuda.synchronize()
     assert np.isfinite(D.cpu().numpy()).all()
     sv.close()
+
+
+def test_layer_through_the_camera_centre(cuda):
+    # a camera z of 4e-36 x or y: x * f / z overflows, and the voxel projects
+    # to no pixel (test_gpu_integrate.py has the dense paths)
+    w, _ = _scene(3, (-0.4375, -0.4375, -32.5 / 64))
+    w.voxel_size = 1 / 64
+    w.intrinsics = (2000.0, 2000.0, 319.5, 239.5)
+    w.poses = np.array([[1, 0, -2e-36, 0, 0, 0, 0], [1, 2e-36, 0, 0, 0, 0, 0],
+                        [1, 0, 2e-36, 0, 0, 0, 0]], np.float64)
+    depth = np.full((3, w.image[1], w.image[0]), 1.0, np.float32)
+    cfg = w.config()
+    sv = recon.SparseVolume(cfg, 1 << 16)
+    so = O.Sparse(O.volume_from_config(cfg))
+    sv.allocate_box((0, 0, 0), w.grid)
+    so.allocate_box((0, 0, 0), w.grid)
+    for f in range(3):
+        sv.integrate(cuda.from_numpy(depth[f]).cuda(), w.poses[f])
+        so.integrate(depth[f], w.poses[f])
+    cuda.cuda.synchronize()
+    D, W = sv.export((0, 0, 0), w.grid)
+    Do, Wo = so.export((0, 0, 0), w.grid)
+    assert (Wo > 0).any() and (Wo[32] == 0).all()
+    assert_bitexact(W.cpu().numpy(), Wo, "W")
+    assert_bitexact(D.cpu().numpy(), Do, "D")
+    sv.close()
