@@ -512,7 +512,9 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
                 if (VARW) {
-                    const float e = dep[j] - vp.noise[2];
+                    // a hole's depth may be infinite or NaN, which must not send the
+                    // wavefront to the divisions: any depth in range stands in for it
+                    const float e = (pass[j] ? dep[j] : vp.maxd) - vp.noise[2];
                     const float sig = vp.noise[0] + (vp.noise[1] * (e * e));
                     const float s2 = sig * sig;
                     const float wo = div_by_rcp(vp.wref, s2, recip_sum(s2, bad));
