@@ -171,15 +171,21 @@ __device__ __forceinline__ void diff_integrate_tile(const VolumeParams& vp, cons
             num[j] = (d[j] * w[j]) + min_bound(vp.trunc, sdf);
         }
         if (!any) return;
+        float least = INFINITY;
 #pragma unroll
-        for (int j = 0; j < NV; ++j) nd[j] = div_by_rcp(num[j], nw[j], recip_sum(nw[j], bad));
-        if (__builtin_expect(__ballot(!(bad < kRecipBad)) != 0, 0)) {
+        for (int j = 0; j < NV; ++j) {
+            const float q = short_average(num[j], nw[j], bad, least);
+            nd[j] = pass[j] ? q : d[j];
+            // NaN unless finite; a volume that was just filled stays within bounds
+            if (!kFresh) bad = __builtin_fmaf(nd[j], 0.0f, bad);
+        }
+        if (__builtin_expect(__ballot(!(bad < kRecipBad) | (!kFresh & (least < kLeast))) != 0, 0)) {
 #pragma unroll
-            for (int j = 0; j < NV; ++j) nd[j] = num[j] / nw[j];
+            for (int j = 0; j < NV; ++j) nd[j] = pass[j] ? num[j] / nw[j] : d[j];
         }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            d[j] = pass[j] ? nd[j] : d[j];
+            d[j] = nd[j];
             w[j] = pass[j] ? min_bound(vp.maxw, nw[j]) : w[j];
             dirty[j] |= pass[j];
         }

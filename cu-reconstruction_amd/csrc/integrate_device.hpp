@@ -507,7 +507,7 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             for (int i = 0; i < G; ++i) any |= pass[G * r + i];
             if (!any) continue;
             // tsdf_volume.cu:178-186 with the weight cap
-            float num[G], nw[G], nd[G], bad = guard_w;
+            float num[G], nw[G], nd[G], bad = guard_w, least = INFINITY;
 #pragma unroll
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
@@ -520,15 +520,16 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                     const float wo = div_by_rcp(vp.wref, s2, recip_sum(s2, bad));
                     nw[i] = w[j] + wo;
                     num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
-                    // a quotient near the denormals is left to the division
-                    bad = (pass[j] & !(fabsf(num[i]) >= 1e-30f)) ? INFINITY : bad;
                 } else {
                     nw[i] = w[j] + 1.0f;
                     num[i] = (d[j] * w[j]) + tsdf[j];
                 }
-                nd[i] = div_by_rcp(num[i], nw[i], recip_sum(nw[i], bad));
+                const float q = short_average(num[i], nw[i], bad, least);
+                nd[i] = pass[j] ? q : d[j];
+                // NaN unless finite; a volume that was just filled stays within bounds
+                if (!FRESH) bad = __builtin_fmaf(nd[i], 0.0f, bad);
             }
-            if (__builtin_expect(__ballot(!(bad < kRecipBad)) != 0, 0)) {
+            if (__builtin_expect(__ballot(!(bad < kRecipBad) | (!FRESH & (least < kLeast))) != 0, 0)) {
 #pragma unroll
                 for (int i = 0; i < G; ++i) {
                     const int j = G * r + i;
@@ -537,14 +538,14 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                         nw[i] = w[j] + wo;
                         num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
                     }
-                    nd[i] = num[i] / nw[i];
+                    nd[i] = pass[j] ? num[i] / nw[i] : d[j];
                 }
             }
 #pragma unroll
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
                 const float w2 = min_bound(vp.maxw, nw[i]);
-                d[j] = pass[j] ? nd[i] : d[j];
+                d[j] = nd[i];
                 w[j] = pass[j] ? w2 : w[j];
                 dirty[j] |= pass[j];
                 if (kOne && !kQuad && pass[j]) {

@@ -268,6 +268,20 @@ __device__ __forceinline__ float recip_sum(float x, float& bad) {
     return __builtin_fmaf(e, y, y);
 }
 
+// The running average's quotient num / nw in short form.  Its bits are the
+// division's if nw's residual is accepted, num and the quotient are at least
+// kLeast (below, their residual may be lost among the denormals) and the
+// quotient is finite (NaN stands for an overflow): `least` collects the smallest
+// magnitude, and the caller sends what is not finite to `bad`.  D and W within
+// the truncation and the number of frames never get there; uploaded ones may.
+constexpr float kLeast = 1e-30f;
+
+__device__ __forceinline__ float short_average(float num, float nw, float& bad, float& least) {
+    const float q = div_by_rcp(num, nw, recip_sum(nw, bad));
+    least = fminf(least, fminf(fabsf(num), fabsf(q)));
+    return q;
+}
+
 // (int)s for any s: v_cvt_i32_f32 truncates, saturates and takes NaN to 0
 // (the language leaves out-of-range conversions undefined).
 __device__ __forceinline__ int to_int_sat(float s) {

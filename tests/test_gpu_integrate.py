@@ -9,6 +9,7 @@ import pytest
 
 from helpers import assert_bitexact, gpu_run, oracle_run
 
+import oracle_ffi as O
 import recon
 from recon import scenes
 
@@ -271,3 +272,71 @@ def test_layer_through_the_camera_centre(cuda, grid, path):
         g["vol"].close()
     assert_bitexact(W, o["W"], "W")
     assert_bitexact(D, o["D"], "D")
+
+
+def _extreme_state(shape, seed):
+    """D and W as a caller may upload them: sentinels, overflowing and
+    vanishing products, whole and fractional weights; weights whose reciprocal
+    is not normal in half of the layers only."""
+    rng = np.random.default_rng(seed)
+    d = np.array([0.0, 0.02, -0.03, np.inf, -np.inf, np.nan, 1e-40, -3e-33, 1e-20, 3e38, 1e30], np.float32)
+    k = np.array([0.0, 0.5, 1.0, 7.25, 127.0, 255.0, 300.0, 1e-30, 1e30, 3e38], np.float32)
+    W = rng.choice(k[:-2], shape)
+    W[2::4] = rng.choice(k, W[2::4].shape)
+    W[3::4] = rng.choice(k, W[3::4].shape)
+    return rng.choice(d, shape), W
+
+
+def _assert_same_values(a, b, what):
+    # any NaN equals any NaN: its sign and payload are not part of the contract
+    assert np.array_equal(np.isnan(a), np.isnan(b)), what
+    assert_bitexact(np.where(np.isnan(a), np.float32(0), a), np.where(np.isnan(b), np.float32(0), b), what)
+
+
+@pytest.mark.parametrize("path", ["single", "counted", "fused", "diff"])
+@pytest.mark.parametrize("grid,weight_type", [((64, 40, 32), 0), ((63, 40, 32), 0), ((64, 40, 32), 1),
+                                              ((256, 256, 257), 0), ((257, 256, 257), 1)])
+def test_uploaded_extremes(cuda, grid, weight_type, path):
+    """One update of a volume whose D and W came from outside: the quotient
+    of the running average is the division's also where it overflows, is not a
+    number or is close to the denormals (a layer at the observed depth, where
+    the update adds exactly 0)."""
+    if path == "diff" and weight_type:
+        pytest.skip("the differentiable integrate weighs every observation 1")
+    w = scenes.tiny(grid=grid, voxel_size=1 / 64, image=(160, 120), num_frames=2)
+    w.intrinsics = (140.0, 140.0, 79.5, 59.5)
+    w.max_weight = 1e30
+    w.truncation = 0.0625
+    w.poses = np.array([[1, 0, 0, 0, 0, 0, 3], [1, 0, 0, 0, 0.5, 0, 3]], np.float64)
+    depth = np.full((2, 120, 160), 3.0 + 0.5 / 64 + (grid[2] % 2) * 0.5 / 64, np.float32)
+    depth[:, ::7, ::5] = 0.0
+    frames = 2 if path in ("fused", "diff") else 1
+    cfg = w.config()
+    cfg.weight_type = weight_type
+    vol = O.volume_from_config(cfg)
+    D, W = O.init(vol)
+    D[...], W[...] = _extreme_state(D.shape, sum(grid))
+    v = recon.TSDFVolume(cfg)
+    v.upload(D, W)
+    dev = cuda.from_numpy(depth).cuda()
+    counter = cuda.zeros(1, dtype=cuda.int64, device="cuda")
+    v.set_update_counter(counter if path == "counted" else None)
+    before = W.copy()
+    if path == "diff":
+        rt = recon.pose_to_matrix(w.poses).astype(np.float32)
+        v.diff_integrate(dev, cuda.from_numpy(rt).cuda())
+        O.lib().oracle_diff_forward_f32(O.C.byref(vol), O._p(D), O._p(W), O._p(depth), 120, 160,
+                                        O._p(np.ascontiguousarray(rt)), 2, 0)
+    else:
+        if path == "fused":
+            v.integrate_frames(dev, w.poses)
+        else:
+            v.integrate(dev[0], w.poses[0])
+        for f in range(frames):
+            O.integrate_f32(vol, D, W, depth[f], w.poses[f])
+    cuda.cuda.synchronize()
+    Dg, Wg = v.download()
+    v.close()
+    assert (W != before).sum() > 100
+    _assert_same_values(Wg, W, "W")
+    _assert_same_values(Dg, D, "D")
