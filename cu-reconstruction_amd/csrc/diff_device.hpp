@@ -158,7 +158,7 @@ __device__ __forceinline__ void diff_integrate_tile(const VolumeParams& vp, cons
             }
         }
         bool pass[NV];
-        float num[NV], nw[NV], nd[NV], bad = 0.0f;
+        float num[NV], nw[NV], nd[NV], bad = kExact ? INFINITY : 0.0f;
         bool any = false;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {

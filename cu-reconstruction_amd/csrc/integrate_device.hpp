@@ -507,7 +507,7 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             for (int i = 0; i < G; ++i) any |= pass[G * r + i];
             if (!any) continue;
             // tsdf_volume.cu:178-186 with the weight cap
-            float num[G], nw[G], nd[G], bad = guard_w, least = INFINITY;
+            float num[G], nw[G], nd[G], bad = kExact ? INFINITY : guard_w, least = INFINITY;
 #pragma unroll
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;

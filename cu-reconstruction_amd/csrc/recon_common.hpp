@@ -137,15 +137,16 @@ __host__ __device__ inline void frame_planes(const VolumeParams& vp, FrameParams
     const double tabs = ::fabs((double)fp->t[0]) + ::fabs((double)fp->t[1]) + ::fabs((double)fp->t[2]);
     fp->zmargin = (float)(1e-6 * (tabs + cmax[0] + cmax[1] + cmax[2]) + 1e-6);
     // The short forms need pixel products below kProductMax (their quotients by
-    // a camera z then stay finite, see kRecipMax), a principal point far from
-    // overflow, row bytes and row numbers below 2^24 (24-bit products), and
-    // 32-bit byte offsets within an image and within a wave-tile; anything
-    // else takes the divisions and 64-bit addresses.
+    // a camera z then stay finite, see kRecipMax), a truncation whose multiples
+    // by a weight stay finite, a principal point far from overflow, row bytes
+    // and row numbers below 2^24 (24-bit products), and 32-bit byte offsets
+    // within an image and within a wave-tile; anything else takes the divisions
+    // and 64-bit addresses.
     double rabs = 0.0;
     for (int i = 0; i < 9; ++i) rabs += ::fabs((double)fp->R[i]);
     const double reach = rabs * (cmax[0] + cmax[1] + cmax[2]) + tabs;
     const bool easy = reach * (::fabs(fx) + ::fabs(fy) + 1.0) < kProductMax && ::fabs(cx) + ::fabs(cy) < 1e30 &&
-                      fp->pitch < (1 << 22) && vp.rows < (1 << 24) && vp.gx < (1 << 26) &&
+                      vp.trunc < kProductMax && fp->pitch < (1 << 22) && vp.rows < (1 << 24) && vp.gx < (1 << 26) &&
                       4.0 * (double)fp->pitch * vp.rows < 4294967296.0;
     fp->guard = easy ? 0.0f : __builtin_inff();
     for (int k = 0; k < 6; ++k) {

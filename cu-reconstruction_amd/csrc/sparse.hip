@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256) void sparse_integrate_kernel(const SparseParam
                     w[j] = Wb[64 * j];
                 }
             }
-            float nd[kHalf], badw = 0.0f;
+            float nd[kHalf], badw = exact ? INFINITY : 0.0f;
 #pragma unroll
             for (int j = 0; j < kHalf; ++j) {
                 // tsdf_volume.cu:178-186 with the weight cap, as the dense path
@@ -570,7 +570,8 @@ extern "C" int recon_sparse_integrate(recon_sparse* h, const recon_depth_view* d
     }
     for (int k = 0; k < 9; ++k) rabs += std::fabs(F.R[k]);
     const bool easy = (rabs * coord + tabs) * ((double)h->p.fx + h->p.fy + 1.0) < kProductMax &&
-                      std::fabs(h->p.cx) + std::fabs(h->p.cy) < 1e30 && F.pitch < (1 << 22) &&
+                      std::fabs(h->p.cx) + std::fabs(h->p.cy) < 1e30 && h->p.trunc < kProductMax &&
+                      F.pitch < (1 << 22) &&
                       depth->cols < (1 << 24) && 4.0 * (double)F.pitch * depth->rows < 4294967296.0;
     F.guard = easy ? 0.0f : INFINITY;
     const auto alloc = sparse_short_forms(h->p, F, depth->cols, depth->rows) ? sparse_alloc_kernel<true>

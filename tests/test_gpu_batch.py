@@ -155,3 +155,21 @@ def test_batch_full_size_64_volumes(cuda):
         ov, _, _, _ = O.mc_extract(o["D"], ws[i].grid, list(o["vol"].voxel_size),
                                    list(o["vol"].offset))
         assert_bitexact(eager[i][2], ov, f"volume {i} ({g}) mesh vs oracle")
+
+
+def test_truncation_near_overflow(cuda):
+    # accepted: truncation 2e37; from weight 17 on D * W overflows, and the
+    # average is infinite as with the division
+    w = scenes.tiny(grid=(36, 20, 12), voxel_size=1 / 64, image=(64, 48), num_frames=24)
+    cfg = w.config()
+    cfg.truncation, cfg.max_depth, cfg.max_weight = 2e37, 3e38, 128.0
+    depth = np.full((24, 48, 64), 1e38, np.float32)
+    o = oracle_run(cfg, depth, w.poses)
+    assert np.isinf(o["D"]).sum() > 1000
+    b = recon.Batch([(cfg, cuda.from_numpy(depth).cuda(), w.poses)])
+    b.run()
+    cuda.cuda.synchronize()
+    D, W = b.download(0)
+    assert_bitexact(W, o["W"], "W")
+    assert_bitexact(D, o["D"], "D")
+    b.close()

@@ -150,3 +150,26 @@ def test_layer_through_the_camera_centre(cuda):
     assert_bitexact(W.cpu().numpy(), Wo, "W")
     assert_bitexact(D.cpu().numpy(), Do, "D")
     sv.close()
+
+
+def test_truncation_near_overflow(cuda):
+    # accepted: truncation 2e37; from weight 17 on D * W overflows, and the
+    # average is infinite as with the division
+    w, _ = _scene(1)
+    cfg = w.config()
+    cfg.truncation, cfg.max_depth, cfg.max_weight = 2e37, 3e38, 128.0
+    depth = np.full((w.image[1], w.image[0]), 1e38, np.float32)
+    sv = recon.SparseVolume(cfg, 1 << 16)
+    so = O.Sparse(O.volume_from_config(cfg))
+    sv.allocate_box((0, 0, 0), w.grid)
+    so.allocate_box((0, 0, 0), w.grid)
+    for _ in range(24):
+        sv.integrate(cuda.from_numpy(depth).cuda(), w.poses[0])
+        so.integrate(depth, w.poses[0])
+    cuda.cuda.synchronize()
+    D, W = sv.export((0, 0, 0), w.grid)
+    Do, Wo = so.export((0, 0, 0), w.grid)
+    assert np.isinf(Do).sum() > 1000
+    assert_bitexact(W.cpu().numpy(), Wo, "W")
+    assert_bitexact(D.cpu().numpy(), Do, "D")
+    sv.close()
