@@ -88,3 +88,30 @@ def test_image_ignored_without_colour(cuda):
     assert_bitexact(Wa, Wb, "W")
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("weight_type", [0, 1])
+@pytest.mark.parametrize("grid", [(256, 256, 257), (257, 256, 257)])
+def test_color_above_the_direct_limit(cuda, grid, weight_type):
+    """Coloured volumes of more than 32768 wave-tiles of 32 x 8 x 2 take the
+    list kernels: lanes of four voxels (gx % 4 == 0) and of a row, both weights."""
+    w = scenes.tiny(grid=grid, voxel_size=0.8 / max(grid), image=(96, 72), num_frames=2)
+    cfg = w.config()
+    cfg.weight_type = weight_type
+    depth = w.render()
+    rgbs = np.random.default_rng(8).integers(0, 256, (2, 72, 96, 3)).astype(np.uint8)
+    vol = recon.TSDFVolume(cfg)
+    vol.enable_color()
+    ov = O.volume_from_config(cfg)
+    Do, Wo = O.init(ov)
+    Co = np.zeros(Do.shape + (4,), np.float32)
+    for f in range(2):
+        vol.integrate(cuda.from_numpy(depth[f]).cuda(), w.poses[f], rgb=cuda.from_numpy(rgbs[f]).cuda())
+        O.integrate_color_f32(ov, Do, Wo, Co, depth[f], rgbs[f], w.poses[f])
+    cuda.cuda.synchronize()
+    D, W = vol.download()
+    assert_bitexact(D, Do, "D")
+    assert_bitexact(W, Wo, "W")
+    assert_bitexact(vol.download_colors(), Co, "colour")
+    assert (Co[..., 3] > 0).sum() > 100000
+    vol.close()

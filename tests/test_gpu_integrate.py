@@ -340,3 +340,20 @@ def test_uploaded_extremes(cuda, grid, weight_type, path):
     assert (W != before).sum() > 100
     _assert_same_values(Wg, W, "W")
     _assert_same_values(Dg, D, "D")
+
+
+@pytest.mark.parametrize("weight_type", [0, 1])
+@pytest.mark.parametrize("grid", [(256, 256, 257), (257, 256, 257)])
+def test_list_kernels_equal_oracle(cuda, grid, weight_type):
+    """One frame a call into a volume just above 32768 wave-tiles, uncounted:
+    the list kernel with lanes of four voxels (gx % 4 == 0) and of a row."""
+    w = scenes.tiny(grid=grid, voxel_size=0.8 / max(grid), image=(96, 72), num_frames=2)
+    cfg = w.config()
+    cfg.weight_type = weight_type
+    depth = w.render()
+    o = oracle_run(cfg, depth, w.poses)
+    assert min(o["counts"]) > 100000
+    g = gpu_run(cfg, depth, w.poses)
+    assert_bitexact(g["W"], o["W"], "W")
+    assert_bitexact(g["D"], o["D"], "D")
+    g["vol"].close()
