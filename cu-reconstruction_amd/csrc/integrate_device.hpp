@@ -14,14 +14,11 @@ namespace recon {
 
 constexpr int kThreads = 256;
 
-// Wave-tile of 4*LX x (64/LX) x NR voxels.  Lane l owns voxels x..x+3
-// (x = x0 + 4*(l % LX)) of row y = y0 + l / LX for z = z0 .. z0+NR-1.  With
-// LX = 8 every row segment of a wave is one aligned 128-byte line of D and W
-// when gx is a multiple of 32.
+// Wave-tile of 4*LX x (64/LX) x NR voxels, a wavefront's unit of work; which
+// of its voxels a lane holds is integrate_tile's LW.  With LX = 8 every row of
+// a tile is one aligned 128-byte line of D and W when gx is a multiple of 32.
 template <int LX, int NR>
 struct TileShape {
-    static constexpr int kLanesX = LX;
-    static constexpr int kRows = NR;
     static constexpr int X = 4 * LX;
     static constexpr int Y = 64 / LX;
     static constexpr int Z = NR;

@@ -6,12 +6,13 @@
 // managed memory.  Here the whole volume is done on the device in four
 // launches with a fixed, deterministic output order:
 //   1-3. signs, counts, scan (mc_signs.hip): a word of signs per 64 voxels,
-//        the triangles per 64-cube chunk from the words, each chunk's first
-//        triangle, and a list of units of up to 256 triangles;
-//   4.   emit - the resident wavefronts stride over the units: a unit's cubes
-//        are classified from the signs (16 a lane), its triangles spread over
-//        the lanes 64 at a time, a lane reading the six field values of its
-//        triangle's edges (marching_cubes.cu:23-74).
+//        the triangles of every 64-cube chunk from the words, and a list of
+//        units (runs of at most 64 chunks with up to 127 cubes that the surface
+//        crosses, so up to 635 triangles), each with its first triangle;
+//   4.   emit - the resident wavefronts stride over the units: a unit's crossed
+//        cubes are spread over the lanes 64 at a time, one a lane, then their
+//        triangles, a lane reading the six field values of its triangle's edges
+//        (marching_cubes.cu:23-74).
 // The allocation-free entry, whose static scratch has no room for the words
 // and the list, keeps to a smaller one (2 B per 64 cubes):
 //   1. chunk count - one wavefront per 4 cube rows (y..y+3, z), streaming

@@ -83,9 +83,6 @@ __device__ __forceinline__ int wave_sum(int v) {
     return v;
 }
 
-// The lane owning element k of per-lane counts whose inclusive wave scan is
-// `incl` (k < incl of lane 63): the number of lanes with incl <= k.  Every
-// lane must call.
 // Inclusive max over the 64 lanes of a wavefront of non-negative values, by
 // DPP moves (row shifts, then row broadcasts of lanes 15 and 31).
 __device__ __forceinline__ int wave_inclusive_max(int v) {
