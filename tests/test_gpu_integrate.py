@@ -55,7 +55,7 @@ def test_plain_small_fused_equals_per_frame(cuda):
 
 @pytest.mark.parametrize("grid", [(37, 29, 23), (66, 8, 9), (4, 4, 4), (1, 1, 1), (130, 5, 7)])
 def test_ragged_grids(cuda, grid):
-    # gx not a multiple of 4 takes the scalar path; gy, gz not multiples of 4
+    # gx not a multiple of 4, gy and gz not of the wave-tile's 8 and 2
     w = scenes.tiny(grid=grid, voxel_size=0.6 / max(grid), image=(40, 30), num_frames=4)
     _check(w, w.render())
 
@@ -357,3 +357,38 @@ def test_list_kernels_equal_oracle(cuda, grid, weight_type):
     assert_bitexact(g["W"], o["W"], "W")
     assert_bitexact(g["D"], o["D"], "D")
     g["vol"].close()
+
+
+@pytest.mark.parametrize("path", ["single", "counted", "fused", "batch", "diff"])
+def test_row_stride_beyond_24_bits(cuda, path):
+    """Rows 2^22 floats apart: their byte offsets do not fit the 24-bit products
+    of the short forms, so the whole frame takes the divisions and 64-bit
+    addresses."""
+    w = scenes.tiny(grid=(61, 37, 29), voxel_size=0.02, image=(64, 12), num_frames=2)
+    depth = w.render()
+    o = oracle_run(w.config(), depth, w.poses)
+    assert min(o["counts"]) > 1000
+    if path in ("batch", "diff"):
+        buf = cuda.zeros((2, 12, 1 << 22), dtype=cuda.float32, device="cuda")
+        buf[:, :, :64] = cuda.from_numpy(depth).cuda()
+    if path == "diff":
+        rt = recon.pose_to_matrix(w.poses).astype(np.float32)
+        o["D"], o["W"] = O.diff_forward_f32(o["vol"], depth, rt)
+        v = recon.TSDFVolume(w.config())
+        v.diff_integrate(buf[:, :, :64], cuda.from_numpy(rt).cuda())
+        cuda.cuda.synchronize()
+        D, W = v.download()
+        v.close()
+    elif path == "batch":
+        b = recon.Batch([(w.config(), buf[:, :, :64], w.poses)])
+        b.run()
+        cuda.cuda.synchronize()
+        D, W = b.download(0)
+        b.close()
+    else:
+        g = gpu_run(w.config(), depth, w.poses, fused=path == "fused", count=path == "counted",
+                    pitch_pad=(1 << 22) - 64)
+        D, W = g["D"], g["W"]
+        g["vol"].close()
+    assert_bitexact(W, o["W"], "W")
+    assert_bitexact(D, o["D"], "D")

@@ -47,9 +47,8 @@ def test_integrated_volume(cuda):
     assert n > 50000
 
 
-# rows of 3, 70, 65 and 129 voxels take the count pass's 4-byte loads; rows
-# of a multiple of 4 its 16-byte loads, 256 cubes a span: one span cut short
-# (4, 64, 68), two (260) and three (516)
+# rows of less than one chunk of 64 voxels, one, one and a voxel or a few more,
+# and up to nine
 @pytest.mark.parametrize("grid", [(3, 2, 2), (70, 3, 5), (65, 66, 7), (129, 2, 3), (4, 3, 3),
                                   (64, 5, 9), (68, 7, 6), (260, 9, 4), (516, 6, 5)])
 def test_random_fields(cuda, grid):
@@ -81,8 +80,8 @@ def test_units_and_quotient_ranges(cuda, grid, scale):
 
 
 def test_unaligned_field_takes_4_byte_loads(cuda):
-    # a field one float past a 16-byte boundary: rows of 68 voxels, but the
-    # 4-byte loads; the same results as the aligned copy
+    # a field one float past a 16-byte boundary: the passes load 4 bytes a lane
+    # at any alignment
     grid = (68, 7, 6)
     rng = np.random.default_rng(7)
     f = rng.standard_normal(grid[::-1]).astype(np.float32)
@@ -99,10 +98,9 @@ def test_unaligned_field_takes_4_byte_loads(cuda):
 
 
 def test_many_tiles(cuda):
-    # 1024 x 1024 cube rows of 7 cubes: 65536 tiles of 16 rows, so the tile
-    # scan makes eight passes and group records carry tile indices past
-    # 2^16; a cylinder along x crosses a quarter of the rows, and noise in
-    # the last 64 layers puts triangles in most chunks there
+    # 1025 x 1025 voxel rows of one chunk each, so 2053 count blocks (two passes
+    # of the scan); a cylinder along x crosses a quarter of the rows, and noise
+    # in the last 64 layers puts triangles in most chunks there
     gx, gy, gz = 8, 1025, 1025
     y = np.arange(gy, dtype=np.float32)[None, :, None]
     z = np.arange(gz, dtype=np.float32)[:, None, None]
@@ -115,18 +113,16 @@ def test_many_tiles(cuda):
 
 
 def test_sparse_chunks_of_wide_rows(cuda):
-    # rows of 2199 cubes: 35 chunks of 64, so chunks 31-34 share the last bit
-    # of the emit pass's chunk mask; 5 cube rows per layer, so each layer has
-    # one group of 4 rows (one mask for the group) and one row of its own.
-    # Surface voxels sit in a few chunks only, at chunk boundaries and at the
-    # row ends, in some rows and not in others.
+    # rows of 2199 cubes: 35 chunks of 64.  Surface voxels sit in a few chunks
+    # only, at chunk boundaries and at the row ends, in some rows and not in
+    # others, so units start and end within rows.
     gx, gy, gz = 2200, 6, 4
     f = np.full((gz, gy, gx), 0.5, np.float32)
     xs = [0, 5, 7 * 64 + 10, 30 * 64 + 63, 31 * 64, 31 * 64 + 3, 33 * 64 + 40, gx - 1]
     for k, x in enumerate(xs):
         z, y = k % gz, (2 * k) % gy
         f[z, y, x] = -0.25 - 0.01 * k
-    f[2, 5, 32 * 64 + 1] = -1.0  # the layer's row outside the 4-row group
+    f[2, 5, 32 * 64 + 1] = -1.0  # the layer's last row
     n = _mc_compare(cuda, f, (gx, gy, gz), (0.01, 0.02, 0.03), (0.1, -0.2, 0.3))
     assert n > 0
 

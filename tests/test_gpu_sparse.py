@@ -173,3 +173,34 @@ def test_truncation_near_overflow(cuda):
     assert_bitexact(W.cpu().numpy(), Wo, "W")
     assert_bitexact(D.cpu().numpy(), Do, "D")
     sv.close()
+
+
+@pytest.mark.parametrize("max_depth,stride", [(2e6, 0), (0.0, 1 << 22)])
+def test_forms_with_divisions(cuda, max_depth, stride):
+    """A depth limit of 1e6 or more sends the allocation to its divisions, rows
+    2^22 floats apart the integrate to its own and to 64-bit addresses: the
+    same bricks."""
+    w, depth = _scene(2)
+    rows, step = 24, 20
+    w.image = (w.image[0], rows)
+    fx, fy, cx, cy = w.intrinsics
+    w.intrinsics = (fx, fy / step, cx, (cy + 0.5) / step - 0.5)
+    depth = np.ascontiguousarray(depth[:, ::step][:, :rows])
+    depth[depth > 20.0] = 0.0   # the same pixels under both limits
+    cfg = w.config()
+    cfg.max_depth = max_depth
+    sv = recon.SparseVolume(cfg, 1 << 16)
+    so = O.Sparse(O.volume_from_config(cfg))
+    for f in range(2):
+        d = cuda.from_numpy(depth[f]).cuda()
+        if stride:
+            buf = cuda.zeros((rows, stride), dtype=cuda.float32, device="cuda")
+            buf[:, :d.shape[1]] = d
+            d = buf[:, :d.shape[1]]
+        sv.integrate(d, w.poses[f])
+        so.integrate(depth[f], w.poses[f])
+    cuda.cuda.synchronize()
+    n, flags = sv.stats()
+    m = _compare_bricks(sv, so, f"max_depth {max_depth} stride {stride}")
+    assert m == n > 100 and sum(W.sum() for _, W in so.bricks().values()) > 10000
+    sv.close()

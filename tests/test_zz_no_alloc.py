@@ -9,7 +9,9 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import oracle_ffi as O
 import recon
+from helpers import assert_bitexact
 from recon import ffi, scenes
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +60,58 @@ def test_noalloc_equals_allocating_extract(cuda):
         # too small an output: the count is reported with RECON_ERR_CAPACITY
         st2, n2, _, _ = _extract(cuda, lib.recon_mc_extract_noalloc, field, grid, vs, off, cap - 1)
         assert st2 == ffi.ERR_CAPACITY and n2 == cap
+
+
+def _noise(grid):
+    gx, gy, gz = grid
+    rng = np.random.default_rng(sum(grid))
+    f = rng.standard_normal((gz, gy, gx)).astype(np.float32)
+    f[rng.random(f.shape) < 0.1] = 0.0           # exact zeros: not < 0
+    f[rng.random(f.shape) < 0.05] = -0.0         # negative zero: not < 0
+    f[rng.random(f.shape) < 0.05] = 1e-41        # denormals
+    return f
+
+
+def _few_chunks():
+    # 35 chunks a cube row, surface voxels in a few of them, at chunk
+    # boundaries and row ends
+    gx, gy, gz = 2200, 6, 4
+    f = np.full((gz, gy, gx), 0.5, np.float32)
+    for k, x in enumerate([0, 5, 7 * 64 + 10, 30 * 64 + 63, 31 * 64, 31 * 64 + 3, 33 * 64 + 40, gx - 1]):
+        f[k % gz, (2 * k) % gy, x] = -0.25 - 0.01 * k
+    f[2, 5, 32 * 64 + 1] = -1.0
+    return f
+
+
+def _many_tiles():
+    # 65536 tiles of 16 cube rows: eight passes of the tile scan
+    gx, gy, gz = 8, 1025, 1025
+    y = np.arange(gy, dtype=np.float32)[None, :, None]
+    z = np.arange(gz, dtype=np.float32)[:, None, None]
+    f = (np.sqrt((y - 500.0) ** 2 + (z - 480.0) ** 2) - 300.0 + np.zeros(gx)).astype(np.float32)
+    f[-64:] = np.random.default_rng(11).standard_normal((64, gy, gx)).astype(np.float32)
+    return f
+
+
+# The passes by chunk counts, which only this entry takes: rows of 3, 70, 65
+# and 129 voxels, and an unaligned field, use the count's 4-byte loads; rows of
+# a multiple of 4 its 16-byte loads, 256 cubes a span: one span cut short (4,
+# 64, 68), two (260) and three (516)
+@pytest.mark.parametrize("case", [(3, 2, 2), (70, 3, 5), (65, 66, 7), (129, 2, 3), (4, 3, 3), (64, 5, 9),
+                                  (68, 7, 6), (260, 9, 4), (516, 6, 5), "unaligned", "few chunks",
+                                  "many tiles"])
+def test_noalloc_equals_oracle(cuda, case):
+    f = _noise(case) if isinstance(case, tuple) else \
+        {"unaligned": lambda: _noise((68, 7, 6)), "few chunks": _few_chunks, "many tiles": _many_tiles}[case]()
+    grid = f.shape[::-1]
+    vs, off = (0.01, 0.02, 0.03), (0.1, -0.2, 0.3)
+    ov, ot, _, _ = O.mc_extract(f, grid, vs, off)
+    shift = 1 if case == "unaligned" else 0
+    buf = cuda.zeros(f.size + shift, dtype=cuda.float32, device="cuda")
+    buf[shift:] = cuda.from_numpy(f.ravel()).cuda()
+    assert buf[shift:].data_ptr() % 16 == 4 * shift
+    print(f"no-alloc marching cubes on {case}: {len(ot)} triangles", flush=True)
+    st, n, v, t = _extract(cuda, ffi.load().recon_mc_extract_noalloc, buf[shift:], grid, vs, off, len(ot))
+    assert st == 0 and n == len(ot) > 0
+    assert_bitexact(v, ov, "vertices")
+    assert np.array_equal(t, ot)
