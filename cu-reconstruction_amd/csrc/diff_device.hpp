@@ -158,7 +158,7 @@ __device__ __forceinline__ void diff_integrate_tile(const VolumeParams& vp, cons
             }
         }
         bool pass[NV];
-        float num[NV], nw[NV], nd[NV], bad = kExact ? INFINITY : 0.0f;
+        float num[NV], nw[NV], nd[NV], least = INFINITY, most = 0.0f;
         bool any = false;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
@@ -168,24 +168,20 @@ __device__ __forceinline__ void diff_integrate_tile(const VolumeParams& vp, cons
             pass[j] = valid & (sdf >= -vp.trunc);
             any |= pass[j];
             nw[j] = w[j] + 1.0f;
-            num[j] = (d[j] * w[j]) + min_bound(vp.trunc, sdf);
+            num[j] = (d[j] * w[j]) + clamp_bound(vp.trunc, sdf);
         }
         if (!any) return;
-        float least = INFINITY;
 #pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const float q = short_average(num[j], nw[j], bad, least);
-            nd[j] = pass[j] ? q : d[j];
-            // NaN unless finite; a volume that was just filled stays within bounds
-            if (!kFresh) bad = __builtin_fmaf(nd[j], 0.0f, bad);
-        }
-        if (__builtin_expect(__ballot(!(bad < kRecipBad) | (!kFresh & (least < kLeast))) != 0, 0)) {
+        for (int j = 0; j < NV; ++j) nd[j] = short_average(num[j], nw[j], least, most);
+        // a volume that was just filled keeps within the bounds (its frames' guard)
+        const bool divide = kExact | (!kFresh & ((least < kLeast) | (most > kMost)));
+        if (__builtin_expect(__ballot(divide) != 0, 0)) {
 #pragma unroll
-            for (int j = 0; j < NV; ++j) nd[j] = pass[j] ? num[j] / nw[j] : d[j];
+            for (int j = 0; j < NV; ++j) nd[j] = num[j] / nw[j];
         }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            d[j] = nd[j];
+            d[j] = pass[j] ? nd[j] : d[j];
             w[j] = pass[j] ? min_bound(vp.maxw, nw[j]) : w[j];
             dirty[j] |= pass[j];
         }

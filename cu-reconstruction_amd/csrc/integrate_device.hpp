@@ -475,7 +475,7 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
         for (int j = 0; j < NV; ++j) {
             const float sdf = dep[j] - pz[j];
             pass[j] = ok[j] & (dep[j] > 0.0f) & (dep[j] <= vp.maxd) & (sdf >= -vp.trunc);
-            tsdf[j] = min_bound(vp.trunc, sdf);
+            tsdf[j] = clamp_bound(vp.trunc, sdf);
             if (COLOR) band[j] = sdf <= vp.trunc;
         }
         const uint32_t place4 = 4u * (uint32_t)place;  // below 2^32 unless exact
@@ -505,7 +505,7 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
             for (int i = 0; i < G; ++i) any |= pass[G * r + i];
             if (!any) continue;
             // tsdf_volume.cu:178-186 with the weight cap
-            float num[G], nw[G], nd[G], bad = kExact ? INFINITY : guard_w, least = INFINITY;
+            float num[G], nw[G], nd[G], bad = guard_w, least = INFINITY, most = 0.0f;
 #pragma unroll
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
@@ -518,16 +518,16 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                     const float wo = div_by_rcp(vp.wref, s2, recip_sum(s2, bad));
                     nw[i] = w[j] + wo;
                     num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
+                    least = fminf(least, fminf(fabsf(nw[i]), fabsf(num[i])));
                 } else {
                     nw[i] = w[j] + 1.0f;
                     num[i] = (d[j] * w[j]) + tsdf[j];
                 }
-                const float q = short_average(num[i], nw[i], bad, least);
-                nd[i] = pass[j] ? q : d[j];
-                // NaN unless finite; a volume that was just filled stays within bounds
-                if (!FRESH) bad = __builtin_fmaf(nd[i], 0.0f, bad);
+                nd[i] = short_average(num[i], nw[i], least, most);
             }
-            if (__builtin_expect(__ballot(!(bad < kRecipBad) | (!FRESH & (least < kLeast))) != 0, 0)) {
+            // a volume that was just filled keeps within the bounds (its frames' guard)
+            const bool divide = kExact | (!FRESH & ((least < kLeast) | (most > kMost))) | (VARW & !(bad < kRecipBad));
+            if (__builtin_expect(__ballot(divide) != 0, 0)) {
 #pragma unroll
                 for (int i = 0; i < G; ++i) {
                     const int j = G * r + i;
@@ -536,14 +536,14 @@ __device__ __forceinline__ void integrate_tile(const VolumeParams& vp, const Fra
                         nw[i] = w[j] + wo;
                         num[i] = (d[j] * w[j]) + (wo * tsdf[j]);
                     }
-                    nd[i] = pass[j] ? num[i] / nw[i] : d[j];
+                    nd[i] = num[i] / nw[i];
                 }
             }
 #pragma unroll
             for (int i = 0; i < G; ++i) {
                 const int j = G * r + i;
                 const float w2 = min_bound(vp.maxw, nw[i]);
-                d[j] = nd[i];
+                d[j] = pass[j] ? nd[i] : d[j];
                 w[j] = pass[j] ? w2 : w[j];
                 dirty[j] |= pass[j];
                 if (kOne && !kQuad && pass[j]) {

@@ -269,18 +269,23 @@ __device__ __forceinline__ float recip_sum(float x, float& bad) {
     return __builtin_fmaf(e, y, y);
 }
 
-// The running average's quotient num / nw in short form.  Its bits are the
-// division's if nw's residual is accepted, num and the quotient are at least
-// kLeast (below, their residual may be lost among the denormals) and the
-// quotient is finite (NaN stands for an overflow): `least` collects the smallest
-// magnitude, and the caller sends what is not finite to `bad`.  D and W within
-// the truncation and the number of frames never get there; uploaded ones may.
-constexpr float kLeast = 1e-30f;
+// The running average's quotient num / nw in short form.  `least` and `most`
+// collect the smallest |q| and the largest of |q| and |num|, q the quotient
+// before its correction.  With least >= kLeast and most <= kMost its bits are the
+// division's: a divisor of 0 gives an infinite q, one beyond the normal
+// reciprocals a q below kLeast (or num is above kMost), and a divisor near the
+// denormals, which no w + 1 is, is the caller's.  NaN stays NaN.  D within the
+// truncation and whole weights keep to that, but for quotients of 0; uploaded
+// ones need not.
+constexpr float kLeast = 1e-15f, kMost = 1e20f;
 
-__device__ __forceinline__ float short_average(float num, float nw, float& bad, float& least) {
-    const float q = div_by_rcp(num, nw, recip_sum(nw, bad));
-    least = fminf(least, fminf(fabsf(num), fabsf(q)));
-    return q;
+__device__ __forceinline__ float short_average(float num, float nw, float& least, float& most) {
+    float y = __builtin_amdgcn_rcpf(nw);
+    y = __builtin_fmaf(__builtin_fmaf(-nw, y, 1.0f), y, y);
+    const float q = num * y;
+    least = fminf(least, fabsf(q));
+    most = fmaxf(most, fmaxf(fabsf(num), fabsf(q)));
+    return __builtin_fmaf(__builtin_fmaf(-q, nw, num), y, q);
 }
 
 // (int)s for any s: v_cvt_i32_f32 truncates, saturates and takes NaN to 0
@@ -296,6 +301,14 @@ __device__ __forceinline__ int to_int_sat(float s) {
 __device__ __forceinline__ float min_bound(float bound, float v) {
     float r;
     asm("v_min_f32 %0, %1, %2" : "=v"(r) : "s"(bound), "v"(v));
+    return r;
+}
+
+// v within a wavefront-uniform bound of 0: the clamp of the update for the
+// voxels that pass (v >= -bound), and finite for a hole whose depth is -infinity.
+__device__ __forceinline__ float clamp_bound(float bound, float v) {
+    float r;
+    asm("v_med3_f32 %0, %2, %1, -%1" : "=v"(r) : "s"(bound), "v"(v));
     return r;
 }
 
