@@ -354,10 +354,10 @@ __device__ __forceinline__ unsigned segment_slot(const unsigned* s_pre, int nseg
 // HBM (a 512^3 volume and a VGA frame move 377 MB at 4.6 TB/s, a large copy
 // 5.1) and next by the address units (79 % busy with LW = 32; 16 and 8 took 6
 // and 19 % longer than 32).  Several frames are bound by the gathers (16 volumes of up to 40 frames of
-// 1280x720: address units 80 % busy, L2 misses at 6.5 TB/s, since a voxel
+// 1280x720: address units 78 % busy, L2 misses at 6.3 TB/s, since a voxel
 // there spans about 6 pixels): the squarest patch.  Lanes of four voxels of a
 // row each, with its branches per voxel and IEEE divisions, took 818 M
-// instructions and 2.21 ms on that batch; this form takes 550 M and 1.88 ms,
+// instructions and 2.21 ms on that batch; this form takes 535 M and 1.9 ms,
 // and 40 HD frames into 301 x 237 x 174 with variance weights fell from 1127
 // to 999 us.  One test per frame and wavefront sends the projections that the
 // short arithmetic does not cover to the divisions, one per layer the averages
